@@ -347,6 +347,32 @@ def test_gapped_columns_are_cut_and_sum_exact_sets():
     ctx.close()
 
 
+@pytest.mark.parametrize("dim,n,box", [(2, 1, 0.5), (2, 257, 0.06), (2, 700, 0.3), (2, 900, 0.13),
+                                       (2, 1500, 0.05), (2, 6000, 0.5)])
+def test_tile_limits_keep_sets_and_bits(dim, n, box):
+    """Clouds at the limits of the 2D tiles: one particle, one cell row with
+    more targets than lanes, windows past the staged candidates, more accepted
+    candidates in a stencil column than the list holds, and sparse ones.  The
+    pair counts are the brute-force sets, and the right-hand side has the bits
+    of the schedule that reads everything from global memory."""
+    h = 0.02
+    rng = np.random.default_rng(n)
+    r = rng.uniform(0.0, box, size=(n, dim))
+    pa = ta.ParticleArray(dim, r, rng.uniform(990.0, 1010.0, n), n, np.zeros((0, dim)),
+                          tuple([-0.1] * dim), tuple([1.0] * dim), v=rng.normal(0, 1, (n, dim)))
+    eq = _eq(dim, 0.5 * h)
+    eq.h = h
+    ctx = _ctx(eq, [pa])
+    want = oracle.naive_search(r, 2.0 * h)
+    counts = ctx.pair_counts().astype(np.int64)
+    assert np.array_equal(counts, np.diff(want[0].astype(np.int64)) - 1)
+    got = ctx.compute_rhs()
+    ctx.set_schedule(0, 0)
+    ref = ctx.compute_rhs()
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+    ctx.close()
+
+
 def test_empty_upload_rejected():
     eq = _eq(2, 0.02)
     ctx = ta.HipContext(eq)

@@ -395,40 +395,43 @@ tit_status build_schedule(tit_hip_ctx* c) {
   }
   if (need > c->chunk_cap) {
     forget(c, c->chunks);
-    forget(c, c->overflow);
     c->chunks = nullptr;
-    c->overflow = nullptr;
     TIT_HIP_TRY(c, dalloc(c, &c->chunks, need));
-    TIT_HIP_TRY(c, dalloc(c, &c->overflow, need));
     c->chunk_cap = need;
   }
   if (!c->chunk_counts) TIT_HIP_TRY(c, dalloc(c, &c->chunk_counts, 4));
-  if (dim == 3 && !c->blocks) {
-    // blocks of kBlk3 x kBlk3 columns; a block chunk holds at least one
-    // particle and one non-empty row of its block
+  if (!c->blocks) {
+    // blocks of kBlk2 columns (2D), kBlk3 x kBlk3 (3D)
+    const int bw = dim == 2 ? kBlk2 : kBlk3;
     std::vector<uint4> blocks;
     for (size_t t = 0; t < c->host_tanks.size(); ++t) {
       const DevTank& T = c->host_tanks[t];
-      for (int bx = 0; bx < T.nc[0]; bx += kBlk3) {
-        for (int by = 0; by < T.nc[1]; by += kBlk3) {
+      for (int bx = 0; bx < T.nc[0]; bx += bw) {
+        for (int by = 0; by < (dim == 2 ? 1 : T.nc[1]); by += bw) {
           blocks.push_back(make_uint4(static_cast<uint32_t>(t), bx, by, 0u));
         }
       }
     }
-    const size_t cap =
-        std::min(static_cast<size_t>(c->n), blocks.size() * static_cast<size_t>(nz_max)) + 1;
     TIT_HIP_TRY(c, dalloc(c, &c->blocks, blocks.size()));
     TIT_HIP_TRY(c, dalloc(c, &c->bcount, blocks.size() + 1));
-    TIT_HIP_TRY(c, dalloc(c, &c->bchunks, cap));
-    TIT_HIP_TRY(c, dalloc(c, &c->boverflow, cap));
     TIT_HIP_TRY(c, hipMemcpy(c->blocks, blocks.data(), blocks.size() * sizeof(uint4),
                              hipMemcpyHostToDevice));
     c->n_blocks = static_cast<uint32_t>(blocks.size());
-    c->bchunk_cap = cap;
+  }
+  const size_t bneed = block_chunk_bound(dim, c->n, c->n_blocks, static_cast<size_t>(nz_max),
+                                         c->chunk_targets, c->lds_cap);
+  if (bneed > c->bchunk_cap) {
+    forget(c, c->bchunks);
+    forget(c, c->boverflow);
+    c->bchunks = nullptr;
+    c->boverflow = nullptr;
+    TIT_HIP_TRY(c, dalloc(c, &c->bchunks, bneed));
+    if (dim == 3) TIT_HIP_TRY(c, dalloc(c, &c->boverflow, bneed));
+    c->bchunk_cap = bneed;
   }
   StageGrids g;
   stage_grids(c->dp, c->n_cu, &g);
-  c->grid_lds = g.lds;
+  c->grid_tile = g.tile;
   c->grid_global = g.global;
   c->grid_lds3 = g.lds3;
   c->grid_block_global = g.block_global;
@@ -450,9 +453,8 @@ StageArgs stage_args(tit_hip_ctx* c) {
   a.chunk_targets = c->chunk_targets;
   a.lds_cap = c->lds_cap;
   a.chunks = c->chunks;
-  a.overflow = c->overflow;
   a.counts = c->chunk_counts;
-  a.grid_lds = c->grid_lds;
+  a.grid_tile = c->grid_tile;
   a.grid_global = c->grid_global;
   a.blocks = c->blocks;
   a.n_blocks = c->n_blocks;
@@ -480,8 +482,10 @@ StageArgs stage_args(tit_hip_ctx* c) {
 }
 
 void enqueue_stage(tit_hip_ctx* c, const DevState& in, const DevState& old,
-                   const DevState& out, int kind, double w, bool final) {
+                   const DevState& out, int kind, double w, bool final, int set) {
   StageArgs a = stage_args(c);
+  a.work = c->work + set * tit_amd::kWorkSet;
+  if (kind == kRhsOnly) launch_clear_work(c->stream, a.work);
   a.in = in;
   a.old = old;
   a.out = out;
@@ -494,17 +498,17 @@ void enqueue_stage(tit_hip_ctx* c, const DevState& in, const DevState& old,
 void enqueue_step(tit_hip_ctx* c) {
   hipStream_t s = c->stream;
   launch_step_begin(s, c->n_tanks, c->dt_min, c->dt, c->vmax, c->disp, c->dp.skin_half,
-                    rebuild_ctl(c));
+                    rebuild_ctl(c), c->work);
   enqueue_rebuild(c, kRebuildMarked);
   enqueue_boundary(c, c->A);
-  enqueue_stage(c, c->A, c->A, c->B, kEuler, 1.0, false);
+  enqueue_stage(c, c->A, c->A, c->B, kEuler, 1.0, false, 0);
   enqueue_boundary(c, c->B);
   if (c->prm.ssprk_order == 2) {
-    enqueue_stage(c, c->B, c->A, c->A, kCombine, 1.0 / 2.0, true);
+    enqueue_stage(c, c->B, c->A, c->A, kCombine, 1.0 / 2.0, true, 1);
   } else {
-    enqueue_stage(c, c->B, c->A, c->C, kCombine, 1.0 / 4.0, false);
+    enqueue_stage(c, c->B, c->A, c->C, kCombine, 1.0 / 4.0, false, 1);
     enqueue_boundary(c, c->C);
-    enqueue_stage(c, c->C, c->A, c->A, kCombine, 2.0 / 3.0, true);
+    enqueue_stage(c, c->C, c->A, c->A, kCombine, 2.0 / 3.0, true, 2);
   }
   launch_step_end(s, c->n_tanks, c->dt, c->vmax, c->time, c->disp,
                   c->dp.skin_half, c->counter + 1);
@@ -965,6 +969,7 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   TIT_HIP_TRY(c, dalloc(c, &c->counter, 4));
   TIT_HIP_TRY(c, dalloc(c, &c->rebuild_ctl, 4));
   TIT_HIP_TRY(c, dalloc(c, &c->tank_need, n_tanks));
+  TIT_HIP_TRY(c, dalloc(c, &c->work, kWorkSets * kWorkSet));
   TIT_HIP_TRY(c, dalloc(c, &c->rebuild_count, 1));
   c->sort.max_tiles = radix_sort_tiles(n);
   TIT_HIP_TRY(c, dalloc(c, &c->sort.hist, 2048ull * std::max<uint32_t>(c->sort.max_tiles, 1)));
@@ -1094,7 +1099,6 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   if (st != TIT_OK) return st;
   c->cols = nullptr;
   c->chunks = nullptr;
-  c->overflow = nullptr;
   c->block_tot = nullptr;
   c->chunk_counts = nullptr;
   c->blocks = nullptr;
@@ -1216,7 +1220,7 @@ tit_status tit_hip_compute_rhs(tit_hip_ctx* c, double* drho_dt, double* dv_dt) {
   TIT_HIP_TRY(c, hipSetDevice(c->device));
   enqueue_rebuild(c, kRebuildPending);
   if (c->walls) enqueue_boundary(c, c->A);  // gamma and face terms of this state
-  enqueue_stage(c, c->A, c->A, c->A, kRhsOnly, 1.0, false);
+  enqueue_stage(c, c->A, c->A, c->A, kRhsOnly, 1.0, false, tit_amd::kWorkSets - 1);
   // reuse the staging buffers: drho -> stage_rho, dv -> stage_v
   launch_export_rhs(c->stream, c->prm.dim, c->n, c->id, c->rhs_drho, c->rhs_dv,
                     c->stage_rho, c->stage_v);
@@ -1236,7 +1240,7 @@ tit_status tit_hip_pair_counts(tit_hip_ctx* c, uint32_t* count) {
   TIT_HIP_TRY(c, hipSetDevice(c->device));
   enqueue_rebuild(c, kRebuildPending);
   if (c->walls) enqueue_boundary(c, c->A);
-  enqueue_stage(c, c->A, c->A, c->A, kRhsOnly, 1.0, false);
+  enqueue_stage(c, c->A, c->A, c->A, kRhsOnly, 1.0, false, tit_amd::kWorkSets - 1);
   uint32_t* out = reinterpret_cast<uint32_t*>(c->stage_rho);  // n doubles >= n u32
   launch_export_u32(c->stream, c->n, c->id, c->rhs_count, out);
   tit_status st = check_launch(c, "pair_counts");

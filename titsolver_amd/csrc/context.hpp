@@ -47,6 +47,7 @@ struct tit_hip_ctx {
   uint32_t* fixed_active = nullptr;  // fixed particles with fluid in their stencil
   uint32_t* counter = nullptr;  // [0] fixed count, [1] flags, [2] fixed_active count
   uint32_t* rebuild_ctl = nullptr;       // RebuildCtl::ctl
+  uint32_t* work = nullptr;              // chunk-queue counters (kWorkSets sets)
   uint32_t* tank_need = nullptr;         // RebuildCtl::need
   unsigned long long* rebuild_count = nullptr;
   SortScratch sort;
@@ -97,14 +98,13 @@ struct tit_hip_ctx {
   uint4* cols = nullptr;
   uint32_t n_cols = 0;
   uint4* chunks = nullptr;
-  uint32_t* overflow = nullptr;
   uint32_t* block_tot = nullptr;
   uint32_t* chunk_counts = nullptr;
   size_t chunk_cap = 0;
   uint32_t chunk_targets = kChunkMax;
   uint32_t lds_cap = 0;
-  uint32_t grid_lds = 0, grid_global = 0;
-  // 3D block chunks of the LDS stage kernel
+  uint32_t grid_tile = 0, grid_global = 0;
+  // block chunks of the LDS stage kernels
   uint4* blocks = nullptr;
   uint32_t n_blocks = 0;
   uint4* bchunks = nullptr;

@@ -702,8 +702,11 @@ __global__ void k_rebuild_clear(uint32_t* ctl) { ctl[0] = 0u; }
 __global__ __launch_bounds__(64) void k_step_begin(unsigned long long* dt_min, double* dt,
                                                    uint32_t* vmax, const double* disp,
                                                    double skin_half, double span, uint32_t* ctl,
-                                                   uint32_t* need) {
+                                                   uint32_t* need, uint32_t* work) {
   const uint32_t t = blockIdx.x;
+  if (t == 0) {
+    for (uint32_t k = threadIdx.x; k < (kWorkSets - 1) * kWorkSet; k += 64) work[k] = 0u;
+  }
   const unsigned long long b = red_fold<false>(dt_min, t, true);
   const uint32_t vb = red_fold<true>(vmax, t, true);
   if (threadIdx.x != 0) return;
@@ -959,10 +962,16 @@ void launch_time_step(hipStream_t s, const DevParams& P, uint32_t n,
 
 void launch_step_begin(hipStream_t s, int n_tanks, unsigned long long* dt_min,
                        double* dt, uint32_t* vmax, const double* disp,
-                       double skin_half, RebuildCtl rc, double span) {
+                       double skin_half, RebuildCtl rc, uint32_t* work, double span) {
   k_rebuild_clear<<<1, 1, 0, s>>>(rc.ctl);
   k_step_begin<<<n_tanks, 64, 0, s>>>(dt_min, dt, vmax, disp, skin_half, span, rc.ctl,
-                                      rc.need);
+                                      rc.need, work);
+}
+
+__global__ void k_clear_work(uint32_t* set) { set[threadIdx.x] = 0u; }
+
+void launch_clear_work(hipStream_t s, uint32_t* set) {
+  k_clear_work<<<1, kWorkSet, 0, s>>>(set);
 }
 
 void launch_force_rebuild(hipStream_t s, int n_tanks, RebuildCtl rc) {

@@ -5,18 +5,27 @@
 
 namespace tit_amd {
 
-// Largest chunk (targets per workgroup) and LDS position capacity of the
-// 2D stage kernel.
+// Largest column chunk (targets per workgroup) and the largest LDS capacity a
+// 2D schedule may name.
 constexpr int kChunkMax = 128;
 constexpr int kStageLdsCap = 1024;
-// Cells a chunk's targets span along a column at most: a column's equal
-// parts are cut further where they span more (a column whose particles are
-// split by empty cells, such as fluid below and a wall's vertices at the
-// top), so that every chunk's window fits the LDS kernel's cell rows.
+// Cells a column chunk's targets span along a column at most: a column's
+// equal parts are cut further where they span more.
 constexpr int kChunkRows = 92;
-// Window columns of a 2D chunk and LDS cell-offset rows of its window.
+// 2D tiles (stage_tile.hip): the cell columns of a tank in blocks of kBlk2; a
+// chunk holds the particles of one block in a range of at most kChunkRows2
+// rows, at most kTileThreads of them, and its window (the block grown by the
+// stencil) at most kTileCap candidates, staged in LDS whole.  kTileList:
+// accepted candidates listed per lane between two pair loops.
+constexpr int kBlk2 = 4;
+constexpr int kChunkRows2 = 28;
+constexpr int kTileThreads = 256;
+constexpr int kTileCap = 744;
+constexpr int kTileList = 42;
+constexpr int kTilePad = 3;
+constexpr int kTileWaves = 3;
+// Stencil columns of a 2D target.
 constexpr int kCols2 = 2 * kStencil + 1;
-constexpr int kRowsMax = kChunkRows + 2 * kStencil;
 // 3D block chunks: the cell columns of a tank in blocks of kBlk3 x kBlk3;
 // a chunk holds the particles of one block in a range of at most
 // kChunkRows3 rows, at most kStage3Threads of them (a row with more goes to
@@ -34,6 +43,12 @@ constexpr int kStage3Threads = 256;
 // rows at most 64 x 10 x 2.9 = 1,860; 2,048 candidates keep the workgroup's
 // LDS under 53 KB: three workgroups of four waves per CU)
 constexpr int kStage3LdsCap = 2048;
+
+// Counters of the chunk queue (stage_common.hpp): one set of 8 per stage of a
+// step, cleared at the step's begin, and one for the right-hand-side hook.
+constexpr uint32_t kWorkStride = 16;
+constexpr uint32_t kWorkSet = 8 * kWorkStride;
+constexpr uint32_t kWorkSets = 4;
 
 struct StageArgs {
   DevParams P;
@@ -64,15 +79,17 @@ struct StageArgs {
   uint32_t chunk_targets;
   uint32_t lds_cap;            // candidate positions staged in LDS at most
   uint4* chunks;
-  uint32_t* overflow;          // 2D chunks whose candidates exceed lds_cap
-  // [0] chunks, [1] overflow chunks, [2] 3D block chunks, [3] block chunks
-  // that take the global-memory kernel
+  // [0] column chunks, [2] block chunks, [3] 3D block chunks that take the
+  // global-memory kernel
   uint32_t* counts;
-  uint32_t grid_lds, grid_global;  // persistent grid sizes
-  // 3D with LDS staging (lds_cap > 0): cell-column blocks (tank, first ix,
+  uint32_t grid_tile, grid_global;  // persistent grid sizes
+  uint32_t* work;                   // this launch's set of chunk-queue counters
+  // with LDS staging (lds_cap > 0): cell-column blocks (tank, first ix,
   // first iy, 0), rebuilt on the device after every cell rebuild: block
-  // chunks (block, first row, end row, targets), per-block chunk counts
-  // (scanned in place), and the block chunks that do not fit
+  // chunks (2D: tank | does not fit the LDS << 31, first ix, first row, end
+  // row; 3D: block, first row, end row, does not fit),
+  // per-block chunk counts (scanned in place), and the 3D block chunks that
+  // do not fit
   const uint4* blocks;
   uint32_t n_blocks;
   uint4* bchunks;
@@ -232,11 +249,20 @@ void launch_post_integrate(hipStream_t s, const PiArgs& a, int n_tanks, double* 
 // dst[id[i]] = src[i] (FP64).
 void launch_export_f64(hipStream_t s, uint32_t n, const uint32_t* id, const double* src,
                        double* dst);
+// Clears one set of chunk-queue counters.
+void launch_clear_work(hipStream_t s, uint32_t* set);
 void launch_stage(hipStream_t s, const StageArgs& a, int kind, bool final);
 uint32_t stage_lds_capacity(int dim);
+// Block chunks the chunk builder can emit at most for n particles in n_blocks
+// blocks of nz rows, with the schedule's target and window limits.
+size_t block_chunk_bound(int dim, size_t n, size_t n_blocks, size_t nz, uint32_t chunk_targets,
+                         uint32_t lds_cap);
+// stage_tile.hip: the 2D stage over tiles, and its workgroups resident per CU.
+void launch_stage_tile(hipStream_t s, const StageArgs& a, int kind, bool final);
+int tile_groups_per_cu();
 // Persistent grid sizes of the stage kernels (multiples of 8 workgroups).
 struct StageGrids {
-  uint32_t lds, global, lds3, block_global;
+  uint32_t tile, global, lds3, block_global;
 };
 void stage_grids(const DevParams& P, int n_cu, StageGrids* g);
 // Rebuilds the chunk list from the cell offsets (after a cell rebuild).
@@ -247,12 +273,13 @@ void launch_time_step(hipStream_t s, const DevParams& P, uint32_t n,
                       const double* dv_ref, unsigned long long* dt_min);
 // The per-tank dt_min / vmax / shift_max buffers hold kRedStripes copies per
 // tank (n_tanks x kRedStripes values); the launchers below fold them.
-// Takes each tank's pending step size dt and decides its rebuild for a step
+// Clears the stages' chunk-queue counters (work, kWorkSets - 1 sets), takes
+// each tank's pending step size dt and decides its rebuild for a step
 // of span x dt: needed when forced or when disp + 2 span dt vmax (vmax of the
 // previous step) could pass 0.9 of half the skin by the end of the step.
 void launch_step_begin(hipStream_t s, int n_tanks, unsigned long long* dt_min,
                        double* dt, uint32_t* vmax, const double* disp,
-                       double skin_half, RebuildCtl rc, double span = 1.0);
+                       double skin_half, RebuildCtl rc, uint32_t* work, double span = 1.0);
 // Marks every tank for the next rebuild sequence.
 void launch_force_rebuild(hipStream_t s, int n_tanks, RebuildCtl rc);
 // Makes a forced rebuild pending (after moves the displacement bound does not

@@ -17,32 +17,7 @@ namespace tit_amd {
 
 namespace {
 
-constexpr int kWords = 5;      // acceptance masks held per lane (LDS path)
 constexpr int kWordsG = 24;    // 32-candidate masks held per lane (global path)
-constexpr uint32_t kWordSpan = 1u << 22;  // candidate global-index span of an LDS chunk
-static_assert(kStageLdsCap <= 1024, "LDS index packs into 10 bits");
-
-// Positions from LDS (2D).
-struct LdsPos {
-  const double2* xy;
-  const uint32_t (*coff)[kRowsMax + 1];  // [column][row - zlo]
-  const uint32_t* gb;                    // global index of each column's row zlo
-  const uint32_t* lb;                    // LDS index of each column's row zlo
-  int zlo, nz, ix, ncx;
-  uint32_t gbase;   // global index of the chunk's first candidate
-
-  // Candidates of column k in rows [w0, w1] (inside the target's 5-row window).
-  __device__ __forceinline__ bool range(int k, int w0, int w1, uint32_t& b,
-                                        uint32_t& e) const {
-    const int ixk = ix - kStencil + k;
-    if (ixk < 0 || ixk >= ncx) return false;
-    const int z0 = max(w0, 0), z1 = min(w1, nz - 1);
-    if (z0 > z1) return false;
-    b = coff[k][z0 - zlo];
-    e = coff[k][z1 + 1 - zlo];
-    return true;
-  }
-};
 
 // Positions from global memory (any dimension).
 template <int DIM>
@@ -120,173 +95,10 @@ __device__ __forceinline__ bool within(const DevParams& P, const double* xb,
   return s <= P.R2;
 }
 
-__device__ __forceinline__ uint32_t pop_lowest(uint64_t& mask) {
-  const uint32_t t = static_cast<uint32_t>(__builtin_ctzll(mask));
-  mask &= mask - 1;
-  return t;
-}
-
 // Candidate order, the same on every path so that all schedules produce the
 // same bits: stencil columns in order, within a column ascending index; the
 // accepted candidates' terms enter the compensated sums two at a time.
 //
-// 2D with LDS positions.  The acceptance masks of up to kWords candidate
-// batches (normally one per stencil column) are queued per lane in registers
-// and their accepted candidates are summed in one loop, so a wave's pair loop
-// runs for the largest accepted count among its lanes, not for the sum over
-// columns of each column's largest count.
-struct WordQueue {
-  uint64_t m[kWords];   // acceptance masks, oldest first (never empty)
-  uint32_t jl[kWords];  // their bit 0: global index - gbase (bits 10..31), LDS index
-
-  // Appends at slot n (a run-time index: one select per slot).
-  __device__ __forceinline__ void put(int n, uint64_t mask, uint32_t v) {
-#pragma unroll
-    for (int q = 0; q < kWords; ++q) {
-      if (q == n) {
-        m[q] = mask;
-        jl[q] = v;
-      }
-    }
-  }
-  // Removes the oldest word.
-  __device__ __forceinline__ void pop(uint64_t& mask, uint32_t& v) {
-    mask = m[0];
-    v = jl[0];
-#pragma unroll
-    for (int q = 0; q + 1 < kWords; ++q) {
-      m[q] = m[q + 1];
-      jl[q] = jl[q + 1];
-    }
-  }
-};
-
-template <int KERNEL, int FLAVOUR>
-__device__ __forceinline__ void sum_words(const DevParams& P, const LdsPos& ps,
-                                          const DevState& S, const Target<2>& a,
-                                          uint32_t n_acc, Sums<2>& acc, WordQueue& wq) {
-  uint64_t m = 0;
-  uint32_t l0 = 0, j0 = 0;
-  // The next of the n_acc accepted candidates.
-  auto take = [&](PairIn<2>& p) {
-    if (m == 0) {
-      uint32_t jl;
-      wq.pop(m, jl);
-      j0 = ps.gbase + (jl >> 10);
-      l0 = jl & 1023u;
-    }
-    const uint32_t t = pop_lowest(m);
-    const double2 x = ps.xy[l0 + t];
-    p.x[0] = x.x;
-    p.x[1] = x.y;
-    p.pv = S.pv[j0 + t];
-    p.aux = S.aux[j0 + t];
-    p.vol = 0.0f;
-  };
-  uint32_t rem = n_acc;
-  PairIn<2> A, B;
-  if (rem == 0) return;
-  if (acc.pend) {  // an odd term of an earlier batch of words waits for its partner
-    take(A);
-    sum_pair<2, KERNEL, FLAVOUR>(P, a, A, acc);
-    if (--rem == 0) return;
-  }
-  // two register sets alternate (the next candidate's loads in flight while
-  // the current one is summed); their terms enter the compensated sums
-  // together
-  take(A);
-  --rem;
-  while (true) {
-    const bool hb = rem > 0;
-    if (hb) {
-      take(B);
-      --rem;
-    }
-    float ca, fa[2];
-    term_of<2, KERNEL, FLAVOUR>(P, a, A, ca, fa);
-    if (!hb) {
-      acc.add(ca, fa);
-      break;
-    }
-    const bool ha = rem > 0;
-    if (ha) {
-      take(A);
-      --rem;
-    }
-    float cb, fb[2];
-    term_of<2, KERNEL, FLAVOUR>(P, a, B, cb, fb);
-    acc.add2(ca, fa, cb, fb);
-    if (!ha) break;
-  }
-}
-
-template <int KERNEL, int FLAVOUR, int NCOL>
-__device__ __forceinline__ void gather_words(const DevParams& P, const LdsPos& ps,
-                                             const DevState& S, const Target<2>& a,
-                                             uint32_t i, int zc, const Windows<2, NCOL>& W,
-                                             Sums<2>& acc, uint32_t& count) {
-  WordQueue wq;
-  int k = 0, kc = 0;
-  uint32_t c0 = 0, e = 0;
-  bool more = true;
-  while (more) {
-    int nw = 0;
-    uint32_t n_acc = 0;
-    while (nw < kWords) {
-      if (c0 >= e) {  // next non-empty column range
-        bool found = false;
-        for (; k < NCOL && !found; ++k) {
-          const uint32_t v = W.get(k);
-          if ((v & 7u) == 7u) continue;
-          const int w0 = zc - kStencil + static_cast<int>(v & 7u);
-          const int w1 = zc - kStencil + static_cast<int>(v >> 3);
-          uint32_t b, eb;
-          if (ps.range(k, w0, w1, b, eb) && b < eb) {
-            found = true;
-            kc = k;
-            c0 = b;
-            e = eb;
-          }
-        }
-        if (!found) {
-          more = false;
-          break;
-        }
-      }
-      const uint32_t len = min(e - c0, 64u);
-      const uint32_t lc = ps.lb[kc] + (c0 - ps.gb[kc]);
-      uint64_t mask = 0;
-      uint32_t t = 0;
-      for (; t + 4 <= len; t += 4) {
-        const double2 p0 = ps.xy[lc + t], p1 = ps.xy[lc + t + 1];
-        const double2 p2 = ps.xy[lc + t + 2], p3 = ps.xy[lc + t + 3];
-        const double x0[2] = {p0.x, p0.y}, x1[2] = {p1.x, p1.y};
-        const double x2[2] = {p2.x, p2.y}, x3[2] = {p3.x, p3.y};
-        const uint64_t mm = (within<2>(P, x0, a.x) ? 1ull : 0ull) |
-                            (within<2>(P, x1, a.x) ? 2ull : 0ull) |
-                            (within<2>(P, x2, a.x) ? 4ull : 0ull) |
-                            (within<2>(P, x3, a.x) ? 8ull : 0ull);
-        mask |= mm << t;
-      }
-      for (; t < len; ++t) {
-        const double2 p0 = ps.xy[lc + t];
-        const double x0[2] = {p0.x, p0.y};
-        if (within<2>(P, x0, a.x)) mask |= 1ull << t;
-      }
-      if (i >= c0 && i < c0 + len) mask &= ~(1ull << (i - c0));  // not self
-      const uint32_t na = static_cast<uint32_t>(__builtin_popcountll(mask));
-      count += na;
-      n_acc += na;
-      if (mask) {
-        wq.put(nw, mask, ((c0 - ps.gbase) << 10) | lc);
-        ++nw;
-      }
-      c0 += len;
-    }
-    sum_words<KERNEL, FLAVOUR>(P, ps, S, a, n_acc, acc, wq);
-  }
-}
-
 // Global-memory path, the same scheme with 32-candidate masks (the 3D stencil
 // has 25 short column ranges): all columns' accepted candidates are summed
 // in one loop per lane, in the common candidate order.
@@ -666,20 +478,17 @@ __device__ __forceinline__ ChunkInfo chunk_info(const StageArgs& A, uint32_t q) 
   return c;
 }
 
-// One target (one lane), particle i of cell column (cx, cy) of tank `tank`
-// (col_row: the global index of the column's first cell): pair sums, then
-// the SSPRK substep / combination of time_integrator.hpp:188-223 in FP64
-// and, on the last stage, the next step's CFL candidate.  The lane's speed
-// and CFL candidate come back in vmax and dtmin for the per-wave reductions.
-template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, class Pos>
-__device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T,
-                                            uint32_t tank, int cx, int cy, uint32_t col_row,
-                                            uint32_t i, bool in_range, const Pos& ps,
-                                            float& vmax, unsigned long long& dtmin) {
-  constexpr int NCOL = DIM == 2 ? kCols2 : kCols2 * kCols2;
+// After the pair sums of one target (one lane): particle i's right-hand side
+// (KIND kRhsOnly), or the SSPRK substep / combination of
+// time_integrator.hpp:188-223 in FP64 and, on the last stage, the next step's
+// CFL candidate.  Fixed particles keep their state.  The lane's speed and CFL
+// candidate come back in vmax and dtmin for the per-wave reductions.
+template <int DIM, int FLAVOUR, int KIND, bool FINAL>
+__device__ __forceinline__ void finish_target(const StageArgs& A, uint32_t tank, uint32_t i,
+                                              bool in_range, bool fluid, const Sums<DIM>& acc,
+                                              uint32_t count, float& vmax,
+                                              unsigned long long& dtmin) {
   const DevParams& P = A.P;
-  const uint32_t tag = in_range ? A.tag[i] : 1u;
-  const bool fluid = in_range && !(tag & 1u);
   vmax = 0.0f;
   dtmin = ~0ull;
   if (in_range && !fluid) {
@@ -708,22 +517,6 @@ __device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T
       va[k] = A.in.v[k][i];
     }
     const double rho_a = A.in.rho[i];
-    Target<DIM> a;
-    make_target<DIM, FLAVOUR>(P, xa, va, rho_a, A.in.aux[i], a);
-    const int zc = static_cast<int>(A.key[i] - col_row);
-    Sums<DIM> acc;
-    acc.init();
-    const Windows<DIM, NCOL> W =
-        stencil_windows<DIM, NCOL>(P, T, xa, cx, cy, zc);
-    uint32_t count = 0;
-    if constexpr (std::is_same_v<Pos, LdsPos>) {
-      gather_words<KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
-    } else if constexpr (std::is_same_v<Pos, LdsPos3>) {
-      gather_words3<KERNEL, FLAVOUR>(P, ps, A.in, a, i, cx, cy, zc, W, acc, count);
-    } else {
-      gather_words_g<DIM, KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
-    }
-    acc.finish();
     if constexpr (KIND == kRhsOnly) {
       if (A.rhs_count) A.rhs_count[i] = count;
     }
@@ -787,6 +580,43 @@ __device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T
   }
 }
 
+// One target (one lane), particle i of cell column (cx, cy) of tank `tank`
+// (col_row: the global index of the column's first cell), by the column-chunk
+// and 3D paths.
+template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, class Pos>
+__device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T,
+                                            uint32_t tank, int cx, int cy, uint32_t col_row,
+                                            uint32_t i, bool in_range, const Pos& ps,
+                                            float& vmax, unsigned long long& dtmin) {
+  constexpr int NCOL = DIM == 2 ? kCols2 : kCols2 * kCols2;
+  const DevParams& P = A.P;
+  const uint32_t tag = in_range ? A.tag[i] : 1u;
+  const bool fluid = in_range && !(tag & 1u);
+  Sums<DIM> acc;
+  acc.init();
+  uint32_t count = 0;
+  if (fluid) {
+    double xa[DIM], va[DIM];
+#pragma unroll
+    for (int k = 0; k < DIM; ++k) {
+      xa[k] = A.in.x[k][i];
+      va[k] = A.in.v[k][i];
+    }
+    Target<DIM> a;
+    make_target<DIM, FLAVOUR>(P, xa, va, A.in.rho[i], A.in.aux[i], a);
+    const int zc = static_cast<int>(A.key[i] - col_row);
+    const Windows<DIM, NCOL> W =
+        stencil_windows<DIM, NCOL>(P, T, xa, cx, cy, zc);
+    if constexpr (std::is_same_v<Pos, LdsPos3>) {
+      gather_words3<KERNEL, FLAVOUR>(P, ps, A.in, a, i, cx, cy, zc, W, acc, count);
+    } else {
+      gather_words_g<DIM, KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
+    }
+    acc.finish();
+  }
+  finish_target<DIM, FLAVOUR, KIND, FINAL>(A, tank, i, in_range, fluid, acc, count, vmax, dtmin);
+}
+
 // The per-wave reductions of one chunk's targets (all of one tank).
 template <int KIND, bool FINAL>
 __device__ __forceinline__ void reduce_chunk(const StageArgs& A, uint32_t tank, float vmax,
@@ -810,6 +640,43 @@ __device__ __forceinline__ void chunk_targets(const StageArgs& A, const ChunkInf
                                                  i < c.t1, ps, vmax, dtmin);
   reduce_chunk<KIND, FINAL>(A, c.t, vmax, dtmin, red);
 }
+
+// Chunk indices handed out to a persistent grid.  Launch index b runs on XCD
+// b % 8, whose eighth of the list is its band (so each XCD's L2 holds a
+// contiguous band of columns): a workgroup starts on its own slot of the band
+// and then draws from the band's counter, and when the band is finished from
+// the other bands'.  A fixed share per workgroup left the 2M-particle 2D
+// launch waiting: workgroups ended between 209 and 329 us.  The counters
+// (kWorkStride apart, one cache line each) are cleared before the launch.
+struct ChunkQueue {
+  uint32_t n, slots, q;
+  __device__ __forceinline__ uint32_t band_end(uint32_t x) const {
+    return static_cast<uint32_t>((static_cast<uint64_t>(n) * (x + 1)) / 8);
+  }
+  __device__ __forceinline__ uint32_t band_begin(uint32_t x) const {
+    return static_cast<uint32_t>((static_cast<uint64_t>(n) * x) / 8);
+  }
+  // The workgroup's first chunk, ~0 if there is none (then no other band
+  // has chunks left to draw either: every band is as long, to within one).
+  __device__ __forceinline__ void init(uint32_t n_chunks) {
+    n = n_chunks;
+    slots = gridDim.x >> 3;
+    const uint32_t x = blockIdx.x & 7u;
+    q = band_begin(x) + (blockIdx.x >> 3);
+    if (q >= band_end(x)) q = ~0u;
+  }
+  // The next chunk, ~0 when there is none left (one thread).
+  __device__ __forceinline__ uint32_t draw(uint32_t* work) const {
+    for (uint32_t k = 0; k < 8; ++k) {
+      const uint32_t x = (blockIdx.x + k) & 7u;
+      const uint32_t b = band_begin(x) + slots, e = band_end(x);
+      if (b >= e) continue;
+      const uint32_t r = atomicAdd(work + x * kWorkStride, 1u);
+      if (r < e - b) return b + r;
+    }
+    return ~0u;
+  }
+};
 
 struct Band {
   uint32_t lo, hi, step;

@@ -1,106 +1,32 @@
 // Fused SSPRK stage kernel: continuity + momentum pair sums, EOS, update.
 //
-// Work unit: a chunk of at most chunk_targets consecutive (cell-sorted)
-// particles of one cell column of one tank, one particle per lane.  After
-// every cell rebuild the chunks are recut on the device so that each column's
-// particles split into equal chunks; a persistent grid then walks the chunk
-// list in XCD-major bands (launch index b runs on XCD b % 8 and takes chunks
-// from that XCD's eighth of the list, so each XCD's L2 holds a contiguous
-// band of columns).
-//
-// 2D: the FP64 positions of the chunk's candidates (the 5 neighbouring
-// columns, the chunk's rows +- 2) are staged in LDS.  Each lane walks its own
-// 5 x 5 cell stencil one column range at a time: the exact FP64 predicate
-// (four LDS loads per batch) builds a 64-bit acceptance mask per batch, queued
-// in registers; then the FP32 pair terms run over the accepted candidates of all
-// batches in one loop, reading their pair records (velocity, m/rho,
-// rho - rho0 and p/rho^2, cs) from L2 one candidate ahead of the arithmetic.
-// Chunks whose candidates exceed the LDS capacity, and 3D, take positions
-// from global memory too.  Every path visits candidates in the same order and
-// rounds identically, so all schedules produce the same bits.
+// Two families of work units, both recut on the device after every cell
+// rebuild and walked by a persistent grid in XCD-major bands (launch index b
+// runs on XCD b % 8 and takes chunks from that XCD's eighth of the list, so
+// each XCD's L2 holds a contiguous band of columns):
+//  - block chunks (schedules with LDS): the particles of a block of cell
+//    columns over a few rows, the block's window staged in LDS.  2D: the
+//    tile kernel of stage_tile.hip; 3D: k_stage_lds3 below;
+//  - column chunks (schedules without LDS): at most chunk_targets consecutive
+//    (cell-sorted) particles of one cell column, positions from global memory.
+// Every path visits a target's candidates in the same order and rounds
+// identically, so all schedules produce the same bits.
 #include "stage_common.hpp"
 
 namespace tit_amd {
 
 namespace {
 
-// 2D chunks with LDS-staged positions; chunks that do not fit go to the
-// overflow list.  18 KB of LDS and at most 128 VGPRs: four waves per SIMD.
-template <int KERNEL, int FLAVOUR, int KIND, bool FINAL, int NT, int CAP>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_stage_lds(
+// Column chunks with positions from global memory (schedules without LDS).
+template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_stage_global(
     StageArgs A) {
-  __shared__ double2 s_xy[CAP];
-  __shared__ uint32_t s_coff[kCols2][kRowsMax + 1];
-  __shared__ uint32_t s_gb[kCols2], s_lb[kCols2 + 1];
-  __shared__ int s_fits;
-  __shared__ uint32_t s_gbase;
-  const int tid = threadIdx.x;
+  __shared__ uint32_t s_wm[NT / 64][kWordsG * 64];
+  __shared__ uint32_t s_wj[NT / 64][kWordsG * 64];
   const Band band = xcd_band(A.counts[0]);
   WaveReduce red;
   for (uint32_t q = band.lo; q < band.hi; q += band.step) {
-    const ChunkInfo c = chunk_info<2>(A, q);
-    const int zf = static_cast<int>(A.key[c.t0] - c.col_row);
-    const int zl = static_cast<int>(A.key[c.t1 - 1] - c.col_row);
-    const int zlo = max(zf - kStencil, 0), zhi = min(zl + kStencil, c.nz - 1);
-    const int nrows = zhi - zlo + 1;
-    __syncthreads();  // the previous chunk's LDS reads are done
-    const bool rows_fit = nrows <= kRowsMax;
-    if (rows_fit) {
-      for (int r = tid; r < kCols2 * (nrows + 1); r += NT) {
-        const int k = r / (nrows + 1), row = r % (nrows + 1);
-        const int ixk = c.cx - kStencil + k;
-        s_coff[k][row] =
-            (ixk >= 0 && ixk < c.T.nc[0])
-                ? A.cell_off[c.T.cell_off + static_cast<uint32_t>(ixk) * c.nz + zlo + row]
-                : 0u;
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t lb = 0, g0 = ~0u, g1 = 0;
-      if (rows_fit) {
-        for (int k = 0; k < kCols2; ++k) {
-          s_gb[k] = s_coff[k][0];
-          s_lb[k] = lb;
-          lb += s_coff[k][nrows] - s_coff[k][0];
-          const int ixk = c.cx - kStencil + k;
-          if (ixk >= 0 && ixk < c.T.nc[0]) {
-            g0 = min(g0, s_coff[k][0]);
-            g1 = max(g1, s_coff[k][nrows]);
-          }
-        }
-        s_lb[kCols2] = lb;
-        s_gbase = g0;
-      }
-      s_fits = rows_fit && lb <= A.lds_cap && g1 - g0 < kWordSpan;
-      if (!s_fits) A.overflow[atomicAdd(A.counts + 1, 1u)] = q;
-    }
-    __syncthreads();
-    if (!s_fits) continue;
-    const uint32_t total = s_lb[kCols2];
-    for (uint32_t l = tid; l < total; l += NT) {
-      int k = 0;
-      while (l >= s_lb[k + 1]) ++k;
-      const uint32_t j = s_gb[k] + (l - s_lb[k]);
-      s_xy[l] = make_double2(A.in.x[0][j], A.in.x[1][j]);
-    }
-    __syncthreads();
-    const LdsPos ps{s_xy, s_coff, s_gb, s_lb, zlo, c.nz, c.cx, c.T.nc[0], s_gbase};
-    chunk_targets<2, KERNEL, FLAVOUR, KIND, FINAL>(A, c, ps, red);
-  }
-  red.flush(A);
-}
-
-// Chunks with positions from global memory: 3D, and 2D overflow chunks.
-template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_stage_global(
-    StageArgs A, const uint32_t* list, const uint32_t* count) {
-  __shared__ uint32_t s_wm[NT / 64][kWordsG * 64];
-  __shared__ uint32_t s_wj[NT / 64][kWordsG * 64];
-  const Band band = xcd_band(*count);
-  WaveReduce red;
-  for (uint32_t q = band.lo; q < band.hi; q += band.step) {
-    const ChunkInfo c = chunk_info<DIM>(A, list ? list[q] : q);
+    const ChunkInfo c = chunk_info<DIM>(A, q);
     const GlobalPos<DIM> ps{c.T,  A.in, A.cell_off, c.cx, c.cy, s_wm[threadIdx.x >> 6],
                             s_wj[threadIdx.x >> 6]};
     chunk_targets<DIM, KERNEL, FLAVOUR, KIND, FINAL>(A, c, ps, red);
@@ -300,67 +226,107 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void
   red.flush(A);
 }
 
-// Block chunks of one block (one 64-lane workgroup per block): the targets of
-// each row over the block's columns, then lane 0 cuts the rows greedily into
-// chunks of at most kStage3Threads targets spanning at most kChunkRows3 rows
-// (a single row with more targets forms a chunk of its own), skipping empty
-// rows at a chunk's ends.  With emit, the chunks are written from the
-// block's scanned offset; otherwise the count goes to bcount.
+// Block chunks of one block (one wave per block).  Greedy from the block's
+// first row: a chunk takes as many rows as keep its targets, its window's
+// candidates and its rows within their limits, the lanes testing the possible
+// end rows at once; rows without targets are skipped at both ends.  A single
+// row beyond a limit forms a chunk of its own that does not fit the LDS (the
+// 3D kernel finds those itself).  T(z) and W(z): particles of the block's and
+// of the window's columns below row z, each a sum of cell offsets (differences
+// are the counts), for a segment of rows in LDS.  With emit, the chunks are
+// written from the block's scanned offset; otherwise the count goes to bcount.
+struct ChunkLimits {
+  uint32_t targets, window;
+  int rows;
+};
+
+template <int DIM>
+__host__ __device__ __forceinline__ ChunkLimits chunk_limits(uint32_t chunk_targets,
+                                                             uint32_t lds_cap) {
+  if (DIM == 2) {
+    // chunk_targets scales the tile from its full size at kChunkMax
+    const uint32_t t = chunk_targets * kTileThreads / kChunkMax;
+    // of the LDS entries, those between the window's columns hold no candidate
+    constexpr uint32_t pad = kTilePad * (kBlk2 + 2 * kStencil);
+    const uint32_t cap = lds_cap < kTileCap ? lds_cap : kTileCap;
+    return ChunkLimits{t > 1u ? t : 1u, cap > pad ? cap - pad : 1u, kChunkRows2};
+  }
+  return ChunkLimits{kStage3Threads, ~0u, kChunkRows3};
+}
+
+constexpr int kSegRows = 256;
+
+template <int DIM>
 __global__ __launch_bounds__(64) void k_block_chunks(StageArgs A, int emit, const uint32_t* ctl) {
   if (!ctl[0]) return;
-  __shared__ uint32_t s_t[64];
+  constexpr int BX = DIM == 2 ? kBlk2 : kBlk3, BY = DIM == 2 ? 1 : kBlk3;
+  constexpr int S = kStencil, SY = DIM == 2 ? 0 : kStencil;
+  __shared__ uint32_t s_T[kSegRows + 2 * S + 1], s_W[kSegRows + 2 * S + 1];
+  const ChunkLimits lim = chunk_limits<DIM>(A.chunk_targets, A.lds_cap);
   const uint32_t b = blockIdx.x;
   const uint4 blk = A.blocks[b];
   const DevTank T = A.tanks[blk.x];
-  const int nz = T.nc[2];
+  const int nz = T.nc[DIM - 1], ny = DIM == 2 ? 1 : T.nc[1];
   const int bx = static_cast<int>(blk.y), by = static_cast<int>(blk.z);
   const int lane = threadIdx.x;
-  int start = -1, last = -1;
-  uint32_t cur = 0, count = 0;
   const uint32_t base = emit ? A.bcount[b] : 0u;
-  auto close = [&]() {
-    if (emit) A.bchunks[base + count] = make_uint4(b, start, last + 1, cur);
-    ++count;
+  int seg = 0;  // s_T[k], s_W[k]: row seg - S + k, clamped to [0, nz]
+  auto load = [&](int z) {
+    seg = z;
+    __syncthreads();
+    for (int k = lane; k < kSegRows + 2 * S + 1; k += 64) {
+      const uint32_t row = static_cast<uint32_t>(min(max(seg - S + k, 0), nz));
+      uint32_t t = 0, w = 0;
+      for (int dx = -S; dx < BX + S; ++dx) {
+        for (int dy = -SY; dy < BY + SY; ++dy) {
+          const int ix = bx + dx, iy = by + dy;
+          if (ix < 0 || ix >= T.nc[0] || iy < 0 || iy >= ny) continue;
+          const uint32_t v =
+              A.cell_off[T.cell_off + (static_cast<uint32_t>(ix) * ny + iy) * nz + row];
+          w += v;
+          if (dx >= 0 && dx < BX && dy >= 0 && dy < BY) t += v;
+        }
+      }
+      s_T[k] = t;
+      s_W[k] = w;
+    }
+    __syncthreads();
   };
-  for (int z0 = 0; z0 < nz; z0 += 64) {
-    const int z = z0 + lane;
-    uint32_t tz = 0;
-    if (z < nz) {
-      for (int q = 0; q < kBlk3 * kBlk3; ++q) {
-        const int ix = bx + q / kBlk3, iy = by + q % kBlk3;
-        if (ix < T.nc[0] && iy < T.nc[1]) {
-          const uint32_t row = column_row3(T, ix, iy);
-          tz += A.cell_off[row + z + 1] - A.cell_off[row + z];
-        }
-      }
+  auto Tz = [&](int z) { return s_T[min(z, nz) - seg + S]; };
+  auto Wz = [&](int z) { return s_W[min(max(z, 0), nz) - seg + S]; };
+  load(0);
+  uint32_t count = 0;
+  int z = 0;
+  while (z < nz) {  // uniform over the wave
+    if (z + 64 > seg + kSegRows) load(z);
+    // rows z .. z + 63 with targets
+    uint64_t m = __ballot(Tz(z + lane + 1) != Tz(z + lane));
+    if (m == 0) {
+      z += 64;
+      continue;
     }
-    s_t[lane] = tz;
-    __syncthreads();
-    if (lane == 0) {
-      const int rows = min(64, nz - z0);
-      for (int r = 0; r < rows; ++r) {
-        const uint32_t t = s_t[r];
-        if (t == 0) continue;
-        const int zz = z0 + r;
-        if (start >= 0 && (cur + t > static_cast<uint32_t>(kStage3Threads) ||
-                           zz - start + 1 > kChunkRows3)) {
-          close();
-          start = -1;
-        }
-        if (start < 0) {
-          start = zz;
-          cur = 0;
-        }
-        cur += t;
-        last = zz;
-      }
+    const int skip = __builtin_ctzll(m);
+    if (skip > 0) {
+      z += skip;
+      continue;
     }
-    __syncthreads();
+    // end rows z + 1 .. z + 64; the tests hold up to the chunk's end
+    const int e = z + 1 + lane;
+    const bool ok = lane < lim.rows && e <= nz && Tz(e) - Tz(z) <= lim.targets &&
+                    Wz(e + S) - Wz(z - S) <= lim.window;
+    const uint64_t fit = ~__ballot(ok);
+    const int rows = max(1, static_cast<int>(__builtin_ctzll(fit)));
+    const uint32_t over = (fit & 1ull) ? 1u : 0u;
+    m &= rows < 64 ? (1ull << rows) - 1ull : ~0ull;
+    const int end = z + 64 - __builtin_clzll(m);
+    if (emit && lane == 0) {
+      A.bchunks[base + count] = DIM == 2 ? make_uint4(blk.x | over << 31, blk.y, z, end)
+                                         : make_uint4(b, z, end, over);
+    }
+    ++count;
+    z = end;
   }
-  if (lane == 0) {
-    if (start >= 0) close();
-    if (!emit) A.bcount[b] = count;
-  }
+  if (lane == 0 && !emit) A.bcount[b] = count;
 }
 
 // ---- chunk list (after every cell rebuild) ----------------------------------
@@ -551,7 +517,8 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_emit(StageArgs A,
   }
 }
 
-// Clears an overflow count (counts[1] of the pair given).
+// Clears the count of the 3D block chunks that do not fit (counts[1] of the
+// pair given).
 __global__ void k_reset_overflow(uint32_t* counts) { counts[1] = 0u; }
 
 // ---- dispatch -------------------------------------------------------------------
@@ -560,21 +527,17 @@ constexpr int kThreads = kChunkMax;
 
 template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL>
 void launch_kind(hipStream_t s, const StageArgs& a) {
-  if constexpr (DIM == 2) {
-    k_reset_overflow<<<1, 1, 0, s>>>(a.counts);
-    k_stage_lds<KERNEL, FLAVOUR, KIND, FINAL, kThreads, kStageLdsCap>
-        <<<a.grid_lds, kThreads, 0, s>>>(a);
-    k_stage_global<2, KERNEL, FLAVOUR, KIND, FINAL, kThreads>
-        <<<a.grid_global, kThreads, 0, s>>>(a, a.overflow, a.counts + 1);
-  } else if (a.lds_cap > 0 && a.n_blocks > 0) {
-    k_reset_overflow<<<1, 1, 0, s>>>(a.counts + 2);
-    k_stage_lds3<KERNEL, FLAVOUR, KIND, FINAL, kStage3Threads, kStage3LdsCap>
-        <<<a.grid_lds3, kStage3Threads, 0, s>>>(a);
-    k_stage_block_global<KERNEL, FLAVOUR, KIND, FINAL, kThreads>
-        <<<a.grid_block_global, kThreads, 0, s>>>(a);
+  if (DIM == 3 && a.lds_cap > 0) {
+    if constexpr (DIM == 3) {
+      k_reset_overflow<<<1, 1, 0, s>>>(a.counts + 2);
+      k_stage_lds3<KERNEL, FLAVOUR, KIND, FINAL, kStage3Threads, kStage3LdsCap>
+          <<<a.grid_lds3, kStage3Threads, 0, s>>>(a);
+      k_stage_block_global<KERNEL, FLAVOUR, KIND, FINAL, kThreads>
+          <<<a.grid_block_global, kThreads, 0, s>>>(a);
+    }
   } else {
-    k_stage_global<3, KERNEL, FLAVOUR, KIND, FINAL, kThreads>
-        <<<a.grid_global, kThreads, 0, s>>>(a, nullptr, a.counts);
+    k_stage_global<DIM, KERNEL, FLAVOUR, KIND, FINAL, kThreads>
+        <<<a.grid_global, kThreads, 0, s>>>(a);
   }
 }
 
@@ -583,11 +546,7 @@ void dispatch_kind(hipStream_t s, const StageArgs& a, int kind, bool final) {
   if (kind == kRhsOnly) {
     launch_kind<DIM, KERNEL, FLAVOUR, kRhsOnly, false>(s, a);
   } else if (kind == kEuler) {
-    if (final) {
-      launch_kind<DIM, KERNEL, FLAVOUR, kEuler, true>(s, a);
-    } else {
-      launch_kind<DIM, KERNEL, FLAVOUR, kEuler, false>(s, a);
-    }
+    launch_kind<DIM, KERNEL, FLAVOUR, kEuler, false>(s, a);
   } else {
     if (final) {
       launch_kind<DIM, KERNEL, FLAVOUR, kCombine, true>(s, a);
@@ -634,7 +593,7 @@ uint32_t stage_lds_capacity(int dim) { return dim == 2 ? kStageLdsCap : kStage3L
 void stage_grids(const DevParams& P, int n_cu, StageGrids* g) {
   int bl = 1, bg, b3 = 1, bb = 1;
   if (P.dim == 2) {
-    bl = occupancy(k_stage_lds<kKernelC2, kFlavourCfg, kCombine, false, kThreads, kStageLdsCap>);
+    bl = tile_groups_per_cu();
     bg = occupancy(k_stage_global<2, kKernelC2, kFlavourCfg, kCombine, false, kThreads>);
   } else {
     bg = occupancy(k_stage_global<3, kKernelC2, kFlavourCfg, kCombine, false, kThreads>);
@@ -645,7 +604,7 @@ void stage_grids(const DevParams& P, int n_cu, StageGrids* g) {
   }
   // multiples of 8: every XCD owns the same number of slots
   auto grid = [&](int per_cu) { return 8u * static_cast<uint32_t>((per_cu * n_cu + 7) / 8); };
-  g->lds = grid(bl);
+  g->tile = grid(bl);
   g->global = grid(bg);
   g->lds3 = grid(b3);
   g->block_global = grid(bb);
@@ -653,21 +612,47 @@ void stage_grids(const DevParams& P, int n_cu, StageGrids* g) {
 
 void launch_build_chunks(hipStream_t s, const StageArgs& a, uint32_t* block_tot,
                          const uint32_t* ctl) {
-  const uint32_t nb = (a.n_cols + kColsPerBlock - 1) / kColsPerBlock;
-  if (nb == 0) return;
-  k_chunk_count<<<nb, kScanBlock, 0, s>>>(a, block_tot, ctl);
-  k_chunk_base<<<1, kScanBlock, 0, s>>>(block_tot, nb, a.counts, ctl);
-  k_chunk_emit<<<nb, kScanBlock, 0, s>>>(a, block_tot, ctl);
-  if (a.P.dim == 3 && a.n_blocks > 0) {
-    k_block_chunks<<<a.n_blocks, 64, 0, s>>>(a, 0, ctl);
+  if (a.n_cols == 0) return;
+  if (a.lds_cap > 0) {
+    if (a.P.dim == 2) {
+      k_block_chunks<2><<<a.n_blocks, 64, 0, s>>>(a, 0, ctl);
+    } else {
+      k_block_chunks<3><<<a.n_blocks, 64, 0, s>>>(a, 0, ctl);
+    }
     k_chunk_base<<<1, kScanBlock, 0, s>>>(a.bcount, a.n_blocks, a.counts + 2, ctl);
-    k_block_chunks<<<a.n_blocks, 64, 0, s>>>(a, 1, ctl);
+    if (a.P.dim == 2) {
+      k_block_chunks<2><<<a.n_blocks, 64, 0, s>>>(a, 1, ctl);
+    } else {
+      k_block_chunks<3><<<a.n_blocks, 64, 0, s>>>(a, 1, ctl);
+    }
+  } else {
+    const uint32_t nb = (a.n_cols + kColsPerBlock - 1) / kColsPerBlock;
+    k_chunk_count<<<nb, kScanBlock, 0, s>>>(a, block_tot, ctl);
+    k_chunk_base<<<1, kScanBlock, 0, s>>>(block_tot, nb, a.counts, ctl);
+    k_chunk_emit<<<nb, kScanBlock, 0, s>>>(a, block_tot, ctl);
   }
+}
+
+// A chunk ends because the next row with targets would pass a limit.  By the
+// target limit at most 2 n / targets times (two neighbouring chunks together
+// pass it); by the row limit nz / rows times per block; by the window limit at
+// most 14 n / window times: a particle is in the windows of at most two blocks
+// per blocked axis and, along the rows, of at most seven chunks with their
+// next row (those that begin within a stencil of it).  One more chunk per
+// block.
+size_t block_chunk_bound(int dim, size_t n, size_t n_blocks, size_t nz, uint32_t chunk_targets,
+                         uint32_t lds_cap) {
+  if (dim == 3) return std::min(n, n_blocks * nz) + 1;
+  const ChunkLimits l = chunk_limits<2>(chunk_targets, std::max(lds_cap, 1u));
+  return std::min(n, 2 * n / l.targets + 14 * n / l.window +
+                         n_blocks * (nz / static_cast<size_t>(l.rows) + 2)) + 1;
 }
 
 void launch_stage(hipStream_t s, const StageArgs& a, int kind, bool final) {
   if (a.n == 0 || a.n_cols == 0) return;
-  if (a.P.dim == 2) {
+  if (a.P.dim == 2 && a.lds_cap > 0) {
+    launch_stage_tile(s, a, kind, final);
+  } else if (a.P.dim == 2) {
     dispatch_kernel<2>(s, a, kind, final);
   } else {
     dispatch_kernel<3>(s, a, kind, final);

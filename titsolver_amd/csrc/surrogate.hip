@@ -1059,7 +1059,7 @@ tit_status infer_current(tit_hip_ctx* c, RebuildMode mode) {
 tit_status learned_step(tit_hip_ctx* c) {
   constexpr double kFactor = 4.0;
   launch_step_begin(c->stream, c->n_tanks, c->dt_min, c->dt, c->vmax, c->disp,
-                    c->dp.skin_half, rebuild_ctl(c), kFactor);
+                    c->dp.skin_half, rebuild_ctl(c), c->work, kFactor);
   tit_status st = infer_current(c, kRebuildMarked);
   if (st != TIT_OK) return st;
   Learned* L = c->learned;
