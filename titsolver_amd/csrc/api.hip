@@ -261,6 +261,39 @@ void enqueue_rebuild(tit_hip_ctx* c, RebuildMode mode) {
   const RebuildCtl rc = rebuild_ctl(c);
   if (mode == kRebuildForce) launch_force_rebuild(s, c->n_tanks, rc);
   if (mode == kRebuildPending) launch_pending_rebuild(s, c->n_tanks, rc);
+  if (c->n <= kSmallN && c->n_cells <= kSmallCells) {
+    SmallRebuildArgs a{};
+    a.n = c->n;
+    a.n_cells = c->n_cells;
+    a.n_tanks = c->n_tanks;
+    a.key_bits = c->key_bits;
+    a.st = c->A;
+    a.tmp = c->T;
+    a.id_tmp = c->id_alt;
+    a.tag_tmp = c->tag_alt;
+    a.item = c->val;
+    a.key = c->key;
+    a.id = c->id;
+    a.tag = c->tag;
+    a.cell_off = c->cell_off;
+    a.fixed_list = c->fixed_list;
+    a.counter = c->counter;
+    a.flags = c->counter + 1;
+    a.cell_fluid = c->cell_fluid;
+    a.disp = c->disp;
+    a.rc = rc;
+    a.b = boundary_args(c, c->A);
+    a.s = stage_args(c);
+    {
+      ProfScope ps(c->prof, s, "rebuild_small");
+      launch_rebuild_small(s, a);
+    }
+    if (c->lds_cap == 0) {  // column chunks
+      ProfScope ps(c->prof, s, "build_chunks");
+      launch_build_chunks(s, a.s, c->block_tot, rc.ctl);
+    }
+    return;
+  }
   {
     ProfScope ps(c->prof, s, "cell_keys");
     launch_cell_keys(s, c->dp, c->tanks, c->n, c->A, c->tag, c->key, c->counter + 1, rc);

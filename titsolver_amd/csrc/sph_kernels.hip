@@ -8,6 +8,7 @@
 // reference's exactly, independent of how the cells were built.
 #include <algorithm>
 
+#include "index_common.hpp"
 #include "pair_math.hpp"
 #include "sph_kernels.hpp"
 
@@ -135,26 +136,8 @@ __global__ __launch_bounds__(kBlock) void k_cell_keys(
   const uint32_t t = tag[i] >> 1;
   if (!need[t]) return;  // the tank keeps its keys, hence its order
   const DevTank& T = tanks[t];
-  uint32_t flat = 0;
   bool bad = false;
-#pragma unroll
-  for (int k = 0; k < DIM; ++k) {
-    const double x = st.x[k][i];
-    const double f = (x - T.lo[k]) * T.inv_c[k];
-    int c;
-    if (!(f == f)) {
-      bad = true;
-      c = 0;
-    } else if (f <= 0.0) {
-      c = 0;
-    } else if (f >= static_cast<double>(T.nc[k] - 1)) {
-      c = T.nc[k] - 1;
-    } else {
-      c = static_cast<int>(f);
-    }
-    flat = flat * static_cast<uint32_t>(T.nc[k]) + static_cast<uint32_t>(c);
-  }
-  key[i] = T.cell_off + flat;
+  key[i] = cell_key<DIM>(T, [&](int k) { return st.x[k][i]; }, bad);
   if (bad) atomicOr(flags, 2u);
 }
 
@@ -298,22 +281,6 @@ constexpr int kBoundaryUnroll = 2;
 // fixed particles per workgroup of k_fixed_active (its LDS list)
 constexpr uint32_t kFixedPerBlock = 1024;
 
-// Cell coordinates (per axis) of particle i's cell in its tank.
-template <int DIM>
-__device__ __forceinline__ void cell_coords(const BoundaryArgs& A, const DevTank& T, uint32_t i,
-                                            int* c) {
-  const uint32_t local = A.key[i] - T.cell_off;
-  if constexpr (DIM == 2) {
-    c[0] = static_cast<int>(local / T.nc[1]);
-    c[1] = static_cast<int>(local % T.nc[1]);
-  } else {
-    const uint32_t q = local / T.nc[2];
-    c[2] = static_cast<int>(local % T.nc[2]);
-    c[1] = static_cast<int>(q % T.nc[1]);
-    c[0] = static_cast<int>(q / T.nc[1]);
-  }
-}
-
 // Whether a cell of the 5^d stencil around cell c held fluid at the last
 // rebuild; the G lanes of a group split the cells.
 template <int DIM, int G>
@@ -347,27 +314,6 @@ __device__ __forceinline__ bool stencil_has_fluid(const BoundaryArgs& A, const D
 #pragma unroll
   for (int off = G / 2; off > 0; off >>= 1) any |= __shfl_xor(any, off, G);
   return any != 0;
-}
-
-// The fixed particle's extrapolated state from the Shepard sums S and H.
-template <int DIM>
-__device__ __forceinline__ void write_fixed(const BoundaryArgs& A, uint32_t i, double S,
-                                            double H) {
-  const DevParams& P = A.P;
-  const double tiny = 6.0554544523933395e-06;  // cbrt(DBL_EPSILON)
-  const double Hs = fabs(S) <= tiny ? 0.0 : H / S;
-  const double rho_e = eos_density_from_potential(P, Hs);
-  A.s.rho[i] = rho_e;
-  const double zero[DIM] = {};
-  const double m_e = particle_mass(P, A.id[i]);
-  write_pair_data<DIM>(P, A.s, i, zero, rho_e, m_e);
-  if (A.wall_rho) {
-    const uint32_t k = A.id[i] - A.wall_id0;
-    A.wall_rho[k] = rho_e;
-    A.s.pv[i].z = static_cast<float>(A.wall_mu[k] * m_e / rho_e);  // V_e = m_e / rho_e
-  }
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) A.s.v[d][i] = 0.0;
 }
 
 // After a cell rebuild: lists the fixed particles with fluid in their
@@ -698,25 +644,56 @@ __global__ __launch_bounds__(kBlock) void k_time_step(
 
 __global__ void k_rebuild_clear(uint32_t* ctl) { ctl[0] = 0u; }
 
-// One wave per tank (the reduction slots' copies folded lane by lane).
-__global__ __launch_bounds__(64) void k_step_begin(unsigned long long* dt_min, double* dt,
-                                                   uint32_t* vmax, const double* disp,
-                                                   double skin_half, double span, uint32_t* ctl,
-                                                   uint32_t* need, uint32_t* work) {
-  const uint32_t t = blockIdx.x;
-  if (t == 0) {
-    for (uint32_t k = threadIdx.x; k < (kWorkSets - 1) * kWorkSet; k += 64) work[k] = 0u;
-  }
+// One wave per tank (the reduction slots' copies folded lane by lane): takes
+// the tank's step size and decides its rebuild.
+__device__ __forceinline__ bool begin_tank(uint32_t t, unsigned long long* dt_min, double* dt,
+                                           uint32_t* vmax, const double* disp, double skin_half,
+                                           double span, bool pending, uint32_t* need) {
   const unsigned long long b = red_fold<false>(dt_min, t, true);
   const uint32_t vb = red_fold<true>(vmax, t, true);
-  if (threadIdx.x != 0) return;
   // A tank without fluid keeps dt = 0 (nothing moves).
   const double h = b == ~0ull ? 0.0 : __longlong_as_double(static_cast<long long>(b));
-  dt[t] = h;
   const double vprev = static_cast<double>(__uint_as_float(vb));
-  const bool nd = ctl[1] != 0u || !(disp[t] + 2.0 * span * h * vprev <= 0.9 * skin_half);
-  need[t] = nd ? 1u : 0u;
-  if (nd) atomicOr(ctl, 1u);
+  const bool nd = pending || !(disp[t] + 2.0 * span * h * vprev <= 0.9 * skin_half);
+  if ((threadIdx.x & 63) == 0) {
+    dt[t] = h;
+    need[t] = nd ? 1u : 0u;
+  }
+  return nd;
+}
+
+__device__ __forceinline__ void clear_work_sets(uint32_t* work) {
+  for (uint32_t k = threadIdx.x; k < (kWorkSets - 1) * kWorkSet; k += blockDim.x) work[k] = 0u;
+}
+
+// Up to kBeginTanks tanks: one workgroup, which also sets ctl[0] (one launch
+// instead of a clear and an atomic per tank).
+constexpr int kBeginTanks = 256;
+__global__ __launch_bounds__(1024) void k_step_begin(int n_tanks, unsigned long long* dt_min,
+                                                     double* dt, uint32_t* vmax,
+                                                     const double* disp, double skin_half,
+                                                     double span, uint32_t* ctl, uint32_t* need,
+                                                     uint32_t* work) {
+  clear_work_sets(work);
+  const bool pending = ctl[1] != 0u;
+  int any = 0;
+  for (int t = threadIdx.x >> 6; t < n_tanks; t += blockDim.x >> 6) {
+    any |= begin_tank(t, dt_min, dt, vmax, disp, skin_half, span, pending, need) ? 1 : 0;
+  }
+  any = __syncthreads_or(any);
+  if (threadIdx.x == 0) ctl[0] = any ? 1u : 0u;
+}
+
+// More tanks: one workgroup each, ctl[0] cleared before.
+__global__ __launch_bounds__(64) void k_step_begin_many(unsigned long long* dt_min, double* dt,
+                                                        uint32_t* vmax, const double* disp,
+                                                        double skin_half, double span,
+                                                        uint32_t* ctl, uint32_t* need,
+                                                        uint32_t* work) {
+  const uint32_t t = blockIdx.x;
+  if (t == 0) clear_work_sets(work);
+  const bool nd = begin_tank(t, dt_min, dt, vmax, disp, skin_half, span, ctl[1] != 0u, need);
+  if (nd && threadIdx.x == 0) atomicOr(ctl, 1u);
 }
 
 __global__ void k_force_rebuild(int n_tanks, uint32_t* ctl, uint32_t* need) {
@@ -963,9 +940,15 @@ void launch_time_step(hipStream_t s, const DevParams& P, uint32_t n,
 void launch_step_begin(hipStream_t s, int n_tanks, unsigned long long* dt_min,
                        double* dt, uint32_t* vmax, const double* disp,
                        double skin_half, RebuildCtl rc, uint32_t* work, double span) {
-  k_rebuild_clear<<<1, 1, 0, s>>>(rc.ctl);
-  k_step_begin<<<n_tanks, 64, 0, s>>>(dt_min, dt, vmax, disp, skin_half, span, rc.ctl,
-                                      rc.need, work);
+  if (n_tanks <= kBeginTanks) {
+    const int threads = 64 * std::min(n_tanks, 16);
+    k_step_begin<<<1, threads, 0, s>>>(n_tanks, dt_min, dt, vmax, disp, skin_half, span, rc.ctl,
+                                       rc.need, work);
+  } else {
+    k_rebuild_clear<<<1, 1, 0, s>>>(rc.ctl);
+    k_step_begin_many<<<n_tanks, 64, 0, s>>>(dt_min, dt, vmax, disp, skin_half, span, rc.ctl,
+                                             rc.need, work);
+  }
 }
 
 __global__ void k_clear_work(uint32_t* set) { set[threadIdx.x] = 0u; }

@@ -181,6 +181,27 @@ struct RebuildCtl {
   unsigned long long* count;
 };
 
+// Rebuild of a small set in one launch (rebuild_small.hip): at most kSmallN
+// particles in kSmallCells cells.  Its arrays are those of the large form's
+// kernels; it also resets the displacements.
+constexpr uint32_t kSmallN = 32768;
+constexpr uint32_t kSmallCells = 65536;
+struct SmallRebuildArgs {
+  uint32_t n, n_cells;
+  int n_tanks, key_bits;
+  DevState st, tmp;  // the state; scratch
+  uint32_t *id_tmp, *tag_tmp, *item;
+  uint32_t *key, *id, *tag, *cell_off, *fixed_list;
+  uint32_t* counter;  // fixed, flags, listed
+  uint32_t* flags;
+  uint8_t* cell_fluid;
+  double* disp;
+  RebuildCtl rc;
+  BoundaryArgs b;
+  StageArgs s;        // chunk lists (block chunks only)
+};
+void launch_rebuild_small(hipStream_t s, const SmallRebuildArgs& a);
+
 // Kernel kinds of the stage launch.
 enum StageKind { kRhsOnly = 0, kEuler = 1, kCombine = 2 };
 

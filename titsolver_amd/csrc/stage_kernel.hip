@@ -11,6 +11,7 @@
 //    (cell-sorted) particles of one cell column, positions from global memory.
 // Every path visits a target's candidates in the same order and rounds
 // identically, so all schedules produce the same bits.
+#include "chunk_build.hpp"
 #include "stage_common.hpp"
 
 namespace tit_amd {
@@ -226,107 +227,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void
   red.flush(A);
 }
 
-// Block chunks of one block (one wave per block).  Greedy from the block's
-// first row: a chunk takes as many rows as keep its targets, its window's
-// candidates and its rows within their limits, the lanes testing the possible
-// end rows at once; rows without targets are skipped at both ends.  A single
-// row beyond a limit forms a chunk of its own that does not fit the LDS (the
-// 3D kernel finds those itself).  T(z) and W(z): particles of the block's and
-// of the window's columns below row z, each a sum of cell offsets (differences
-// are the counts), for a segment of rows in LDS.  With emit, the chunks are
-// written from the block's scanned offset; otherwise the count goes to bcount.
-struct ChunkLimits {
-  uint32_t targets, window;
-  int rows;
-};
-
-template <int DIM>
-__host__ __device__ __forceinline__ ChunkLimits chunk_limits(uint32_t chunk_targets,
-                                                             uint32_t lds_cap) {
-  if (DIM == 2) {
-    // chunk_targets scales the tile from its full size at kChunkMax
-    const uint32_t t = chunk_targets * kTileThreads / kChunkMax;
-    // of the LDS entries, those between the window's columns hold no candidate
-    constexpr uint32_t pad = kTilePad * (kBlk2 + 2 * kStencil);
-    const uint32_t cap = lds_cap < kTileCap ? lds_cap : kTileCap;
-    return ChunkLimits{t > 1u ? t : 1u, cap > pad ? cap - pad : 1u, kChunkRows2};
-  }
-  return ChunkLimits{kStage3Threads, ~0u, kChunkRows3};
-}
-
-constexpr int kSegRows = 256;
-
+// One wave per block; with emit from the block's scanned offset, otherwise the
+// count goes to bcount.
 template <int DIM>
 __global__ __launch_bounds__(64) void k_block_chunks(StageArgs A, int emit, const uint32_t* ctl) {
   if (!ctl[0]) return;
-  constexpr int BX = DIM == 2 ? kBlk2 : kBlk3, BY = DIM == 2 ? 1 : kBlk3;
-  constexpr int S = kStencil, SY = DIM == 2 ? 0 : kStencil;
-  __shared__ uint32_t s_T[kSegRows + 2 * S + 1], s_W[kSegRows + 2 * S + 1];
-  const ChunkLimits lim = chunk_limits<DIM>(A.chunk_targets, A.lds_cap);
+  __shared__ ChunkScratch sc;
   const uint32_t b = blockIdx.x;
-  const uint4 blk = A.blocks[b];
-  const DevTank T = A.tanks[blk.x];
-  const int nz = T.nc[DIM - 1], ny = DIM == 2 ? 1 : T.nc[1];
-  const int bx = static_cast<int>(blk.y), by = static_cast<int>(blk.z);
-  const int lane = threadIdx.x;
-  const uint32_t base = emit ? A.bcount[b] : 0u;
-  int seg = 0;  // s_T[k], s_W[k]: row seg - S + k, clamped to [0, nz]
-  auto load = [&](int z) {
-    seg = z;
-    __syncthreads();
-    for (int k = lane; k < kSegRows + 2 * S + 1; k += 64) {
-      const uint32_t row = static_cast<uint32_t>(min(max(seg - S + k, 0), nz));
-      uint32_t t = 0, w = 0;
-      for (int dx = -S; dx < BX + S; ++dx) {
-        for (int dy = -SY; dy < BY + SY; ++dy) {
-          const int ix = bx + dx, iy = by + dy;
-          if (ix < 0 || ix >= T.nc[0] || iy < 0 || iy >= ny) continue;
-          const uint32_t v =
-              A.cell_off[T.cell_off + (static_cast<uint32_t>(ix) * ny + iy) * nz + row];
-          w += v;
-          if (dx >= 0 && dx < BX && dy >= 0 && dy < BY) t += v;
-        }
-      }
-      s_T[k] = t;
-      s_W[k] = w;
-    }
-    __syncthreads();
-  };
-  auto Tz = [&](int z) { return s_T[min(z, nz) - seg + S]; };
-  auto Wz = [&](int z) { return s_W[min(max(z, 0), nz) - seg + S]; };
-  load(0);
-  uint32_t count = 0;
-  int z = 0;
-  while (z < nz) {  // uniform over the wave
-    if (z + 64 > seg + kSegRows) load(z);
-    // rows z .. z + 63 with targets
-    uint64_t m = __ballot(Tz(z + lane + 1) != Tz(z + lane));
-    if (m == 0) {
-      z += 64;
-      continue;
-    }
-    const int skip = __builtin_ctzll(m);
-    if (skip > 0) {
-      z += skip;
-      continue;
-    }
-    // end rows z + 1 .. z + 64; the tests hold up to the chunk's end
-    const int e = z + 1 + lane;
-    const bool ok = lane < lim.rows && e <= nz && Tz(e) - Tz(z) <= lim.targets &&
-                    Wz(e + S) - Wz(z - S) <= lim.window;
-    const uint64_t fit = ~__ballot(ok);
-    const int rows = max(1, static_cast<int>(__builtin_ctzll(fit)));
-    const uint32_t over = (fit & 1ull) ? 1u : 0u;
-    m &= rows < 64 ? (1ull << rows) - 1ull : ~0ull;
-    const int end = z + 64 - __builtin_clzll(m);
-    if (emit && lane == 0) {
-      A.bchunks[base + count] = DIM == 2 ? make_uint4(blk.x | over << 31, blk.y, z, end)
-                                         : make_uint4(b, z, end, over);
-    }
-    ++count;
-    z = end;
-  }
-  if (lane == 0 && !emit) A.bcount[b] = count;
+  const uint32_t n = block_chunks<DIM>(A, b, emit != 0, emit ? A.bcount[b] : 0u, sc);
+  if (threadIdx.x == 0 && !emit) A.bcount[b] = n;
 }
 
 // ---- chunk list (after every cell rebuild) ----------------------------------
