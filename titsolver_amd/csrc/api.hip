@@ -455,19 +455,14 @@ tit_status build_schedule(tit_hip_ctx* c) {
                                          c->chunk_targets, c->lds_cap);
   if (bneed > c->bchunk_cap) {
     forget(c, c->bchunks);
-    forget(c, c->boverflow);
     c->bchunks = nullptr;
-    c->boverflow = nullptr;
     TIT_HIP_TRY(c, dalloc(c, &c->bchunks, bneed));
-    if (dim == 3) TIT_HIP_TRY(c, dalloc(c, &c->boverflow, bneed));
     c->bchunk_cap = bneed;
   }
   StageGrids g;
   stage_grids(c->dp, c->n_cu, &g);
   c->grid_tile = g.tile;
   c->grid_global = g.global;
-  c->grid_lds3 = g.lds3;
-  c->grid_block_global = g.block_global;
   drop_graph(c);
   if (c->rebuild_ctl) {
     // the chunk list follows the schedule: recut it from the current cell
@@ -492,10 +487,7 @@ StageArgs stage_args(tit_hip_ctx* c) {
   a.blocks = c->blocks;
   a.n_blocks = c->n_blocks;
   a.bchunks = c->bchunks;
-  a.boverflow = c->boverflow;
   a.bcount = c->bcount;
-  a.grid_lds3 = c->grid_lds3;
-  a.grid_block_global = c->grid_block_global;
   a.P = c->dp;
   a.tanks = c->tanks;
   a.key = c->key;
@@ -1136,7 +1128,6 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   c->chunk_counts = nullptr;
   c->blocks = nullptr;
   c->bchunks = nullptr;
-  c->boverflow = nullptr;
   c->bcount = nullptr;
   c->n_blocks = 0;
   c->bchunk_cap = 0;

@@ -21,7 +21,7 @@ __host__ __device__ __forceinline__ ChunkLimits chunk_limits(uint32_t chunk_targ
     const uint32_t cap = lds_cap < kTileCap ? lds_cap : kTileCap;
     return ChunkLimits{t > 1u ? t : 1u, cap > pad ? cap - pad : 1u, kChunkRows2};
   }
-  return ChunkLimits{kStage3Threads, ~0u, kChunkRows3};
+  return ChunkLimits{kStage3Threads, lds_cap * kTile3Cap / kStage3LdsCap, kChunkRows3};
 }
 
 constexpr int kSegRows = 256;
@@ -42,8 +42,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // first row: a chunk takes as many rows as keep its targets, its window's
 // candidates and its rows within their limits, the lanes testing the possible
 // end rows at once; rows without targets are skipped at both ends.  A single
-// row beyond a limit forms a chunk of its own that does not fit the LDS (the
-// 3D kernel finds those itself).  T(z) and W(z): particles of the block's and
+// row beyond a limit forms a chunk of its own that does not fit the LDS.  T(z) and W(z): particles of the block's and
 // of the window's columns below row z, each a sum of cell offsets (differences
 // are the counts), for a segment of rows in LDS.  With emit, the chunks are
 // written from `base` on.  Returns their number.

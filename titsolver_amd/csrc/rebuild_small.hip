@@ -249,10 +249,7 @@ __global__ __launch_bounds__(NT) void k_rebuild_small(SmallRebuildArgs R) {
     for (uint32_t b = wave; b < A.n_blocks; b += kWaves) {
       (void)block_chunks<DIM>(A, b, true, A.bcount[b], chunk_scratch[wave]);
     }
-    if (tid == 0) {
-      A.counts[2] = before;
-      A.counts[3] = 0u;
-    }
+    if (tid == 0) A.counts[2] = before;
   }
   for (int t = tid; t < R.n_tanks; t += NT) {
     if (R.rc.need[t]) R.disp[t] = 0.0;

@@ -26,22 +26,21 @@ constexpr int kTilePad = 3;
 constexpr int kTileWaves = 3;
 // Stencil columns of a 2D target.
 constexpr int kCols2 = 2 * kStencil + 1;
-// 3D block chunks: the cell columns of a tank in blocks of kBlk3 x kBlk3;
-// a chunk holds the particles of one block in a range of at most
-// kChunkRows3 rows, at most kStage3Threads of them (a row with more goes to
-// the global-memory kernel whole).  Its window is the block grown by the
-// stencil (kWin3 x kWin3 columns, kRows3 rows), FP64 positions of at most
-// kStage3LdsCap candidates staged in LDS.
+// 3D tiles (stage_tile3.hip): the cell columns of a tank in blocks of kBlk3 x
+// kBlk3; a chunk holds the particles of one block in a range of at most
+// kChunkRows3 rows, at most kStage3Threads of them.  Its window is the block
+// grown by the stencil (kWin3 x kWin3 columns, kRows3 rows), FP64 positions of
+// at most kTile3Cap candidates staged in LDS.  A full chunk of the 3D dam
+// break spans 5 rows, its window about 64 x 9 x 2.9 = 1,680 candidates; with
+// these limits a workgroup takes just under 80 KB, two per CU.
 constexpr int kBlk3 = 4;
 constexpr int kWin3 = kBlk3 + 2 * kStencil;
 constexpr int kChunkRows3 = 6;
 constexpr int kRows3 = kChunkRows3 + 2 * kStencil;
-constexpr int kWords3 = 6;
 constexpr int kStage3Threads = 256;
-// (a chunk of 256 targets in the 3D dam break spans 5-6 rows of 16 columns,
-// so its window holds about 64 x 9.5 x 2.9 = 1,800 candidates, and one of 6
-// rows at most 64 x 10 x 2.9 = 1,860; 2,048 candidates keep the workgroup's
-// LDS under 53 KB: three workgroups of four waves per CU)
+constexpr int kTile3Cap = 1860;
+constexpr int kTile3List = 64;
+// the largest LDS capacity a 3D schedule may name (all of kTile3Cap)
 constexpr int kStage3LdsCap = 2048;
 
 // Counters of the chunk queue (stage_common.hpp): one set of 8 per stage of a
@@ -79,23 +78,18 @@ struct StageArgs {
   uint32_t chunk_targets;
   uint32_t lds_cap;            // candidate positions staged in LDS at most
   uint4* chunks;
-  // [0] column chunks, [2] block chunks, [3] 3D block chunks that take the
-  // global-memory kernel
-  uint32_t* counts;
+  uint32_t* counts;            // [0] column chunks, [2] block chunks
   uint32_t grid_tile, grid_global;  // persistent grid sizes
   uint32_t* work;                   // this launch's set of chunk-queue counters
   // with LDS staging (lds_cap > 0): cell-column blocks (tank, first ix,
   // first iy, 0), rebuilt on the device after every cell rebuild: block
   // chunks (2D: tank | does not fit the LDS << 31, first ix, first row, end
-  // row; 3D: block, first row, end row, does not fit),
-  // per-block chunk counts (scanned in place), and the 3D block chunks that
-  // do not fit
+  // row; 3D: block, first row, end row, does not fit) and per-block chunk
+  // counts (scanned in place)
   const uint4* blocks;
   uint32_t n_blocks;
   uint4* bchunks;
-  uint32_t* boverflow;
   uint32_t* bcount;
-  uint32_t grid_lds3, grid_block_global;
   double* dv_last[3];          // final stage: its acceleration (post-integration only)
   // semi-analytic wall (kFlavourWall): per slot, the face terms of drho/dt
   // and dv/dt already divided by gamma, then gamma
@@ -281,9 +275,12 @@ size_t block_chunk_bound(int dim, size_t n, size_t n_blocks, size_t nz, uint32_t
 // stage_tile.hip: the 2D stage over tiles, and its workgroups resident per CU.
 void launch_stage_tile(hipStream_t s, const StageArgs& a, int kind, bool final);
 int tile_groups_per_cu();
+// stage_tile3.hip: the 3D stage over tiles.
+void launch_stage_tile3(hipStream_t s, const StageArgs& a, int kind, bool final);
+int tile3_groups_per_cu();
 // Persistent grid sizes of the stage kernels (multiples of 8 workgroups).
 struct StageGrids {
-  uint32_t tile, global, lds3, block_global;
+  uint32_t tile, global;
 };
 void stage_grids(const DevParams& P, int n_cu, StageGrids* g);
 // Rebuilds the chunk list from the cell offsets (after a cell rebuild).

@@ -1,7 +1,7 @@
-// Device code shared by the stage kernels (stage_kernel.hip: 2D and the
-// column-chunk global path; stage3d.hip: 3D block chunks): candidate
-// accessors, the per-target stencil walk with acceptance masks, the pair
-// loops, the per-target SSPRK update and the per-wave reductions.  Every
+// Device code shared by the stage kernels (stage_kernel.hip: the column-chunk
+// global path; stage_tile.hip, stage_tile3.hip: tiles): pair inputs, the
+// global path's stencil walk with acceptance masks and pair loop, the
+// per-target SSPRK update, the per-wave reductions and the chunk queue.  Every
 // path visits a target's candidates in the same order and rounds
 // identically, so all schedules produce the same bits.
 #pragma once
@@ -231,189 +231,6 @@ __device__ __forceinline__ void gather_words_g(const DevParams& P, const GlobalP
   }
 }
 
-// Positions from LDS, 3D block chunks.  A chunk's targets are the particles
-// of a block of kBlk3 x kBlk3 cell columns in a range of rows; its window is
-// the block grown by the stencil, kWin3 x kWin3 columns over rows
-// [zlo, zlo + nrows).  Each window column's candidates sit contiguously in
-// LDS from lb[kw] on (FP64 x, y, z in three arrays), and delta[kw] turns an
-// LDS index of column kw into the particle's global index.
-struct LdsPos3 {
-  const double* sx;
-  const double* sy;
-  const double* sz;
-  const uint32_t (*coff)[kRows3 + 1];  // [window column][row - zlo]: global index
-  const uint32_t* lb;
-  const uint32_t* delta;
-  int zlo, nz, wx0, wy0, ncx, ncy;
-
-  // LDS range of stencil column k of target column (cx, cy), rows [w0, w1]
-  // (inside the target's 5-row window, so inside the chunk's window).
-  __device__ __forceinline__ bool range(int cx, int cy, int k, int w0, int w1, uint32_t& b,
-                                        uint32_t& e, int& kw) const {
-    const int ix = cx - kStencil + k / kCols2, iy = cy - kStencil + k % kCols2;
-    if (ix < 0 || ix >= ncx || iy < 0 || iy >= ncy) return false;
-    const int z0 = max(w0, 0), z1 = min(w1, nz - 1);
-    if (z0 > z1) return false;
-    kw = (ix - wx0) * kWin3 + (iy - wy0);
-    const uint32_t base = coff[kw][0];
-    b = lb[kw] + (coff[kw][z0 - zlo] - base);
-    e = lb[kw] + (coff[kw][z1 + 1 - zlo] - base);
-    return true;
-  }
-};
-
-// gather_words3's words, queued per lane in registers: 32-bit acceptance mask
-// | LDS index of its bit 0 << 32 | window column << 48 (never an empty mask).
-struct WordQueue3 {
-  uint64_t w[kWords3];  // oldest first
-
-  // Appends at slot n (a run-time index: one select per slot).
-  __device__ __forceinline__ void put(int n, uint64_t v) {
-#pragma unroll
-    for (int q = 0; q < kWords3; ++q) {
-      if (q == n) w[q] = v;
-    }
-  }
-  // Removes the oldest word.
-  __device__ __forceinline__ uint64_t pop() {
-    const uint64_t v = w[0];
-#pragma unroll
-    for (int q = 0; q + 1 < kWords3; ++q) w[q] = w[q + 1];
-    return v;
-  }
-};
-
-// The pair loop of gather_words3's queued words (as sum_words_g).
-template <int KERNEL, int FLAVOUR>
-__device__ __forceinline__ void sum_words3(const DevParams& P, const LdsPos3& ps,
-                                           const DevState& S, const Target<3>& a,
-                                           uint32_t n_acc, Sums<3>& acc, WordQueue3& wq) {
-  uint32_t m = 0, l0 = 0, d0 = 0;
-  // the next of the n_acc accepted candidates
-  auto take = [&](PairIn<3>& p) {
-    if (m == 0) {
-      const uint64_t next = wq.pop();
-      m = static_cast<uint32_t>(next);
-      l0 = static_cast<uint32_t>(next >> 32) & 0xFFFFu;
-      d0 = ps.delta[static_cast<uint32_t>(next >> 48)];
-    }
-    const uint32_t l = l0 + static_cast<uint32_t>(__builtin_ctz(m));
-    m &= m - 1u;
-    p.x[0] = ps.sx[l];
-    p.x[1] = ps.sy[l];
-    p.x[2] = ps.sz[l];
-    const uint32_t j = l + d0;
-    p.pv = S.pv[j];
-    p.aux = S.aux[j];
-    p.vol = mass_flavour(FLAVOUR) ? S.vol[j] : 0.0f;
-  };
-  uint32_t rem = n_acc;
-  PairIn<3> A, B;
-  if (rem == 0) return;
-  if (acc.pend) {  // an odd term of an earlier batch of words waits for its partner
-    take(A);
-    sum_pair<3, KERNEL, FLAVOUR>(P, a, A, acc);
-    if (--rem == 0) return;
-  }
-  take(A);
-  --rem;
-  while (true) {
-    const bool hb = rem > 0;
-    if (hb) {
-      take(B);
-      --rem;
-    }
-    float ca, fa[3];
-    term_of<3, KERNEL, FLAVOUR>(P, a, A, ca, fa);
-    if (!hb) {
-      acc.add(ca, fa);
-      break;
-    }
-    const bool ha = rem > 0;
-    if (ha) {
-      take(A);
-      --rem;
-    }
-    float cb, fb[3];
-    term_of<3, KERNEL, FLAVOUR>(P, a, B, cb, fb);
-    acc.add2(ca, fa, cb, fb);
-    if (!ha) break;
-  }
-}
-
-// 3D with LDS positions: the global path's walk (stencil columns in order,
-// 32-candidate masks), the predicate reading the staged positions, up to
-// kWords3 masks per pair loop.
-template <int KERNEL, int FLAVOUR>
-__device__ __forceinline__ void gather_words3(const DevParams& P, const LdsPos3& ps,
-                                              const DevState& S, const Target<3>& a,
-                                              uint32_t i, int cx, int cy, int zc,
-                                              const Windows<3, kCols2 * kCols2>& W,
-                                              Sums<3>& acc, uint32_t& count) {
-  constexpr int NCOL = kCols2 * kCols2;
-  WordQueue3 wq;
-  int k = 0, kw = 0;
-  uint32_t c0 = 0, e = 0;
-  bool more = true;
-  while (more) {
-    int nw = 0;
-    uint32_t n_acc = 0;
-    while (nw < kWords3) {
-      if (c0 >= e) {  // next non-empty column range
-        bool found = false;
-        for (; k < NCOL && !found; ++k) {
-          const uint32_t v = W.get(k);
-          if ((v & 7u) == 7u) continue;
-          const int w0 = zc - kStencil + static_cast<int>(v & 7u);
-          const int w1 = zc - kStencil + static_cast<int>(v >> 3);
-          uint32_t b, eb;
-          int kk;
-          if (ps.range(cx, cy, k, w0, w1, b, eb, kk) && b < eb) {
-            found = true;
-            c0 = b;
-            e = eb;
-            kw = kk;
-          }
-        }
-        if (!found) {
-          more = false;
-          break;
-        }
-      }
-      const uint32_t len = min(e - c0, 32u);
-      uint32_t mask = 0;
-      uint32_t t = 0;
-      for (; t + 4 <= len; t += 4) {
-        const double x0[3] = {ps.sx[c0 + t], ps.sy[c0 + t], ps.sz[c0 + t]};
-        const double x1[3] = {ps.sx[c0 + t + 1], ps.sy[c0 + t + 1], ps.sz[c0 + t + 1]};
-        const double x2[3] = {ps.sx[c0 + t + 2], ps.sy[c0 + t + 2], ps.sz[c0 + t + 2]};
-        const double x3[3] = {ps.sx[c0 + t + 3], ps.sy[c0 + t + 3], ps.sz[c0 + t + 3]};
-        const uint32_t mm = (within<3>(P, x0, a.x) ? 1u : 0u) |
-                            (within<3>(P, x1, a.x) ? 2u : 0u) |
-                            (within<3>(P, x2, a.x) ? 4u : 0u) |
-                            (within<3>(P, x3, a.x) ? 8u : 0u);
-        mask |= mm << t;
-      }
-      for (; t < len; ++t) {
-        const double x0[3] = {ps.sx[c0 + t], ps.sy[c0 + t], ps.sz[c0 + t]};
-        if (within<3>(P, x0, a.x)) mask |= 1u << t;
-      }
-      const uint32_t g0 = c0 + ps.delta[kw];  // global index of bit 0
-      if (i >= g0 && i < g0 + len) mask &= ~(1u << (i - g0));  // not self
-      const uint32_t na = static_cast<uint32_t>(__builtin_popcount(mask));
-      count += na;
-      n_acc += na;
-      if (mask) {
-        wq.put(nw, static_cast<uint64_t>(mask) | (static_cast<uint64_t>(c0) << 32) |
-                       (static_cast<uint64_t>(kw) << 48));
-        ++nw;
-      }
-      c0 += len;
-    }
-    sum_words3<KERNEL, FLAVOUR>(P, ps, S, a, n_acc, acc, wq);
-  }
-}
-
 __device__ __forceinline__ float wave_max_f32(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
@@ -478,13 +295,40 @@ __device__ __forceinline__ ChunkInfo chunk_info(const StageArgs& A, uint32_t q) 
   return c;
 }
 
+// What finish_target reads of particle i, loaded together (loaded where each
+// value is used, the 2M-particle 2D launch takes 295 us instead of 285).
+template <int DIM>
+struct TargetState {
+  double x[DIM], v[DIM], rho;
+  double ox[DIM], ov[DIM], orho;  // the step's start (combination stages)
+  double dt;
+};
+
+template <int DIM, int KIND>
+__device__ __forceinline__ void load_target(const StageArgs& A, uint32_t tank, uint32_t i,
+                                            TargetState<DIM>& t) {
+#pragma unroll
+  for (int k = 0; k < DIM; ++k) {
+    t.x[k] = A.in.x[k][i];
+    t.v[k] = A.in.v[k][i];
+    if constexpr (KIND == kCombine) {
+      t.ox[k] = A.old.x[k][i];
+      t.ov[k] = A.old.v[k][i];
+    }
+  }
+  t.rho = A.in.rho[i];
+  if constexpr (KIND == kCombine) t.orho = A.old.rho[i];
+  if constexpr (KIND != kRhsOnly) t.dt = A.dt[tank];
+}
+
 // After the pair sums of one target (one lane): particle i's right-hand side
 // (KIND kRhsOnly), or the SSPRK substep / combination of
 // time_integrator.hpp:188-223 in FP64 and, on the last stage, the next step's
 // CFL candidate.  Fixed particles keep their state.  The lane's speed and CFL
 // candidate come back in vmax and dtmin for the per-wave reductions.
 template <int DIM, int FLAVOUR, int KIND, bool FINAL>
-__device__ __forceinline__ void finish_target(const StageArgs& A, uint32_t tank, uint32_t i,
+__device__ __forceinline__ void finish_target(const StageArgs& A,
+                                              const TargetState<DIM>& t, uint32_t i,
                                               bool in_range, bool fluid, const Sums<DIM>& acc,
                                               uint32_t count, float& vmax,
                                               unsigned long long& dtmin) {
@@ -510,13 +354,8 @@ __device__ __forceinline__ void finish_target(const StageArgs& A, uint32_t tank,
     }
   }
   if (fluid) {
-    double xa[DIM], va[DIM];
-#pragma unroll
-    for (int k = 0; k < DIM; ++k) {
-      xa[k] = A.in.x[k][i];
-      va[k] = A.in.v[k][i];
-    }
-    const double rho_a = A.in.rho[i];
+    const double *xa = t.x, *va = t.v;
+    const double rho_a = t.rho;
     if constexpr (KIND == kRhsOnly) {
       if (A.rhs_count) A.rhs_count[i] = count;
     }
@@ -545,7 +384,7 @@ __device__ __forceinline__ void finish_target(const StageArgs& A, uint32_t tank,
 #pragma unroll
       for (int k = 0; k < DIM; ++k) v2 = v2 + va[k] * va[k];
       vmax = static_cast<float>(sqrt(v2));
-      const double h = A.dt[tank];
+      const double h = t.dt;
       double rn[DIM], vn[DIM];
 #pragma unroll
       for (int k = 0; k < DIM; ++k) {
@@ -557,10 +396,10 @@ __device__ __forceinline__ void finish_target(const StageArgs& A, uint32_t tank,
         const double wn = A.w, wo = 1.0 - A.w;
 #pragma unroll
         for (int k = 0; k < DIM; ++k) {
-          rn[k] = wo * A.old.x[k][i] + wn * rn[k];
-          vn[k] = wo * A.old.v[k][i] + wn * vn[k];
+          rn[k] = wo * t.ox[k] + wn * rn[k];
+          vn[k] = wo * t.ov[k] + wn * vn[k];
         }
-        rhon = wo * A.old.rho[i] + wn * rhon;
+        rhon = wo * t.orho + wn * rhon;
       }
 #pragma unroll
       for (int k = 0; k < DIM; ++k) {
@@ -582,7 +421,7 @@ __device__ __forceinline__ void finish_target(const StageArgs& A, uint32_t tank,
 
 // One target (one lane), particle i of cell column (cx, cy) of tank `tank`
 // (col_row: the global index of the column's first cell), by the column-chunk
-// and 3D paths.
+// path.
 template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, class Pos>
 __device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T,
                                             uint32_t tank, int cx, int cy, uint32_t col_row,
@@ -595,6 +434,7 @@ __device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T
   Sums<DIM> acc;
   acc.init();
   uint32_t count = 0;
+  TargetState<DIM> ts;
   if (fluid) {
     double xa[DIM], va[DIM];
 #pragma unroll
@@ -607,14 +447,11 @@ __device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T
     const int zc = static_cast<int>(A.key[i] - col_row);
     const Windows<DIM, NCOL> W =
         stencil_windows<DIM, NCOL>(P, T, xa, cx, cy, zc);
-    if constexpr (std::is_same_v<Pos, LdsPos3>) {
-      gather_words3<KERNEL, FLAVOUR>(P, ps, A.in, a, i, cx, cy, zc, W, acc, count);
-    } else {
-      gather_words_g<DIM, KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
-    }
+    gather_words_g<DIM, KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
     acc.finish();
+    load_target<DIM, KIND>(A, tank, i, ts);
   }
-  finish_target<DIM, FLAVOUR, KIND, FINAL>(A, tank, i, in_range, fluid, acc, count, vmax, dtmin);
+  finish_target<DIM, FLAVOUR, KIND, FINAL>(A, ts, i, in_range, fluid, acc, count, vmax, dtmin);
 }
 
 // The per-wave reductions of one chunk's targets (all of one tank).
@@ -650,6 +487,7 @@ __device__ __forceinline__ void chunk_targets(const StageArgs& A, const ChunkInf
 // (kWorkStride apart, one cache line each) are cleared before the launch.
 struct ChunkQueue {
   uint32_t n, slots, q;
+  uint32_t k;  // bands given up so far (the own one first)
   __device__ __forceinline__ uint32_t band_end(uint32_t x) const {
     return static_cast<uint32_t>((static_cast<uint64_t>(n) * (x + 1)) / 8);
   }
@@ -661,17 +499,29 @@ struct ChunkQueue {
   __device__ __forceinline__ void init(uint32_t n_chunks) {
     n = n_chunks;
     slots = gridDim.x >> 3;
+    k = 0;
     const uint32_t x = blockIdx.x & 7u;
     q = band_begin(x) + (blockIdx.x >> 3);
     if (q >= band_end(x)) q = ~0u;
   }
-  // The next chunk, ~0 when there is none left (one thread).
-  __device__ __forceinline__ uint32_t draw(uint32_t* work) const {
-    for (uint32_t k = 0; k < 8; ++k) {
+  // One thread draws: take() asks the current band's counter, before a
+  // chunk's last part, so that the answer arrives during it (asked at the
+  // chunk's start, every workgroup would hold a chunk it cannot begin, and
+  // where a launch has few rounds the idle ones would find none left); next()
+  // turns the answer into the next chunk, ~0 when every band is finished.  A
+  // finished band is not asked again: 768 workgroups asking it for every
+  // chunk wait for each other (11.5 ns per atomic on one address).
+  __device__ __forceinline__ uint32_t take(uint32_t* work) const {
+    const uint32_t x = (blockIdx.x + k) & 7u;
+    if (k >= 8 || band_begin(x) + slots >= band_end(x)) return ~0u;  // no second round
+    return atomicAdd(work + x * kWorkStride, 1u);
+  }
+  __device__ __forceinline__ uint32_t next(uint32_t* work, uint32_t r) {
+    for (bool asked = true; k < 8; ++k, asked = false) {
       const uint32_t x = (blockIdx.x + k) & 7u;
       const uint32_t b = band_begin(x) + slots, e = band_end(x);
       if (b >= e) continue;
-      const uint32_t r = atomicAdd(work + x * kWorkStride, 1u);
+      if (!asked) r = atomicAdd(work + x * kWorkStride, 1u);
       if (r < e - b) return b + r;
     }
     return ~0u;

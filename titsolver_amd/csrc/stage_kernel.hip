@@ -5,8 +5,8 @@
 // runs on XCD b % 8 and takes chunks from that XCD's eighth of the list, so
 // each XCD's L2 holds a contiguous band of columns):
 //  - block chunks (schedules with LDS): the particles of a block of cell
-//    columns over a few rows, the block's window staged in LDS.  2D: the
-//    tile kernel of stage_tile.hip; 3D: k_stage_lds3 below;
+//    columns over a few rows, the block's window staged in LDS: the tile
+//    kernels of stage_tile.hip (2D) and stage_tile3.hip (3D);
 //  - column chunks (schedules without LDS): at most chunk_targets consecutive
 //    (cell-sorted) particles of one cell column, positions from global memory.
 // Every path visits a target's candidates in the same order and rounds
@@ -31,198 +31,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void
     const GlobalPos<DIM> ps{c.T,  A.in, A.cell_off, c.cx, c.cy, s_wm[threadIdx.x >> 6],
                             s_wj[threadIdx.x >> 6]};
     chunk_targets<DIM, KERNEL, FLAVOUR, KIND, FINAL>(A, c, ps, red);
-  }
-  red.flush(A);
-}
-
-// ---- 3D block chunks ------------------------------------------------------------
-
-struct BlockChunk {
-  uint32_t tank;
-  DevTank T;
-  int bx, by;    // first cell column of the block
-  int zs, ze;    // the chunk's rows [zs, ze)
-  uint32_t n;    // targets
-};
-
-__device__ __forceinline__ BlockChunk block_chunk(const StageArgs& A, uint32_t q) {
-  const uint4 ch = A.bchunks[q];
-  const uint4 blk = A.blocks[ch.x];
-  BlockChunk c;
-  c.tank = blk.x;
-  c.T = A.tanks[c.tank];
-  c.bx = static_cast<int>(blk.y);
-  c.by = static_cast<int>(blk.z);
-  c.zs = static_cast<int>(ch.y);
-  c.ze = static_cast<int>(ch.z);
-  c.n = ch.w;
-  return c;
-}
-
-// Global index of the first cell of column (ix, iy) of tank T.
-__device__ __forceinline__ uint32_t column_row3(const DevTank& T, int ix, int iy) {
-  return T.cell_off + (static_cast<uint32_t>(ix) * T.nc[1] + static_cast<uint32_t>(iy)) *
-                          static_cast<uint32_t>(T.nc[2]);
-}
-
-// Target t of a block chunk (s_tb: prefix of the targets over the block's
-// kBlk3 x kBlk3 columns): its particle index and column.
-__device__ __forceinline__ void block_target(const BlockChunk& c, const uint32_t* s_tb,
-                                             const uint32_t* s_first, uint32_t t, uint32_t& i,
-                                             int& cx, int& cy) {
-  int q = 0;
-  while (q + 1 < kBlk3 * kBlk3 && t >= s_tb[q + 1]) ++q;
-  i = s_first[q] + (t - s_tb[q]);
-  cx = c.bx + q / kBlk3;
-  cy = c.by + q % kBlk3;
-}
-
-// 3D chunks with LDS-staged positions: the block's window (kWin3 x kWin3
-// columns, the chunk's rows +- 2) in LDS, one target per thread.  Chunks whose
-// window has more rows or candidates than the LDS holds, or more targets
-// than threads, go to the overflow list.
-template <int KERNEL, int FLAVOUR, int KIND, bool FINAL, int NT, int CAP>
-__global__ __launch_bounds__(NT) void k_stage_lds3(StageArgs A) {
-  constexpr int NW = kWin3 * kWin3;
-  constexpr int NB = kBlk3 * kBlk3;
-  __shared__ double s_x[CAP], s_y[CAP], s_z[CAP];
-  __shared__ uint32_t s_coff[NW][kRows3 + 1];
-  __shared__ uint32_t s_lb[NW + 1], s_delta[NW];
-  __shared__ uint32_t s_tb[NB + 1], s_first[NB];
-  __shared__ int s_fits;
-  const int tid = threadIdx.x;
-  const Band band = xcd_band(A.counts[2]);
-  WaveReduce red;
-  for (uint32_t q = band.lo; q < band.hi; q += band.step) {
-    const BlockChunk c = block_chunk(A, q);
-    const int nz = c.T.nc[2];
-    const int zlo = max(c.zs - kStencil, 0), zhi = min(c.ze - 1 + kStencil, nz - 1);
-    const int nrows = zhi - zlo + 1;
-    const int wx0 = c.bx - kStencil, wy0 = c.by - kStencil;
-    __syncthreads();  // the previous chunk's LDS reads are done
-    const bool rows_fit = nrows <= kRows3;
-    if (rows_fit) {
-      for (int r = tid; r < NW * (nrows + 1); r += NT) {
-        const int kw = r / (nrows + 1), row = r % (nrows + 1);
-        const int ix = wx0 + kw / kWin3, iy = wy0 + kw % kWin3;
-        const bool in = ix >= 0 && ix < c.T.nc[0] && iy >= 0 && iy < c.T.nc[1];
-        s_coff[kw][row] = in ? A.cell_off[column_row3(c.T, ix, iy) + zlo + row] : 0u;
-      }
-    }
-    __syncthreads();
-    static_assert(NW == 64, "one lane of the first wave per window column");
-    if (tid < 64) {
-      // wave 0: LDS offsets of the window columns (lane = column) and the
-      // targets of the block's columns (lanes 0..NB-1), by shuffle scans
-      uint32_t len = 0, nb = 0, first = 0;
-      if (rows_fit) {
-        len = s_coff[tid][nrows] - s_coff[tid][0];
-        if (tid < NB) {
-          const int kw = (kStencil + tid / kBlk3) * kWin3 + kStencil + tid % kBlk3;
-          first = s_coff[kw][c.zs - zlo];
-          nb = s_coff[kw][c.ze - zlo] - first;
-        }
-      }
-      uint32_t sl = len, sb = nb;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t yl = __shfl_up(sl, off), yb = __shfl_up(sb, off);
-        if (tid >= off) {
-          sl += yl;
-          sb += yb;
-        }
-      }
-      s_lb[tid] = sl - len;
-      s_delta[tid] = s_coff[tid][0] - (sl - len);
-      if (tid < NB) {
-        s_tb[tid] = sb - nb;
-        s_first[tid] = first;
-      }
-      const uint32_t lb = __shfl(sl, 63), nt = __shfl(sb, 63);
-      if (tid == 0) {
-        s_lb[NW] = lb;
-        s_tb[NB] = nt;
-        s_fits = rows_fit && lb <= A.lds_cap && nt <= static_cast<uint32_t>(NT);
-        if (!s_fits) A.boverflow[atomicAdd(A.counts + 3, 1u)] = q;
-      }
-    }
-    __syncthreads();
-    if (!s_fits) continue;
-    // each window column's candidates by 32 lanes (a column holds about 30)
-    for (int r = tid; r < NW * 32; r += NT) {
-      const int kw = r >> 5;
-      const uint32_t e = s_lb[kw + 1], d = s_delta[kw];
-      for (uint32_t l = s_lb[kw] + (r & 31); l < e; l += 32) {
-        const uint32_t j = l + d;
-        s_x[l] = A.in.x[0][j];
-        s_y[l] = A.in.x[1][j];
-        s_z[l] = A.in.x[2][j];
-      }
-    }
-    __syncthreads();
-    const LdsPos3 ps{s_x, s_y, s_z, s_coff, s_lb, s_delta, zlo, nz, wx0, wy0,
-                     c.T.nc[0], c.T.nc[1]};
-    const uint32_t t = static_cast<uint32_t>(tid);
-    const bool in_range = t < s_tb[NB];
-    uint32_t i = 0;
-    int cx = c.bx, cy = c.by;
-    if (in_range) block_target(c, s_tb, s_first, t, i, cx, cy);
-    float vmax;
-    unsigned long long dtmin;
-    target_step<3, KERNEL, FLAVOUR, KIND, FINAL>(A, c.T, c.tank, cx, cy,
-                                                 column_row3(c.T, cx, cy), i, in_range, ps,
-                                                 vmax, dtmin);
-    reduce_chunk<KIND, FINAL>(A, c.tank, vmax, dtmin, red);
-  }
-  red.flush(A);
-}
-
-// The block chunks that did not fit, positions from global memory, in rounds
-// of NT targets.
-template <int KERNEL, int FLAVOUR, int KIND, bool FINAL, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_stage_block_global(
-    StageArgs A) {
-  constexpr int NB = kBlk3 * kBlk3;
-  __shared__ uint32_t s_wm[NT / 64][kWordsG * 64];
-  __shared__ uint32_t s_wj[NT / 64][kWordsG * 64];
-  __shared__ uint32_t s_tb[NB + 1], s_first[NB];
-  const Band band = xcd_band(A.counts[3]);
-  WaveReduce red;
-  for (uint32_t q = band.lo; q < band.hi; q += band.step) {
-    const BlockChunk c = block_chunk(A, A.boverflow[q]);
-    __syncthreads();  // the previous chunk's table reads are done
-    if (threadIdx.x == 0) {
-      uint32_t nt = 0;
-      for (int b = 0; b < NB; ++b) {
-        const int ix = c.bx + b / kBlk3, iy = c.by + b % kBlk3;
-        uint32_t f = 0, e = 0;
-        if (ix < c.T.nc[0] && iy < c.T.nc[1]) {
-          const uint32_t row = column_row3(c.T, ix, iy);
-          f = A.cell_off[row + c.zs];
-          e = A.cell_off[row + c.ze];
-        }
-        s_tb[b] = nt;
-        s_first[b] = f;
-        nt += e - f;
-      }
-      s_tb[NB] = nt;
-    }
-    __syncthreads();
-    for (uint32_t base = 0; base < s_tb[NB]; base += NT) {
-      const uint32_t t = base + threadIdx.x;
-      const bool in_range = t < s_tb[NB];
-      uint32_t i = 0;
-      int cx = c.bx, cy = c.by;
-      if (in_range) block_target(c, s_tb, s_first, t, i, cx, cy);
-      const GlobalPos<3> ps{c.T, A.in, A.cell_off, cx, cy, s_wm[threadIdx.x >> 6],
-                            s_wj[threadIdx.x >> 6]};
-      float vmax;
-      unsigned long long dtmin;
-      target_step<3, KERNEL, FLAVOUR, KIND, FINAL>(A, c.T, c.tank, cx, cy,
-                                                   column_row3(c.T, cx, cy), i, in_range, ps,
-                                                   vmax, dtmin);
-      reduce_chunk<KIND, FINAL>(A, c.tank, vmax, dtmin, red);
-    }
   }
   red.flush(A);
 }
@@ -426,28 +234,13 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_emit(StageArgs A,
   }
 }
 
-// Clears the count of the 3D block chunks that do not fit (counts[1] of the
-// pair given).
-__global__ void k_reset_overflow(uint32_t* counts) { counts[1] = 0u; }
-
 // ---- dispatch -------------------------------------------------------------------
 
 constexpr int kThreads = kChunkMax;
 
 template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL>
 void launch_kind(hipStream_t s, const StageArgs& a) {
-  if (DIM == 3 && a.lds_cap > 0) {
-    if constexpr (DIM == 3) {
-      k_reset_overflow<<<1, 1, 0, s>>>(a.counts + 2);
-      k_stage_lds3<KERNEL, FLAVOUR, KIND, FINAL, kStage3Threads, kStage3LdsCap>
-          <<<a.grid_lds3, kStage3Threads, 0, s>>>(a);
-      k_stage_block_global<KERNEL, FLAVOUR, KIND, FINAL, kThreads>
-          <<<a.grid_block_global, kThreads, 0, s>>>(a);
-    }
-  } else {
-    k_stage_global<DIM, KERNEL, FLAVOUR, KIND, FINAL, kThreads>
-        <<<a.grid_global, kThreads, 0, s>>>(a);
-  }
+  k_stage_global<DIM, KERNEL, FLAVOUR, KIND, FINAL, kThreads><<<a.grid_global, kThreads, 0, s>>>(a);
 }
 
 template <int DIM, int KERNEL, int FLAVOUR>
@@ -500,23 +293,18 @@ int occupancy(F* f, int threads = kThreads) {
 uint32_t stage_lds_capacity(int dim) { return dim == 2 ? kStageLdsCap : kStage3LdsCap; }
 
 void stage_grids(const DevParams& P, int n_cu, StageGrids* g) {
-  int bl = 1, bg, b3 = 1, bb = 1;
+  int bt, bg;
   if (P.dim == 2) {
-    bl = tile_groups_per_cu();
+    bt = tile_groups_per_cu();
     bg = occupancy(k_stage_global<2, kKernelC2, kFlavourCfg, kCombine, false, kThreads>);
   } else {
+    bt = tile3_groups_per_cu();
     bg = occupancy(k_stage_global<3, kKernelC2, kFlavourCfg, kCombine, false, kThreads>);
-    b3 = occupancy(k_stage_lds3<kKernelC2, kFlavourCfg, kCombine, false, kStage3Threads,
-                                kStage3LdsCap>,
-                   kStage3Threads);
-    bb = occupancy(k_stage_block_global<kKernelC2, kFlavourCfg, kCombine, false, kThreads>);
   }
   // multiples of 8: every XCD owns the same number of slots
   auto grid = [&](int per_cu) { return 8u * static_cast<uint32_t>((per_cu * n_cu + 7) / 8); };
-  g->tile = grid(bl);
+  g->tile = grid(bt);
   g->global = grid(bg);
-  g->lds3 = grid(b3);
-  g->block_global = grid(bb);
 }
 
 void launch_build_chunks(hipStream_t s, const StageArgs& a, uint32_t* block_tot,
@@ -551,7 +339,7 @@ void launch_build_chunks(hipStream_t s, const StageArgs& a, uint32_t* block_tot,
 // block.
 size_t block_chunk_bound(int dim, size_t n, size_t n_blocks, size_t nz, uint32_t chunk_targets,
                          uint32_t lds_cap) {
-  if (dim == 3) return std::min(n, n_blocks * nz) + 1;
+  if (dim == 3) return std::min(n, n_blocks * nz) + 1;  // a row or more each
   const ChunkLimits l = chunk_limits<2>(chunk_targets, std::max(lds_cap, 1u));
   return std::min(n, 2 * n / l.targets + 14 * n / l.window +
                          n_blocks * (nz / static_cast<size_t>(l.rows) + 2)) + 1;
@@ -559,8 +347,12 @@ size_t block_chunk_bound(int dim, size_t n, size_t n_blocks, size_t nz, uint32_t
 
 void launch_stage(hipStream_t s, const StageArgs& a, int kind, bool final) {
   if (a.n == 0 || a.n_cols == 0) return;
-  if (a.P.dim == 2 && a.lds_cap > 0) {
-    launch_stage_tile(s, a, kind, final);
+  if (a.lds_cap > 0) {
+    if (a.P.dim == 2) {
+      launch_stage_tile(s, a, kind, final);
+    } else {
+      launch_stage_tile3(s, a, kind, final);
+    }
   } else if (a.P.dim == 2) {
     dispatch_kernel<2>(s, a, kind, final);
   } else {

@@ -18,12 +18,12 @@
 // global-memory path (stage_common.hpp), so every schedule gives the same
 // bits.
 //
-// Bound: VALU issue, 93 % of it at 2M particles (1.52e8 wave instructions
-// per launch: about half in the pair loop, 43 per pair, and a third in the
-// predicate, 10.5 per candidate).  The 2M-particle dam break's launch takes
-// 296 us; strips of one column with acceptance masks in registers and the
+// Bound: VALU issue (93 % of it at 2M particles: 1.52e8 wave instructions per
+// launch, about half in the pair loop, 43 per pair, and a third in the
+// predicate, 10.5 per candidate) and close behind it the LDS, about 80 % busy.
+// The 2M-particle dam break's launch takes 285 us; strips of one column with acceptance masks in registers and the
 // records gathered from L2 took 361 us and 1.71e8 (95 per pair).  Of that,
-// drawing chunks from a queue instead of fixed shares gave 40 us.
+// drawing chunks from a queue instead of fixed shares gave 50 us.
 #include "stage_common.hpp"
 
 namespace tit_amd {
@@ -37,6 +37,11 @@ constexpr int NT = kTileThreads;
 // that a lane can test four candidates at a time past its range's end (past
 // it in the same column lie rows beyond the stencil, which fail it too).
 constexpr uint32_t kPad = kTilePad;
+
+// Pair records as plain vectors (arrays of the HIP vector classes go to
+// scratch memory here).
+typedef __attribute__((ext_vector_type(4))) float Rec4;
+typedef __attribute__((ext_vector_type(2))) float Rec2;
 
 struct TileChunk {
   uint32_t tank;
@@ -218,13 +223,13 @@ k_stage_tile(StageArgs A) {
   ChunkQueue queue;
   queue.init(A.counts[2]);
   WaveReduce red;
-  for (uint32_t q = queue.q; q != ~0u; q = queue.q) {
+  for (uint32_t q = queue.q; q != ~0u;) {
     const TileChunk c = tile_chunk(A, q);
     const DevTank& T = *c.T;
     const int nz = T.nc[1];
     const int zlo = max(c.zs - kStencil, 0), zhi = min(c.ze - 1 + kStencil, nz - 1);
     const int nrows = zhi - zlo + 1;
-    __syncthreads();  // the previous chunk's LDS reads are done
+    uint32_t drawn = ~0u;
     // target t of the chunk: its particle, column in the block, tag and row
     auto target_of = [&](uint32_t t, uint32_t& i, int& b, uint32_t& tag, int& zc) {
       i = 0;
@@ -283,12 +288,11 @@ k_stage_tile(StageArgs A) {
         s_row[k][row] = static_cast<uint16_t>(l);
       }
       const uint32_t total = s_lb[kWinC];
-      if (tid == 0) s_next = queue.draw(A.work);
       // every load of the window in flight before the first LDS write
       constexpr int kPer = (kTileCap + NT - 1) / NT;
       double2 gx[kPer];
-      float4 gp[kPer];
-      float2 ga[kPer];
+      Rec4 gp[kPer];
+      Rec2 ga[kPer];
       bool real[kPer];
 #pragma unroll
       for (int v = 0; v < kPer; ++v) {
@@ -299,16 +303,16 @@ k_stage_tile(StageArgs A) {
         real[v] = l + kPad < s_lb[k + 1];
         const uint32_t j = real[v] ? l + s_d[k] : 0u;  // (idle: any particle)
         gx[v] = make_double2(A.in.x[0][j], A.in.x[1][j]);
-        gp[v] = A.in.pv[j];
-        ga[v] = A.in.aux[j];
+        gp[v] = reinterpret_cast<const Rec4*>(A.in.pv)[j];
+        ga[v] = reinterpret_cast<const Rec2*>(A.in.aux)[j];
       }
 #pragma unroll
       for (int v = 0; v < kPer; ++v) {
         const uint32_t l = tid + v * NT;
         if (real[v]) {
           s_xy[l] = gx[v];
-          s_pv[l] = gp[v];
-          s_aux[l] = ga[v];
+          reinterpret_cast<Rec4*>(s_pv)[l] = gp[v];
+          reinterpret_cast<Rec2*>(s_aux)[l] = ga[v];
         } else if (l < total) {
           s_xy[l] = make_double2(1e300, 1e300);
         }
@@ -316,7 +320,6 @@ k_stage_tile(StageArgs A) {
       __syncthreads();
     } else {
       if (tid == 0) {
-        s_next = queue.draw(A.work);
         uint32_t nt = 0;
         for (int b = 0; b < kBlk2; ++b) {
           s_tb[b] = nt;
@@ -340,7 +343,7 @@ k_stage_tile(StageArgs A) {
       Sums<2> acc;
       acc.init();
       uint32_t count = 0;
-      if (!c.over) {
+      if (!c.over && __any(fluid)) {
         Target<2> a;
         // its LDS index, in its row's range (a valid one for an idle lane)
         const uint32_t self = in_range ? i - s_d[b + kStencil] : s_lb[kStencil];
@@ -401,7 +404,7 @@ k_stage_tile(StageArgs A) {
         }
         count += cnt;
         tile_flush<KERNEL, FLAVOUR, true>(P, tile, a, self8, cnt, acc);
-      } else if (fluid) {
+      } else if (c.over && fluid) {
         Target<2> a;
         target_of_record<FLAVOUR>(P, make_double2(A.in.x[0][i], A.in.x[1][i]), A.in.pv[i],
                                   A.in.aux[i], a);
@@ -409,11 +412,16 @@ k_stage_tile(StageArgs A) {
       }
       float vmax;
       unsigned long long dtmin;
-      finish_target<2, FLAVOUR, KIND, FINAL>(A, c.tank, i, in_range, fluid, acc, count, vmax,
+      if (tid == 0 && base + NT >= n_t) drawn = queue.take(A.work);
+      TargetState<2> ts;
+      load_target<2, KIND>(A, c.tank, i, ts);
+      finish_target<2, FLAVOUR, KIND, FINAL>(A, ts, i, in_range, fluid, acc, count, vmax,
                                              dtmin);
       reduce_chunk<KIND, FINAL>(A, c.tank, vmax, dtmin, red);
     }
-    queue.q = s_next;
+    if (tid == 0) s_next = queue.next(A.work, drawn);
+    __syncthreads();  // this chunk's LDS reads are done
+    q = s_next;
   }
   red.flush(A);
 }
