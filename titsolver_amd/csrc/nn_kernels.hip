@@ -110,36 +110,6 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
   }
 }
 
-__global__ void k_act_backward(int M, int N, const float* dy, int ld_dy,
-                                int group, const float* pre, float* dx32,
-                                bf16* dx16) {
-  const size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<size_t>(M) * N) return;
-  const size_t m = t / N, n = t % N;
-  const float g = dy[(m / group) * ld_dy + n] * nn_act_grad(pre[t]);
-  if (dx32) dx32[t] = g;
-  if (dx16) dx16[t] = static_cast<bf16>(g);
-}
-
-__global__ void k_group_sum(int rows, int N, int group, const float* in,
-                            float* out, bf16* out16, int ld16, int col16) {
-  const size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<size_t>(rows) * N) return;
-  const size_t r = t / N, n = t % N;
-  float s = 0.0f;
-  for (int k = 0; k < group; ++k) s += in[(r * group + k) * N + n];
-  if (out) out[t] = s;
-  if (out16) out16[r * ld16 + col16 + n] = static_cast<bf16>(s);
-}
-
-__global__ void k_scatter_add_rows(int M, int N, const float* in,
-                                   const uint32_t* idx, float* out) {
-  const size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<size_t>(M) * N) return;
-  const size_t m = t / N, n = t % N;
-  atomicAdd(out + static_cast<size_t>(idx[m]) * N + n, in[t]);
-}
-
 __global__ void k_column_sum(int M, int N, const float* in, float* col_sum) {
   // one block per 64 columns x 256 row slices
   const int n = blockIdx.x * 64 + (threadIdx.x & 63);
@@ -149,27 +119,6 @@ __global__ void k_column_sum(int M, int N, const float* in, float* col_sum) {
   float s = 0.0f;
   for (int m = slice * per; m < min(M, (slice + 1) * per); ++m) s += in[static_cast<size_t>(m) * N + n];
   atomicAdd(col_sum + n, s);
-}
-
-__global__ void k_to_bf16_block(int M, int N, const float* src, int lds, bf16* dst,
-                                int ldd, int col0) {
-  const size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<size_t>(M) * N) return;
-  const size_t m = t / N, n = t % N;
-  dst[m * ldd + col0 + n] = static_cast<bf16>(src[m * lds + n]);
-}
-
-__global__ void k_copy_cols(int M, int N, const float* src, int lds, int col0,
-                            float* dst, int ldd, int add) {
-  const size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<size_t>(M) * N) return;
-  const size_t m = t / N, n = t % N;
-  const float v = src[m * lds + col0 + n];
-  if (add) {
-    dst[m * ldd + n] += v;
-  } else {
-    dst[m * ldd + n] = v;
-  }
 }
 
 __global__ void k_adam(int n, float* w, bf16* w16, const float* g, float* m,
@@ -205,49 +154,10 @@ void gemm_bf16(hipStream_t s, const GemmArgs& g) {
   k_gemm<<<grid, 256, 0, s>>>(g);
 }
 
-void act_backward(hipStream_t s, int M, int N, const float* dy, int ld_dy,
-                   int group, const float* pre, float* dx32, bf16* dx16) {
-  const size_t n = static_cast<size_t>(M) * N;
-  if (n) {
-    k_act_backward<<<blocks(n), 256, 0, s>>>(M, N, dy, ld_dy, group, pre, dx32,
-                                              dx16);
-  }
-}
-
-void group_sum(hipStream_t s, int rows, int N, int group, const float* in,
-               float* out, bf16* out16, int ld16, int col16) {
-  const size_t n = static_cast<size_t>(rows) * N;
-  if (n) k_group_sum<<<blocks(n), 256, 0, s>>>(rows, N, group, in, out, out16, ld16, col16);
-}
-
-void scatter_add_rows(hipStream_t s, int M, int N, const float* in,
-                      const uint32_t* idx, float* out) {
-  const size_t n = static_cast<size_t>(M) * N;
-  if (n) k_scatter_add_rows<<<blocks(n), 256, 0, s>>>(M, N, in, idx, out);
-}
-
 void column_sum(hipStream_t s, int M, int N, const float* in, float* col_sum) {
   if (M <= 0 || N <= 0) return;
   const int slices = std::min(1024, std::max(1, M / 256));
   k_column_sum<<<dim3((N + 63) / 64, slices), 256, 0, s>>>(M, N, in, col_sum);
-}
-
-void to_bf16_block(hipStream_t s, int M, int N, const float* src, int lds,
-                   bf16* dst, int ldd, int col0) {
-  const size_t n = static_cast<size_t>(M) * N;
-  if (n) k_to_bf16_block<<<blocks(n), 256, 0, s>>>(M, N, src, lds, dst, ldd, col0);
-}
-
-void copy_cols(hipStream_t s, int M, int N, const float* src, int lds, int col0,
-               float* dst, int ldd) {
-  const size_t n = static_cast<size_t>(M) * N;
-  if (n) k_copy_cols<<<blocks(n), 256, 0, s>>>(M, N, src, lds, col0, dst, ldd, 0);
-}
-
-void add_cols(hipStream_t s, int M, int N, const float* src, int lds, int col0,
-              float* dst, int ldd) {
-  const size_t n = static_cast<size_t>(M) * N;
-  if (n) k_copy_cols<<<blocks(n), 256, 0, s>>>(M, N, src, lds, col0, dst, ldd, 1);
 }
 
 void adam_update(hipStream_t s, int n, float* w, bf16* w16, const float* g,

@@ -58,34 +58,57 @@ struct GemmArgs {
 
 void gemm_bf16(hipStream_t s, const GemmArgs& g);
 
-// dx = dy * act'(pre) for an M x N block; dy row m is read from row
-// m / group (leading dimension ld_dy), so group > 1 broadcasts one upstream
-// row to `group` rows.  Writes FP32 (dx32) and/or BF16 (dx16) copies, both
-// M x N.  In place (dx32 == dy) is allowed when group == 1 and ld_dy == N.
-void act_backward(hipStream_t s, int M, int N, const float* dy, int ld_dy,
-                   int group, const float* pre, float* dx32, bf16* dx16);
-// out[r][n] = sum_{k < group} in[r * group + k][n]; optional BF16 copy with
-// its own leading dimension and column offset.
-void group_sum(hipStream_t s, int rows, int N, int group, const float* in,
-               float* out, bf16* out16, int ld16, int col16);
-// out[idx[m]][n] += in[m][n] (atomics).
-void scatter_add_rows(hipStream_t s, int M, int N, const float* in,
-                      const uint32_t* idx, float* out);
 // col_sum[n] += sum_m in[m][n].
 void column_sum(hipStream_t s, int M, int N, const float* in, float* col_sum);
-// BF16 copy of an FP32 block into a wider matrix: dst[m][col0 + n] = src[m][n].
-void to_bf16_block(hipStream_t s, int M, int N, const float* src, int lds,
-                   bf16* dst, int ldd, int col0);
-// dst[m][n] = src[m][col0 + n] (FP32 column block copy).
-void copy_cols(hipStream_t s, int M, int N, const float* src, int lds, int col0,
-               float* dst, int ldd);
-// dst[m][n] += src[m][col0 + n].
-void add_cols(hipStream_t s, int M, int N, const float* src, int lds, int col0,
-              float* dst, int ldd);
 // Adam on FP32 master weights, refreshing the BF16 copy.
 void adam_update(hipStream_t s, int n, float* w, bf16* w16, const float* g,
                  float* m, float* v, float lr, float b1, float b2, float eps,
                  float bc1, float bc2);
 void fill_f32(hipStream_t s, size_t n, float* p, float value);
+
+// ---- dense layers of the training (nn_train.hip) -----------------------------
+// out = act(A . B + bias), A M x K row-major BF16, B = W (K x N row-major) or,
+// with trans, the transpose of the row-major N x K matrix W; K and N are the
+// network's layer sizes.  pre (M x N): the value before the activation;
+// group16: BF16 sums of every eight rows of the output.  With bpre (M x N):
+// out16 = (A . B) act'(bpre), colsum[n] += its column sums; out16 may be A.
+struct DenseArgs {
+  int M = 0, N = 0;
+  const bf16* A = nullptr;
+  int lda = 0;
+  const bf16* W = nullptr;
+  int ldw = 0;
+  bool trans = false;
+  const float* bias = nullptr;
+  int act = kActNone;
+  float* pre = nullptr;
+  bf16* out16 = nullptr;
+  int ldo16 = 0;
+  float* out32 = nullptr;
+  int ldo32 = 0;
+  bf16* group16 = nullptr;
+  int ldg = 0, colg = 0;
+  const float* bpre = nullptr;
+  float* colsum = nullptr;
+};
+void dense(hipStream_t s, int K, const DenseArgs& g);
+// d16[m][n] = dy[m / group][n] act'(pre[m][n]) (M x N), colsum[n] += its
+// column sums.
+void edge_grad(hipStream_t s, int M, int N, const float* dy, int ld_dy, int group,
+               const float* pre, bf16* d16, float* colsum);
+// Partial products X^T dY (X: K x M, dY: K x N, BF16 row-major) over
+// wgrad_slices(K) row slices, M x N each; wgrad_sum adds every listed
+// matrix's slices to its place in the gradient.
+int wgrad_slices(size_t K);
+void wgrad_part(hipStream_t s, int M, int N, size_t K, const bf16* X, const bf16* dY,
+                float* part);
+struct WgradTable {
+  static constexpr int kMax = 10;
+  int n = 0;
+  const float* part[kMax];
+  int slices[kMax];
+  uint32_t size[kMax], dst[kMax], first_block[kMax];
+};
+void wgrad_sum(hipStream_t s, WgradTable& t, float* g);
 
 }  // namespace tit_amd

@@ -535,7 +535,6 @@ struct Activations {
   float* pre1[kRounds] = {};     // E x kHidden (training)
   bf16* a1[kRounds] = {};        // E x kHidden
   float* pre2[kRounds] = {};     // E x kHidden (training)
-  float* msg = nullptr;          // E x kHidden (one round at a time)
   bf16* Y[kRounds] = {};         // n x kNodeCat
   float* pre3[kRounds] = {};     // n x kHidden (training)
   bf16* a3[kRounds] = {};
@@ -543,11 +542,10 @@ struct Activations {
   bf16* a4[kRounds] = {};
   float* u[kRounds] = {};        // n x kOut
   // backward scratch
-  float* dE = nullptr;           // E x kHidden
-  bf16* dE16 = nullptr;
+  bf16* dE16 = nullptr;          // E x kHidden
   float* dX = nullptr;           // E x kEdgeIn
-  float* dN = nullptr;           // n x kHidden
-  bf16* dN16 = nullptr;
+  bf16* dN16 = nullptr;          // n x kHidden
+  float* part = nullptr;         // weight-gradient partials, every matrix's slices
   float* dY = nullptr;           // n x kNodeCat
   float* du = nullptr;           // n x kOut
   bf16* du16 = nullptr;
@@ -689,23 +687,16 @@ hipError_t alloc_acts(Activations& A, uint32_t n, bool training) {
     }
     TIT_TRY_E(lalloc(m, &A.u[r], static_cast<size_t>(n) * kOut));
   }
-  TIT_TRY_E(lalloc(m, &A.msg, E * kHidden));
   if (training) {
-    TIT_TRY_E(lalloc(m, &A.dE, E * kHidden));
     TIT_TRY_E(lalloc(m, &A.dE16, E * kHidden));
     TIT_TRY_E(lalloc(m, &A.dX, E * kEdgeIn));
-    TIT_TRY_E(lalloc(m, &A.dN, static_cast<size_t>(n) * kHidden));
+    TIT_TRY_E(lalloc(m, &A.part, static_cast<size_t>(wgrad_slices(E)) * kParams));
     TIT_TRY_E(lalloc(m, &A.dN16, static_cast<size_t>(n) * kHidden));
     TIT_TRY_E(lalloc(m, &A.dY, static_cast<size_t>(n) * kNodeCat));
     TIT_TRY_E(lalloc(m, &A.du, static_cast<size_t>(n) * kOut));
     TIT_TRY_E(lalloc(m, &A.du16, static_cast<size_t>(n) * kOut));
   }
   return hipSuccess;
-}
-
-// Split-K count for a weight-gradient GEMM over K samples.
-int wgrad_splits(size_t K) {
-  return static_cast<int>(std::clamp<size_t>(K / 4096, 1, 512));
 }
 
 struct RoundW {
@@ -727,76 +718,46 @@ void forward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
   const RoundW W = round_w(L, r);
   constexpr int G = kEdgeIn / 8;
   k_gather_edges<<<nblk(E * G), kBlk, 0, s>>>(n, ef, A.H[r], nbr, A.X[r]);
-  GemmArgs g{};
-  // edge layer 1
-  g.M = static_cast<int>(E);
-  g.N = kHidden;
-  g.K = kEdgeIn;
-  g.A = A.X[r];
-  g.lda = kEdgeIn;
-  g.B = W.w16 + RoundLayout::W1;
-  g.ldb = kHidden;
-  g.bias = W.w32 + RoundLayout::b1;
-  g.act = kActHswish;
+  // a layer of the network on A: outputs are set by the caller
+  auto layer = [&](int M, int N, const bf16* in, int lda, int w, int bias, int act) {
+    DenseArgs g{};
+    g.M = M;
+    g.N = N;
+    g.A = in;
+    g.lda = lda;
+    g.W = W.w16 + w;
+    g.ldw = N;
+    g.bias = W.w32 + bias;
+    g.act = act;
+    return g;
+  };
+  const int m = static_cast<int>(n), me = static_cast<int>(E);
+  DenseArgs g = layer(me, kHidden, A.X[r], kEdgeIn, RoundLayout::W1, RoundLayout::b1, kActHswish);
   g.pre = A.training ? A.pre1[r] : nullptr;
-  g.ldpre = kHidden;
   g.out16 = A.a1[r];
   g.ldo16 = kHidden;
-  gemm_bf16(s, g);
-  // edge layer 2 -> messages
-  g = GemmArgs{};
-  g.M = static_cast<int>(E);
-  g.N = kHidden;
-  g.K = kHidden;
-  g.A = A.a1[r];
-  g.lda = kHidden;
-  g.B = W.w16 + RoundLayout::W2;
-  g.ldb = kHidden;
-  g.bias = W.w32 + RoundLayout::b2;
-  g.act = kActHswish;
+  dense(s, kEdgeIn, g);
+  // messages, summed over each node's edges: y = [H | sum]
+  g = layer(me, kHidden, A.a1[r], kHidden, RoundLayout::W2, RoundLayout::b2, kActHswish);
   g.pre = A.training ? A.pre2[r] : nullptr;
-  g.ldpre = kHidden;
-  g.out32 = A.msg;
-  g.ldo32 = kHidden;
-  gemm_bf16(s, g);
-  // y = [H | sum of messages]
+  g.group16 = A.Y[r];
+  g.ldg = kNodeCat;
+  g.colg = kNodeIn;
+  dense(s, kHidden, g);
   k_copy_bf16_cols<<<nblk(static_cast<size_t>(n) * (kNodeIn / 8)), kBlk, 0, s>>>(
       n, kNodeIn, A.H[r], kNodeIn, A.Y[r], kNodeCat, 0);
-  group_sum(s, static_cast<int>(n), kHidden, kKnn, A.msg, nullptr, A.Y[r], kNodeCat, kNodeIn);
   // node layers
-  g = GemmArgs{};
-  g.M = static_cast<int>(n);
-  g.N = kHidden;
-  g.K = kNodeCat;
-  g.A = A.Y[r];
-  g.lda = kNodeCat;
-  g.B = W.w16 + RoundLayout::W3;
-  g.ldb = kHidden;
-  g.bias = W.w32 + RoundLayout::b3;
-  g.act = kActHswish;
+  g = layer(m, kHidden, A.Y[r], kNodeCat, RoundLayout::W3, RoundLayout::b3, kActHswish);
   g.pre = A.training ? A.pre3[r] : nullptr;
-  g.ldpre = kHidden;
   g.out16 = A.a3[r];
   g.ldo16 = kHidden;
-  gemm_bf16(s, g);
-  g.K = kHidden;
-  g.A = A.a3[r];
-  g.lda = kHidden;
-  g.B = W.w16 + RoundLayout::W4;
-  g.bias = W.w32 + RoundLayout::b4;
+  dense(s, kNodeCat, g);
+  g = layer(m, kHidden, A.a3[r], kHidden, RoundLayout::W4, RoundLayout::b4, kActHswish);
   g.pre = A.training ? A.pre4[r] : nullptr;
   g.out16 = A.a4[r];
-  gemm_bf16(s, g);
-  g = GemmArgs{};
-  g.M = static_cast<int>(n);
-  g.N = kOut;
-  g.K = kHidden;
-  g.A = A.a4[r];
-  g.lda = kHidden;
-  g.B = W.w16 + RoundLayout::W5;
-  g.ldb = kOut;
-  g.bias = W.w32 + RoundLayout::b5;
-  g.act = kActNone;
+  g.ldo16 = kHidden;
+  dense(s, kHidden, g);
+  g = layer(m, kOut, A.a4[r], kHidden, RoundLayout::W5, RoundLayout::b5, kActNone);
   g.out32 = A.u[r];
   g.ldo32 = kOut;
   if (r + 1 < kRounds) {
@@ -805,80 +766,82 @@ void forward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
     g.out16 = A.H[r + 1] + kNodeFeat;
     g.ldo16 = kNodeIn;
   }
-  gemm_bf16(s, g);
-}
-
-// dW += X^T dY over K rows (X: K x M BF16 row-major, dY: K x N BF16).
-void wgrad(hipStream_t s, int M, int N, size_t K, const bf16* X, const bf16* dY,
-           float* gW) {
-  GemmArgs g{};
-  g.M = M;
-  g.N = N;
-  g.K = static_cast<int>(K);
-  g.A = X;
-  g.lda = M;
-  g.transA = true;
-  g.B = dY;
-  g.ldb = N;
-  g.accumulate = true;
-  g.out32 = gW;
-  g.ldo32 = N;
-  g.k_splits = wgrad_splits(K);
-  gemm_bf16(s, g);
-}
-
-// dX = dY W^T (dY: M x N BF16, W: K x N BF16 row-major) -> M x K FP32.
-void dgrad(hipStream_t s, size_t M, int N, int K, const bf16* dY, const bf16* W,
-           float* dX) {
-  GemmArgs g{};
-  g.M = static_cast<int>(M);
-  g.N = K;
-  g.K = N;
-  g.A = dY;
-  g.lda = N;
-  g.B = W;
-  g.ldb = N;
-  g.transB = true;
-  g.out32 = dX;
-  g.ldo32 = K;
-  gemm_bf16(s, g);
+  dense(s, kHidden, g);
 }
 
 // Backward of round r from A.du (n x kOut FP32).  For r > 0 leaves the
-// gradient of the previous round's output in du_prev.
+// gradient of the previous round's output in du_prev.  The weight gradients'
+// partials are listed in wt.
 void backward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
-                    const uint32_t* nbr, float* du_prev) {
+                    const uint32_t* nbr, float* du_prev, WgradTable& wt) {
   const size_t E = static_cast<size_t>(n) * kKnn;
   const RoundW W = round_w(L, r);
   float* g = W.g;
+  auto wgrad = [&](int M, int N, size_t K, const bf16* X, const bf16* dY, int dst) {
+    float* part = A.part + static_cast<size_t>(wgrad_slices(E)) *
+                               (static_cast<size_t>(r) * RoundLayout::size + dst);
+    wgrad_part(s, M, N, K, X, dY, part);
+    wt.part[wt.n] = part;
+    wt.slices[wt.n] = wgrad_slices(K);
+    wt.size[wt.n] = static_cast<uint32_t>(M * N);
+    wt.dst[wt.n] = static_cast<uint32_t>(r * RoundLayout::size + dst);
+    ++wt.n;
+  };
+  // dX = dY W^T; with bpre through the activation that made X, into BF16
+  auto dgrad = [&](int M, int K, int N, const bf16* dY, int w) {
+    DenseArgs d{};
+    d.M = M;
+    d.N = N;
+    d.A = dY;
+    d.lda = K;
+    d.W = W.w16 + w;
+    d.ldw = K;
+    d.trans = true;
+    return d;
+  };
+  const int m = static_cast<int>(n), me = static_cast<int>(E);
   // output layer
   k_to_bf16<<<nblk(static_cast<size_t>(n) * kOut), kBlk, 0, s>>>(
       static_cast<size_t>(n) * kOut, A.du, A.du16);
-  column_sum(s, static_cast<int>(n), kOut, A.du, g + RoundLayout::b5);
-  wgrad(s, kHidden, kOut, n, A.a4[r], A.du16, g + RoundLayout::W5);
-  dgrad(s, n, kOut, kHidden, A.du16, W.w16 + RoundLayout::W5, A.dN);
+  column_sum(s, m, kOut, A.du, g + RoundLayout::b5);
+  wgrad(kHidden, kOut, n, A.a4[r], A.du16, RoundLayout::W5);
+  DenseArgs d = dgrad(m, kOut, kHidden, A.du16, RoundLayout::W5);
+  d.bpre = A.pre4[r];
+  d.out16 = A.dN16;
+  d.ldo16 = kHidden;
+  d.colsum = g + RoundLayout::b4;
+  dense(s, kOut, d);
   // node layer 2
-  act_backward(s, static_cast<int>(n), kHidden, A.dN, kHidden, 1, A.pre4[r], A.dN, A.dN16);
-  column_sum(s, static_cast<int>(n), kHidden, A.dN, g + RoundLayout::b4);
-  wgrad(s, kHidden, kHidden, n, A.a3[r], A.dN16, g + RoundLayout::W4);
-  dgrad(s, n, kHidden, kHidden, A.dN16, W.w16 + RoundLayout::W4, A.dN);
+  wgrad(kHidden, kHidden, n, A.a3[r], A.dN16, RoundLayout::W4);
+  d = dgrad(m, kHidden, kHidden, A.dN16, RoundLayout::W4);
+  d.bpre = A.pre3[r];
+  d.out16 = A.dN16;
+  d.ldo16 = kHidden;
+  d.colsum = g + RoundLayout::b3;
+  dense(s, kHidden, d);
   // node layer 1
-  act_backward(s, static_cast<int>(n), kHidden, A.dN, kHidden, 1, A.pre3[r], A.dN, A.dN16);
-  column_sum(s, static_cast<int>(n), kHidden, A.dN, g + RoundLayout::b3);
-  wgrad(s, kNodeCat, kHidden, n, A.Y[r], A.dN16, g + RoundLayout::W3);
-  dgrad(s, n, kHidden, kNodeCat, A.dN16, W.w16 + RoundLayout::W3, A.dY);
+  wgrad(kNodeCat, kHidden, n, A.Y[r], A.dN16, RoundLayout::W3);
+  d = dgrad(m, kHidden, kNodeCat, A.dN16, RoundLayout::W3);
+  d.out32 = A.dY;
+  d.ldo32 = kNodeCat;
+  dense(s, kHidden, d);
   // edge layer 2 (message gradient = dY[:, kNodeIn:] broadcast to the edges)
-  act_backward(s, static_cast<int>(E), kHidden, A.dY + kNodeIn, kNodeCat, kKnn,
-                A.pre2[r], A.dE, A.dE16);
-  column_sum(s, static_cast<int>(E), kHidden, A.dE, g + RoundLayout::b2);
-  wgrad(s, kHidden, kHidden, E, A.a1[r], A.dE16, g + RoundLayout::W2);
-  dgrad(s, E, kHidden, kHidden, A.dE16, W.w16 + RoundLayout::W2, A.dE);
+  edge_grad(s, me, kHidden, A.dY + kNodeIn, kNodeCat, kKnn, A.pre2[r], A.dE16,
+            g + RoundLayout::b2);
+  wgrad(kHidden, kHidden, E, A.a1[r], A.dE16, RoundLayout::W2);
+  d = dgrad(me, kHidden, kHidden, A.dE16, RoundLayout::W2);
+  d.bpre = A.pre1[r];
+  d.out16 = A.dE16;
+  d.ldo16 = kHidden;
+  d.colsum = g + RoundLayout::b1;
+  dense(s, kHidden, d);
   // edge layer 1
-  act_backward(s, static_cast<int>(E), kHidden, A.dE, kHidden, 1, A.pre1[r], A.dE, A.dE16);
-  column_sum(s, static_cast<int>(E), kHidden, A.dE, g + RoundLayout::b1);
-  wgrad(s, kEdgeIn, kHidden, E, A.X[r], A.dE16, g + RoundLayout::W1);
+  wgrad(kEdgeIn, kHidden, E, A.X[r], A.dE16, RoundLayout::W1);
   if (r > 0) {
-    dgrad(s, E, kHidden, kEdgeIn, A.dE16, W.w16 + RoundLayout::W1, A.dX);
+    d = dgrad(me, kHidden, kEdgeIn, A.dE16, RoundLayout::W1);
+    d.out32 = A.dX;
+    d.ldo32 = kEdgeIn;
+    dense(s, kHidden, d);
     k_latent_grad_gather<<<nblk(static_cast<size_t>(n) * kLatent), kBlk, 0, s>>>(
         n, A.dY, A.dX, du_prev);
     k_latent_grad_scatter<<<nblk(E * kLatent), kBlk, 0, s>>>(n, A.dX, nbr, du_prev);
@@ -897,14 +860,16 @@ hipError_t loss_and_grad(hipStream_t s, Learned* L, int dim, const Sample& S,
       1.0f / static_cast<float>(std::max<uint32_t>(S.n_fluid, 1) * (dim + 1));
   k_loss<<<nblk(S.n), kBlk, 0, s>>>(S.n, dim, A.u[kRounds - 1], S.target, S.fluid, L->sc,
                                     inv_count, A.du, loss);
+  WgradTable wt{};
   for (int r = kRounds - 1; r >= 0; --r) {
     float* du_prev = r > 0 ? A.u[r - 1] : nullptr;  // u[r-1] is no longer needed
-    backward_round(s, L, A, r, S.n, S.nbr, du_prev);
+    backward_round(s, L, A, r, S.n, S.nbr, du_prev, wt);
     if (r > 0) {
       TIT_TRY_E(hipMemcpyAsync(A.du, du_prev, static_cast<size_t>(S.n) * kOut * sizeof(float),
                                hipMemcpyDeviceToDevice, s));
     }
   }
+  wgrad_sum(s, wt, L->grad);
   return hipSuccess;
 }
 
