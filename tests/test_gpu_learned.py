@@ -136,6 +136,27 @@ def test_loss_and_gradient_vs_oracle():
     ctx.close()
 
 
+@pytest.mark.parametrize("dr,tank,column", [(0.5, (1.0, 1.0), (0.5, 0.5)),
+                                            (0.25, (1.5, 1.0), (0.75, 0.5)),
+                                            (0.04, (2.0, 1.5), (1.0, 0.9))])
+def test_loss_and_gradient_of_ragged_sizes(dr, tank, column):
+    """The gradient where the node count is below one tile of rows, just
+    beyond one, and leaves a remainder in every row split.  Tolerances as in
+    test_loss_and_gradient_vs_oracle: BF16 operands (2^-9) through the ten
+    layers of a round and its backward."""
+    ctx, eq, pa = _dam(dr=dr, steps=3, tank=tank, column=column)
+    L = ta.LearnedStep(ctx, seed=7)
+    smp = L.sample(L.record(4))
+    loss, grad = L.loss_grad(0)
+    loss_o, grad_o = S.loss_and_grad(L.params(), smp["node_feat"], smp["edge_feat"], smp["nbr"],
+                                     smp["target"], smp["fluid"], L.scales()[2:6], eq.dim)
+    rel = np.linalg.norm(grad - grad_o) / np.linalg.norm(grad_o)
+    print(f"n {pa.n}: loss rel {abs(loss - loss_o) / loss_o:.2e}; gradient rel L2 {rel:.2e}")
+    assert abs(loss - loss_o) / loss_o < 2e-2
+    assert rel < 5e-2
+    ctx.close()
+
+
 def _batched(seed, n_tanks, dr):
     rng = np.random.default_rng(seed)
     arrays = []

@@ -348,9 +348,11 @@ def test_gapped_columns_are_cut_and_sum_exact_sets():
 
 
 @pytest.mark.parametrize("dim,n,box", [(2, 1, 0.5), (2, 257, 0.06), (2, 700, 0.3), (2, 900, 0.13),
-                                       (2, 1500, 0.05), (2, 6000, 0.5)])
+                                       (2, 1500, 0.05), (2, 6000, 0.5),
+                                       (3, 1, 0.5), (3, 300, 0.03), (3, 1861, 0.06),
+                                       (3, 2500, 0.12), (3, 6000, 0.4)])
 def test_tile_limits_keep_sets_and_bits(dim, n, box):
-    """Clouds at the limits of the 2D tiles: one particle, one cell row with
+    """Clouds at the limits of the tiles: one particle, one cell row with
     more targets than lanes, windows past the staged candidates, more accepted
     candidates in a stencil column than the list holds, and sparse ones.  The
     pair counts are the brute-force sets, and the right-hand side has the bits
@@ -370,6 +372,59 @@ def test_tile_limits_keep_sets_and_bits(dim, n, box):
     ctx.set_schedule(0, 0)
     ref = ctx.compute_rhs()
     assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+    ctx.close()
+
+
+@pytest.mark.parametrize("dim,n,width", [(2, 1, 0.1), (2, 1023, 0.5), (2, 1025, 5.0),
+                                         (2, 32768, 2.1), (3, 4097, 0.4)])
+def test_small_rebuild_equals_large(dim, n, width):
+    """A set at the edges of the single-launch rebuild (one particle, a
+    workgroup's thread count, many empty cells, the largest set) gives the
+    trajectory bits that the same tank has beside one that makes the whole too
+    large for it."""
+    dr = 0.01
+    rng = np.random.default_rng(n)
+    side = int(np.ceil(n ** (1.0 / dim)))
+    r = np.stack(np.meshgrid(*[np.arange(side) * dr] * dim, indexing="ij"), axis=-1)
+    r = r.reshape(-1, dim)[:n]
+    r = rng.permutation(r + rng.uniform(-0.2 * dr, 0.2 * dr, r.shape))
+    none = np.zeros((0, dim))
+    pa = ta.ParticleArray(dim, r, np.full(n, 1000.0), n, none, tuple([-0.05] * dim),
+                          tuple([width] * dim), v=rng.normal(0.0, 3.0, (n, dim)))
+    m = 32768
+    other = ta.ParticleArray(dim, rng.uniform(0.0, 4.0 if dim == 2 else 0.7, (m, dim)),
+                             np.full(m, 1000.0), m, none, tuple([0.0] * dim),
+                             tuple([4.0 if dim == 2 else 0.7] * dim))
+    eq = _eq(dim, dr)
+    one, two = _ctx(eq, [pa]), _ctx(eq, [pa, other])
+    off, idx = one.neighbors()
+    off2, idx2 = two.neighbors()
+    assert np.array_equal(off, off2[:n + 1]) and np.array_equal(idx, idx2[:off[n]])
+    one.step(12)
+    two.step(12)
+    assert n == 1 or one.counts()[1] > 1  # more than the first rebuild
+    a, b = one.download(), two.download()
+    for f in ("r", "v", "rho"):
+        assert np.array_equal(a[f], b[f][:n]), f
+    one.close()
+    two.close()
+
+
+@pytest.mark.parametrize("n", [1, 16384, 16385, 120000, 160001])
+def test_download_pieces(n):
+    """Frames around the limits of the download's staging (1 MiB in one copy,
+    8 pieces of 1 MiB among the workers): what was uploaded comes back, in
+    the uploaded order."""
+    rng = np.random.default_rng(n)
+    r = rng.uniform(0.0, 1.0, (n, 3))
+    v = rng.normal(0.0, 1.0, (n, 3))
+    rho = rng.uniform(990.0, 1010.0, n)
+    pa = ta.ParticleArray(3, r, rho, n, np.zeros((0, 3)), (0.0,) * 3, (1.0,) * 3, v=v)
+    ctx = _ctx(_eq(3, 0.02), [pa])
+    for _ in range(2):
+        out = ctx.download()
+        assert np.array_equal(out["r"], r) and np.array_equal(out["v"], v)
+        assert np.array_equal(out["rho"], rho)
     ctx.close()
 
 

@@ -18,6 +18,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -784,6 +785,7 @@ void tit_hip_destroy(tit_hip_ctx* c) {
   destroy_learned(c);
   free_all(c);
   c->prof.clear();
+  if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1154,6 +1156,136 @@ tit_status tit_hip_step(tit_hip_ctx* c, int n_steps, double* dt_last) {
   return TIT_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// One device array to copy to the caller's memory.
+struct HostCopy {
+  char* dst;
+  const char* src;
+  size_t bytes;
+};
+
+// Device arrays to pageable host memory through pinned staging.  The runtime's
+// own copy to pageable memory runs on one thread, at 7 to 16 GB/s, much of it
+// page faults of a freshly allocated destination, and costs 25 to 45 us for
+// each array.  Up to one piece (1 MiB) is staged whole and copied out by the
+// caller: 95 -> 52 us for 800 particles, 180 -> 66 us for 4,900.  From 8
+// pieces on, worker threads each own a staging slot: a worker queues its
+// piece's transfer, waits for it and copies it out while the other workers'
+// pieces are in flight: 2.3 -> 1.2 ms for 24 MB, 9.4 -> 3.3 ms for 97 MB,
+// 12.8 -> 5.7 ms for 129 MB.  Between the two the runtime's copy is as fast
+// (6 MB: 350 and 360 us).  Smaller pieces wait too often: 97 MB take 7.2 ms in
+// pieces of 256 KiB and 4.8 ms in pieces of 512 KiB.  The staging (8 MiB at
+// most) stays with the context.
+// A destination that the runtime knows (pinned memory) is copied to directly.
+constexpr size_t kPiece = size_t(1) << 20;
+constexpr int kSlots = 8;
+
+bool pageable(const void* p) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // host memory that the runtime does not know
+    return true;
+  }
+  return at.type == hipMemoryTypeUnregistered;
+}
+
+hipError_t copy_out(tit_hip_ctx* c, const HostCopy* copies, int n_copies) {
+  size_t total = 0, n_pieces = 0;
+  bool staged = true;
+  for (int k = 0; k < n_copies; ++k) {
+    total += copies[k].bytes;
+    n_pieces += (copies[k].bytes + kPiece - 1) / kPiece;
+    staged = staged && pageable(copies[k].dst);
+  }
+  if (total == 0) return hipStreamSynchronize(c->stream);
+  const bool one = total <= kPiece;
+  staged = staged && (one || n_pieces >= kSlots);
+  const size_t need = one ? total : kSlots * kPiece;
+  if (staged && c->pinned_bytes < need) {
+    if (c->pinned) (void)hipHostFree(c->pinned);
+    c->pinned = nullptr;
+    c->pinned_bytes = 0;
+    if (hipHostMalloc(&c->pinned, need, hipHostMallocDefault) == hipSuccess) {
+      c->pinned_bytes = need;
+    } else {
+      (void)hipGetLastError();
+      c->pinned = nullptr;
+    }
+  }
+  if (!staged || !c->pinned) {
+    for (int k = 0; k < n_copies; ++k) {
+      const hipError_t e = hipMemcpyAsync(copies[k].dst, copies[k].src, copies[k].bytes,
+                                          hipMemcpyDeviceToHost, c->stream);
+      if (e != hipSuccess) return e;
+    }
+    return hipStreamSynchronize(c->stream);
+  }
+  char* stage = static_cast<char*>(c->pinned);
+  if (one) {
+    size_t o = 0;
+    for (int k = 0; k < n_copies; ++k) {
+      const hipError_t e = hipMemcpyAsync(stage + o, copies[k].src, copies[k].bytes,
+                                          hipMemcpyDeviceToHost, c->stream);
+      if (e != hipSuccess) {
+        (void)hipStreamSynchronize(c->stream);  // nothing is left writing to the staging
+        return e;
+      }
+      o += copies[k].bytes;
+    }
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return e;
+    o = 0;
+    for (int k = 0; k < n_copies; ++k) {
+      std::memcpy(copies[k].dst, stage + o, copies[k].bytes);
+      o += copies[k].bytes;
+    }
+    return hipSuccess;
+  }
+  // worker w: pieces w, w + kSlots, ... of the arrays taken one after another
+  hipError_t err[kSlots] = {};
+  auto work = [&](int w) {
+    hipEvent_t done = nullptr;
+    hipError_t e = hipSetDevice(c->device);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+    char* slot = stage + w * kPiece;
+    size_t piece = 0;
+    for (int k = 0; k < n_copies && e == hipSuccess; ++k) {
+      const HostCopy& h = copies[k];
+      for (size_t o = 0; o < h.bytes && e == hipSuccess; o += kPiece, ++piece) {
+        if (piece % kSlots != static_cast<size_t>(w)) continue;
+        const size_t bytes = std::min(kPiece, h.bytes - o);
+        e = hipMemcpyAsync(slot, h.src + o, bytes, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipEventRecord(done, c->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(done);
+        if (e == hipSuccess) std::memcpy(h.dst + o, slot, bytes);
+      }
+    }
+    if (done) (void)hipEventDestroy(done);
+    err[w] = e;
+  };
+  std::thread threads[kSlots];
+  int started = 1;  // the caller is worker 0
+  try {
+    for (; started < kSlots; ++started) threads[started] = std::thread(work, started);
+  } catch (...) {  // no more threads: the caller does the rest
+  }
+  work(0);
+  for (int w = started; w < kSlots; ++w) work(w);
+  for (int w = 1; w < started; ++w) threads[w].join();
+  const hipError_t e = hipStreamSynchronize(c->stream);
+  for (hipError_t x : err) {
+    if (x != hipSuccess) return x;
+  }
+  return e;
+}
+
+}  // namespace
+
+extern "C" {
+
 tit_status tit_hip_download(tit_hip_ctx* c, double* r, double* v, double* rho,
                             double* p) {
   if (!c) return TIT_E_ARG;
@@ -1165,11 +1297,19 @@ tit_status tit_hip_download(tit_hip_ctx* c, double* r, double* v, double* rho,
                 c->stage_rho, c->stage_p);
   tit_status st = check_launch(c, "download");
   if (st != TIT_OK) return st;
-  if (r) TIT_HIP_TRY(c, hipMemcpyAsync(r, c->stage_r, n * dim * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (v) TIT_HIP_TRY(c, hipMemcpyAsync(v, c->stage_v, n * dim * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (rho) TIT_HIP_TRY(c, hipMemcpyAsync(rho, c->stage_rho, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  if (p) TIT_HIP_TRY(c, hipMemcpyAsync(p, c->stage_p, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  TIT_HIP_TRY(c, hipStreamSynchronize(c->stream));
+  HostCopy copies[4];
+  int n_copies = 0;
+  auto add = [&](double* dst, const double* src, size_t count) {
+    if (dst) {
+      copies[n_copies++] = HostCopy{reinterpret_cast<char*>(dst),
+                                    reinterpret_cast<const char*>(src), count * sizeof(double)};
+    }
+  };
+  add(r, c->stage_r, n * dim);
+  add(v, c->stage_v, n * dim);
+  add(rho, c->stage_rho, n);
+  add(p, c->stage_p, n);
+  TIT_HIP_TRY(c, copy_out(c, copies, n_copies));
   return TIT_OK;
 }
 

@@ -118,6 +118,10 @@ struct tit_hip_ctx {
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   hipGraph_t graph_def[2] = {nullptr, nullptr};
 
+  // pinned staging of the downloads (tit_hip_download), made on first use
+  void* pinned = nullptr;
+  size_t pinned_bytes = 0;
+
   // learned step (surrogate.hip), created on first use
   tit_amd::Learned* learned = nullptr;
 };
