@@ -410,6 +410,25 @@ def test_small_rebuild_equals_large(dim, n, width):
     two.close()
 
 
+@pytest.mark.parametrize("dim,dr", [(2, 0.02), (3, 0.08)])
+def test_wide_boundary_groups_keep_the_bits(dim, dr):
+    """The extrapolation with a wave per fixed particle (few of them) and with
+    16 lanes (the same tank among enough others): the same state bits."""
+    one = ta.dam_break(dim, dr, [1.6] * dim, [0.6] * dim)
+    limit = 8192 if dim == 2 else 32768
+    many = limit // (one.n - one.n_fluid) + 1
+    eq = ta.cfg_equations(dim, dr, 0.6)
+    a, b = _ctx(eq, [one]), _ctx(eq, [one] * many)
+    a.step(5)
+    b.step(5)
+    x, y = a.download(), b.download()
+    for f in ("r", "v", "rho"):
+        assert np.array_equal(x[f], y[f][:one.n]), f
+        assert np.array_equal(x[f], y[f][-one.n:]), f
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("n", [1, 16384, 16385, 120000, 160001])
 def test_download_pieces(n):
     """Frames around the limits of the download's staging (1 MiB in one copy,

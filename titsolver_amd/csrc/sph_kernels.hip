@@ -278,6 +278,12 @@ __global__ __launch_bounds__(kBlock) void k_cell_gaps(uint32_t* __restrict__ off
 constexpr int kBoundaryLanes = 16;
 // candidates whose loads a lane of k_boundary has in flight at once
 constexpr int kBoundaryUnroll = 2;
+// Fixed particles up to which k_boundary gives each one a wave.  16 and 64
+// lanes each, us per launch between events: 2D 1,215 fixed 15.0 and 12.1;
+// 6,015 15.4 and 13.9; 12,015 16.8 and 17.5; 24,015 19.9 and 25.8; 3D 6,819
+// 44.8 and 23.7; 24,891 52.4 and 40.7; 66,378 66.6 and 72.7.  Beyond, the chip
+// is full and the wider groups' idle lanes and shuffles cost more.
+constexpr uint32_t boundary_wide(int dim) { return dim == 2 ? 8192u : 32768u; }
 // fixed particles per workgroup of k_fixed_active (its LDS list)
 constexpr uint32_t kFixedPerBlock = 1024;
 
@@ -361,13 +367,18 @@ __global__ __launch_bounds__(kBlock) void k_fixed_active(BoundaryArgs A, const u
 }
 
 // Extrapolation of the listed fixed particles, one group of G lanes each.
+// G is 64 for small lists: a launch there is one chain of latencies, and with
+// 16 lanes half of it is the FP64 terms of the 4 to 8 candidates of each lane.
+// The sums are those of 16 lanes whatever G is: slot l adds the candidates
+// l, l + 16, ... in order, a wider group only evaluates the terms of four
+// slots' rounds at once and every lane adds its slot's four by shuffles.
 // XI_INT: the Tait exponent is a small integer (P.xi_int), so H(rho) takes
 // integer powers; the general FP64 pow otherwise (it alone needs about 55
 // more VGPRs, which would cost a wave per SIMD).
-template <int DIM, int KERNEL, bool XI_INT>
+template <int DIM, int KERNEL, bool XI_INT, int G>
 __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
   constexpr int NCOL = DIM == 2 ? 2 * kStencil + 1 : (2 * kStencil + 1) * (2 * kStencil + 1);
-  constexpr int G = kBoundaryLanes;
+  static_assert(G == kBoundaryLanes || G == 64, "a slot per lane, or a wave");
   const uint32_t k = blockIdx.x * (kBlock / G) + (threadIdx.x / G);
   const int lane = threadIdx.x % G;
   if (k >= *A.n_active) return;  // uniform in the group
@@ -513,19 +524,32 @@ __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (!ok[u]) continue;
-      const double rho_b = rho[u];
-      const double V_b = mb[u] / rho_b;
-      const double W = w0 * kernel_value_poly_f64<KERNEL>(h_inv * sqrt(s2[u]));
-      double rn = dd[u][0] * ne[0];
+      double tS = 0.0, tH = 0.0;  // (a sum of zero leaves S and H as they are)
+      if (ok[u]) {
+        const double rho_b = rho[u];
+        const double V_b = mb[u] / rho_b;
+        const double W = w0 * kernel_value_poly_f64<KERNEL>(h_inv * sqrt(s2[u]));
+        double rn = dd[u][0] * ne[0];
 #pragma unroll
-      for (int d = 1; d < DIM; ++d) rn = rn + dd[u][d] * ne[d];
-      // H(rho_b) = cs0^2 ((rho_b/rho0)^(xi-1) - 1) / (xi - 1)
-      const double ratio = rho_b * P.inv_rho0;
-      const double rp = XI_INT ? ipow_f64(ratio, P.xi_int - 1) : pow_general(ratio, xi_1);
-      const double H_b = cs2 * (rp - 1.0) * inv_xi_1;
-      S += V_b * W;
-      H += V_b * (H_b + P.g * rn * ne[1]) * W;
+        for (int d = 1; d < DIM; ++d) rn = rn + dd[u][d] * ne[d];
+        // H(rho_b) = cs0^2 ((rho_b/rho0)^(xi-1) - 1) / (xi - 1)
+        const double ratio = rho_b * P.inv_rho0;
+        const double rp = XI_INT ? ipow_f64(ratio, P.xi_int - 1) : pow_general(ratio, xi_1);
+        const double H_b = cs2 * (rp - 1.0) * inv_xi_1;
+        tS = V_b * W;
+        tH = V_b * (H_b + P.g * rn * ne[1]) * W;
+      }
+      if constexpr (G == kBoundaryLanes) {
+        S += tS;
+        H += tH;
+      } else {
+#pragma unroll
+        for (int r = 0; r < G; r += kBoundaryLanes) {
+          const int from = r + (lane & (kBoundaryLanes - 1));
+          S += __shfl(tS, from);
+          H += __shfl(tH, from);
+        }
+      }
     }
   };
   if constexpr (DIM == 2) {
@@ -536,7 +560,8 @@ __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
       while (t >= rl[q + 1]) ++q;
       return rb[q] + (t - rl[q]);
     };
-    for (uint32_t t = lane; t < n_cand; t += U * G) {
+    for (uint32_t base = 0; base < n_cand; base += U * G) {  // uniform in the group
+      const uint32_t t = base + lane;
       uint32_t j[U];
       bool live[U];
 #pragma unroll
@@ -548,7 +573,7 @@ __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
     }
   } else {
     // The 25 trimmed column ranges, laid end to end: each lane loads two
-    // columns' bounds, the group scans their lengths, and the lanes then
+    // columns' bounds (one, in a wave), the group scans their lengths, and the lanes then
     // take every G-th candidate of the whole list (no round trip per
     // column).
     __shared__ uint32_t s_rb[kBlock / G][NCOL];
@@ -582,8 +607,10 @@ __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
       }
     }
     const uint32_t tot0 = __shfl(x0, G - 1, G), tot1 = __shfl(x1, G - 1, G);
-    s_rb[grp][lane] = beg[0];
-    s_rl[grp][lane] = x0 - len[0];
+    if (lane < NCOL) {
+      s_rb[grp][lane] = beg[0];
+      s_rl[grp][lane] = x0 - len[0];
+    }
     if (lane + G < NCOL) {
       s_rb[grp][lane + G] = beg[1];
       s_rl[grp][lane + G] = tot0 + x1 - len[1];
@@ -599,7 +626,8 @@ __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
       while (t >= s_rl[grp][q + 1]) ++q;
       return s_rb[grp][q] + (t - s_rl[grp][q]);
     };
-    for (uint32_t t = lane; t < n_cand; t += U * G) {
+    for (uint32_t base = 0; base < n_cand; base += U * G) {  // uniform in the group
+      const uint32_t t = base + lane;
       uint32_t j[U];
       bool live[U];
 #pragma unroll
@@ -611,7 +639,7 @@ __global__ __launch_bounds__(kBlock) void k_boundary(BoundaryArgs A) {
     }
   }
 #pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) {
+  for (int off = kBoundaryLanes / 2; off > 0; off >>= 1) {
     S += __shfl_xor(S, off);
     H += __shfl_xor(H, off);
   }
@@ -903,26 +931,35 @@ void launch_fixed_active(hipStream_t s, const BoundaryArgs& a, const uint32_t* c
   }
 }
 
+namespace {
+
+template <int DIM, int KERNEL, bool XI_INT>
+void boundary_lanes(hipStream_t s, const BoundaryArgs& a) {
+  if (a.n_fixed <= boundary_wide(DIM)) {
+    k_boundary<DIM, KERNEL, XI_INT, 64><<<grid_for(a.n_fixed, kBlock / 64), kBlock, 0, s>>>(a);
+  } else {
+    k_boundary<DIM, KERNEL, XI_INT, kBoundaryLanes>
+        <<<grid_for(a.n_fixed, kBlock / kBoundaryLanes), kBlock, 0, s>>>(a);
+  }
+}
+
+template <int DIM, int KERNEL>
+void boundary_kernel(hipStream_t s, const BoundaryArgs& a) {
+  if (a.P.xi_int != 0) boundary_lanes<DIM, KERNEL, true>(s, a);
+  else boundary_lanes<DIM, KERNEL, false>(s, a);
+}
+
+}  // namespace
+
 void launch_boundary(hipStream_t s, const BoundaryArgs& a) {
   if (a.n_fixed == 0) return;
-  const uint32_t g = grid_for(a.n_fixed, kBlock / kBoundaryLanes);
-  const bool c4 = a.P.kernel == kKernelC4, xi_int = a.P.xi_int != 0;
+  const bool c4 = a.P.kernel == kKernelC4;
   if (a.P.dim == 2) {
-    if (c4) {
-      if (xi_int) k_boundary<2, kKernelC4, true><<<g, kBlock, 0, s>>>(a);
-      else k_boundary<2, kKernelC4, false><<<g, kBlock, 0, s>>>(a);
-    } else {
-      if (xi_int) k_boundary<2, kKernelC2, true><<<g, kBlock, 0, s>>>(a);
-      else k_boundary<2, kKernelC2, false><<<g, kBlock, 0, s>>>(a);
-    }
+    if (c4) boundary_kernel<2, kKernelC4>(s, a);
+    else boundary_kernel<2, kKernelC2>(s, a);
   } else {
-    if (c4) {
-      if (xi_int) k_boundary<3, kKernelC4, true><<<g, kBlock, 0, s>>>(a);
-      else k_boundary<3, kKernelC4, false><<<g, kBlock, 0, s>>>(a);
-    } else {
-      if (xi_int) k_boundary<3, kKernelC2, true><<<g, kBlock, 0, s>>>(a);
-      else k_boundary<3, kKernelC2, false><<<g, kBlock, 0, s>>>(a);
-    }
+    if (c4) boundary_kernel<3, kKernelC4>(s, a);
+    else boundary_kernel<3, kKernelC2>(s, a);
   }
 }
 
