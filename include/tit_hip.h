@@ -222,13 +222,14 @@ tit_status tit_hip_kernel_stats(tit_hip_ctx* ctx, tit_hip_kernel_stat* out,
                                 int cap, int* n_out);
 
 /* Schedule of the fused stage kernel.  Two families:
- *  - column chunks: each workgroup takes a chunk of at most chunk_targets
- *    consecutive particles of one cell column (one per lane); in 2D up to
- *    lds_capacity candidate positions of a chunk are staged in LDS;
- *  - 3D block chunks (lds_capacity > 0 in 3D): a workgroup of 256 lanes takes
- *    the particles of a 4 x 4 block of cell columns over a few rows, with up
- *    to lds_capacity candidate positions of the block's window in LDS.
- * lds_capacity 0 reads positions from global memory (column chunks).  Results
+ *  - tiles (lds_capacity > 0): a workgroup of 256 lanes takes the particles of
+ *    a block of cell columns over a few rows (4 columns in 2D, 4 x 4 in 3D)
+ *    with the block's window in LDS; lds_capacity bounds the window's
+ *    candidates (in 3D in proportion to the kernel's own capacity), and in 2D
+ *    chunk_targets the tile's particles (2 chunk_targets of them);
+ *  - column chunks (lds_capacity 0): a workgroup takes at most chunk_targets
+ *    consecutive particles of one cell column, one per lane, and reads
+ *    positions from global memory.  Results
  * are bitwise identical on every schedule.  occupancy is the mean number of
  * particles per occupied cell at upload.  cached (tit_hip_autotune only): 1
  * when the schedule came from the process's tuning cache.  No reference

@@ -373,10 +373,19 @@ def test_tile_limits_keep_sets_and_bits(dim, n, box):
     ref = ctx.compute_rhs()
     assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
     ctx.close()
+    if dim == 2:  # beside a tank that makes the set too large for four lanes per target
+        m = 70000
+        q = rng.uniform(0.0, 3.0, size=(m, dim))
+        other = ta.ParticleArray(dim, q, np.full(m, 1000.0), m, np.zeros((0, dim)),
+                                 (0.0, 0.0), (3.0, 3.0))
+        ctx = _ctx(eq, [pa, other])
+        two = ctx.compute_rhs()
+        assert np.array_equal(two[0][:n], ref[0]) and np.array_equal(two[1][:n], ref[1])
+        ctx.close()
 
 
 @pytest.mark.parametrize("dim,n,width", [(2, 1, 0.1), (2, 1023, 0.5), (2, 1025, 5.0),
-                                         (2, 32768, 2.1), (3, 4097, 0.4)])
+                                         (2, 16384, 2.1), (3, 4097, 0.4)])
 def test_small_rebuild_equals_large(dim, n, width):
     """A set at the edges of the single-launch rebuild (one particle, a
     workgroup's thread count, many empty cells, the largest set) gives the

@@ -248,6 +248,15 @@ double cell_size(const tit_hip_ctx* c) {
 
 StageArgs stage_args(tit_hip_ctx* c);
 
+// Whether the 2D tiles give each target four lanes (stage_tile.hip), and the
+// chunk length that the schedule then has: a quarter of the lanes' targets.
+bool quad_tiles(const tit_hip_ctx* c) {
+  return c->dp.dim == 2 && c->lds_cap > 0 && c->n <= kQuadN;
+}
+uint32_t tile_targets(const tit_hip_ctx* c) {
+  return quad_tiles(c) ? std::min<uint32_t>(c->chunk_targets, kChunkMax / 4) : c->chunk_targets;
+}
+
 RebuildCtl rebuild_ctl(tit_hip_ctx* c) {
   return RebuildCtl{c->rebuild_ctl, c->tank_need, c->rebuild_count};
 }
@@ -453,7 +462,7 @@ tit_status build_schedule(tit_hip_ctx* c) {
     c->n_blocks = static_cast<uint32_t>(blocks.size());
   }
   const size_t bneed = block_chunk_bound(dim, c->n, c->n_blocks, static_cast<size_t>(nz_max),
-                                         c->chunk_targets, c->lds_cap);
+                                         tile_targets(c), c->lds_cap);
   if (bneed > c->bchunk_cap) {
     forget(c, c->bchunks);
     c->bchunks = nullptr;
@@ -479,8 +488,9 @@ StageArgs stage_args(tit_hip_ctx* c) {
   StageArgs a{};
   a.cols = c->cols;
   a.n_cols = c->n_cols;
-  a.chunk_targets = c->chunk_targets;
+  a.chunk_targets = tile_targets(c);
   a.lds_cap = c->lds_cap;
+  a.quad = quad_tiles(c);
   a.chunks = c->chunks;
   a.counts = c->chunk_counts;
   a.grid_tile = c->grid_tile;

@@ -1,5 +1,5 @@
 // Per-pair arithmetic of the continuity and momentum right-hand sides, shared
-// by every traversal (LDS-staged strips and the global-memory path) so that
+// by every traversal (the tiles and the global-memory path) so that
 // all paths round identically.
 //
 // With r_ab = r_a - r_b and grad W_ab = G(q) r_ab (device_common.hpp):

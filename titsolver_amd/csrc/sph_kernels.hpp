@@ -77,6 +77,7 @@ struct StageArgs {
   uint32_t n_cols;
   uint32_t chunk_targets;
   uint32_t lds_cap;            // candidate positions staged in LDS at most
+  bool quad;                   // 2D tiles: four lanes per target
   uint4* chunks;
   uint32_t* counts;            // [0] column chunks, [2] block chunks
   uint32_t grid_tile, grid_global;  // persistent grid sizes
@@ -177,9 +178,19 @@ struct RebuildCtl {
 
 // Rebuild of a small set in one launch (rebuild_small.hip): at most kSmallN
 // particles in kSmallCells cells.  Its arrays are those of the large form's
-// kernels; it also resets the displacements.
-constexpr uint32_t kSmallN = 32768;
+// kernels; it also resets the displacements.  A full rebuild of 1,865, 6,215,
+// 14,735 and 26,278 particles takes 42, 101, 189 and 298 us in one workgroup,
+// some 100 us in the chain, whose launches cost 40 us of every step without a
+// rebuild: at 16,384 particles one launch wins up to 3 rebuilds in 10 steps
+// (2 to 10 in 100 on dam breaks), at 26,000 up to 2.
+constexpr uint32_t kSmallN = 16384;
 constexpr uint32_t kSmallCells = 65536;
+
+// Particles up to which the 2D tiles give each target four lanes.  One and
+// four lanes, us per launch between events: 1,295 and 6,215 particles 24.5 and
+// 18.1; 22,415 25.1 and 24.7; 38,727 25.9 and 30.3; 131,015 36.8 and 59.0
+// (four times the chunks, and each pair's sums added by all four lanes).
+constexpr uint32_t kQuadN = 24576;
 struct SmallRebuildArgs {
   uint32_t n, n_cells;
   int n_tanks, key_bits;

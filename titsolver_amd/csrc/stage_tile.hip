@@ -21,9 +21,11 @@
 // Bound: VALU issue (93 % of it at 2M particles: 1.52e8 wave instructions per
 // launch, about half in the pair loop, 43 per pair, and a third in the
 // predicate, 10.5 per candidate) and close behind it the LDS, about 80 % busy.
-// The 2M-particle dam break's launch takes 285 us; strips of one column with acceptance masks in registers and the
-// records gathered from L2 took 361 us and 1.71e8 (95 per pair).  Of that,
-// drawing chunks from a queue instead of fixed shares gave 50 us.
+// The 2M-particle dam break's launch takes 281 us; strips of one column with
+// acceptance masks in registers and the records gathered from L2 took 361 us
+// and 1.71e8 (95 per pair).  Of that, drawing chunks from a queue instead of
+// fixed shares gave 50 us.
+#include "chunk_build.hpp"
 #include "stage_common.hpp"
 
 namespace tit_amd {
@@ -182,6 +184,121 @@ __device__ __forceinline__ void tile_flush(const DevParams& P, const Tile& t, co
   }
 }
 
+// ---- four lanes per target ---------------------------------------------------
+// A set too small to fill the chip is one latency chain per lane: about 100
+// candidates tested and 25 term pairs summed in turn, 24.5 us a launch whatever
+// the chunk length, 18.1 with this (kQuadN has the sizes).  There a target has
+// the four lanes of a quad: each tests a
+// contiguous quarter of a pass of 4 kQuadPart candidates (so that the quad's
+// list keeps the candidate order), evaluates every fourth pair of terms, and
+// all four add the pairs in order, taking each other's by DPP.  Same bits.
+constexpr uint32_t kQuadPart = 6;
+constexpr uint32_t kQuadStride = 174;  // entries per target (87 words: spreads the banks)
+constexpr uint32_t kQuadList = kQuadStride - 2;
+static_assert(kQuadStride * (NT / 4) <= (kTileList + 2) * NT && kQuadStride % 2 == 0,
+              "lists of the quads fit those of the lanes, pairs word-aligned");
+
+// Value of lane S of this lane's quad.
+template <int S>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_mov_dpp(static_cast<int>(v), S * 0x55, 0xf, 0xf, true));
+}
+template <int S>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __uint_as_float(quad_lane<S>(__float_as_uint(v)));
+}
+
+// Adds lane S's pair sums if the quad has that pair.
+template <int S>
+__device__ __forceinline__ void quad_add(Sums<2>& acc, bool has, float c, float f0, float f1) {
+  const float cs = quad_lane<S>(c), s0 = quad_lane<S>(f0), s1 = quad_lane<S>(f1);
+  if (has) {
+    acc.rho.add(cs);
+    acc.v[0].add(s0);
+    acc.v[1].add(s1);
+  }
+}
+
+// tile_flush of a quad's list (t.list: its first entry; cnt the same in all
+// four lanes).
+template <int KERNEL, int FLAVOUR, bool LAST>
+__device__ __forceinline__ void quad_flush(const DevParams& P, const Tile& t, const Target<2>& a,
+                                           uint32_t& cnt, Sums<2>& acc) {
+  wave_lds_sync();  // entries of the other lanes
+  const uint32_t j = threadIdx.x & 3u, np = cnt >> 1;
+  for (uint32_t p = 0; p < np; p += 4) {  // uniform in the quad
+    const uint32_t w =
+        reinterpret_cast<const uint32_t*>(t.list)[min(p + j, np - 1)];
+    PairIn<2> A, B;
+    tile_take(t, w & 0xffffu, A);
+    tile_take(t, w >> 16, B);
+    float ca, fa[2], cb, fb[2];
+    term_of<2, KERNEL, FLAVOUR>(P, a, A, ca, fa);
+    term_of<2, KERNEL, FLAVOUR>(P, a, B, cb, fb);
+    const float c = ca + cb, f0 = fa[0] + fb[0], f1 = fa[1] + fb[1];
+    quad_add<0>(acc, true, c, f0, f1);
+    quad_add<1>(acc, p + 1 < np, c, f0, f1);
+    quad_add<2>(acc, p + 2 < np, c, f0, f1);
+    quad_add<3>(acc, p + 3 < np, c, f0, f1);
+  }
+  if (cnt & 1u) {
+    const uint32_t e = t.list[cnt - 1];
+    if constexpr (LAST) {
+      PairIn<2> A;
+      tile_take(t, e, A);
+      float ca, fa[2];
+      const float z[2] = {};
+      term_of<2, KERNEL, FLAVOUR>(P, a, A, ca, fa);
+      acc.add2(ca, fa, 0.0f, z);
+    } else {
+      wave_lds_sync();
+      t.list[0] = static_cast<uint16_t>(e);  // all four lanes write the same
+    }
+  }
+  if constexpr (!LAST) cnt &= 1u;
+  wave_lds_sync();
+}
+
+// One column's range [l, le) (uniform in the quad).
+template <int KERNEL, int FLAVOUR>
+__device__ __forceinline__ void quad_column(const DevParams& P, const Tile& t,
+                                            const Target<2>& a, uint32_t self, uint32_t l,
+                                            uint32_t le, uint32_t& cnt, uint32_t& count,
+                                            Sums<2>& acc) {
+  const uint32_t j = threadIdx.x & 3u;
+  while (__any(l < le)) {
+    if (__any(cnt + 4 * kQuadPart > kQuadList)) {
+      count += cnt & ~1u;
+      quad_flush<KERNEL, FLAVOUR, false>(P, t, a, cnt, acc);
+    }
+    const uint32_t c0 = l + kQuadPart * j;
+    double2 x[kQuadPart];
+#pragma unroll
+    for (uint32_t u = 0; u < kQuadPart; ++u) x[u] = t.xy[c0 + u < le ? c0 + u : self];
+    uint32_t mask = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kQuadPart; ++u) {
+      const double xb[2] = {x[u].x, x[u].y};
+      // (a candidate past the range's end stands for the target itself)
+      const bool ok = within<2>(P, xb, a.x) && c0 + u < le && c0 + u != self;
+      mask |= ok ? 1u << u : 0u;
+    }
+    const uint32_t n = static_cast<uint32_t>(__builtin_popcount(mask));
+    const uint32_t n0 = quad_lane<0>(n), n1 = quad_lane<1>(n), n2 = quad_lane<2>(n),
+                   n3 = quad_lane<3>(n);
+    uint32_t pos = cnt + (j > 0 ? n0 : 0u) + (j > 1 ? n1 : 0u) + (j > 2 ? n2 : 0u);
+#pragma unroll
+    for (uint32_t u = 0; u < kQuadPart; ++u) {  // the others go to the spare entry
+      const bool ok = (mask >> u) & 1u;
+      t.list[ok ? pos : kQuadStride - 1] = static_cast<uint16_t>((c0 + u) * 8);
+      pos += ok ? 1u : 0u;
+    }
+    cnt += n0 + n1 + n2 + n3;
+    l += 4 * kQuadPart;
+  }
+}
+
 // A target whose chunk does not fit: candidates straight from global memory,
 // the whole stencil.
 template <int KERNEL, int FLAVOUR>
@@ -207,18 +324,21 @@ __device__ __forceinline__ void sum_global(const StageArgs& A, const DevTank& T,
   acc.finish();
 }
 
-template <int KERNEL, int FLAVOUR, int KIND, bool FINAL>
+// Q: lanes per target, 1 or 4.
+template <int KERNEL, int FLAVOUR, int KIND, bool FINAL, int Q>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kTileWaves, kTileWaves))) void
 k_stage_tile(StageArgs A) {
   __shared__ double2 s_xy[kTileCap + 8];  // a lane loads up to 8 past its range
   __shared__ float4 s_pv[kTileCap];
   __shared__ float2 s_aux[kTileCap];
-  __shared__ uint16_t s_list[(kTileList + 2) * NT];
+  __shared__ __attribute__((aligned(4))) uint16_t s_list[(kTileList + 2) * NT];
   __shared__ uint16_t s_row[kWinC][kRows2 + 1];  // LDS index of each row's first candidate
   __shared__ uint32_t s_lb[kWinC + 1], s_d[kWinC];  // LDS index of each column; + d = global
   __shared__ uint32_t s_tb[kBlk2 + 1], s_first[kBlk2];  // targets before column; its first
   const DevParams& P = A.P;
   const int tid = threadIdx.x;
+  const uint32_t slot = tid / Q;           // target of the round
+  const bool lead = Q == 1 || tid % Q == 0;  // the lane that updates it
   __shared__ uint32_t s_next;
   ChunkQueue queue;
   queue.init(A.counts[2]);
@@ -277,7 +397,7 @@ k_stage_tile(StageArgs A) {
         }
       }
       __syncthreads();
-      target_of(tid, i, b, tag, zc);  // its loads overlap the staging's
+      target_of(slot, i, b, tag, zc);  // its loads overlap the staging's
       for (int r = tid; r < kWinC * (nrows + 1); r += NT) {
         const int k = r / (nrows + 1), row = r % (nrows + 1);
         const int ix = c.bx - kStencil + k;
@@ -336,9 +456,9 @@ k_stage_tile(StageArgs A) {
     }
     // targets, one per lane (a chunk that does not fit may need more rounds)
     const uint32_t n_t = s_tb[kBlk2];
-    for (uint32_t base = 0; base < n_t; base += NT) {
-      if (c.over) target_of(base + tid, i, b, tag, zc);
-      const bool in_range = base + tid < n_t, fluid = !(tag & 1u);
+    for (uint32_t base = 0; base < n_t; base += NT / Q) {
+      if (c.over) target_of(base + slot, i, b, tag, zc);
+      const bool in_range = base + slot < n_t, fluid = !(tag & 1u);
       const int cx = c.bx + b;
       Sums<2> acc;
       acc.init();
@@ -349,7 +469,7 @@ k_stage_tile(StageArgs A) {
         const uint32_t self = in_range ? i - s_d[b + kStencil] : s_lb[kStencil];
         const double2 xa = s_xy[self];
         target_of_record<FLAVOUR>(P, xa, s_pv[self], s_aux[self], a);
-        const Tile tile{s_xy, s_pv, s_aux, s_list + tid};
+        const Tile tile{s_xy, s_pv, s_aux, Q == 1 ? s_list + tid : s_list + slot * kQuadStride};
         const RowSpans W = row_spans(P, T, xa, cx, zc);
         const uint32_t self8 = self * 8;
         uint32_t cnt = 0;
@@ -363,6 +483,10 @@ k_stage_tile(StageArgs A) {
           e = min(e, zhi + 1);
           uint32_t l = s_row[b + k][f - zlo], le = s_row[b + k][e - zlo];
           if (!fluid || !(g2 <= W.t0)) le = l;
+          if constexpr (Q == 4) {
+            quad_column<KERNEL, FLAVOUR>(P, tile, a, self, l, le, cnt, count, acc);
+            continue;
+          }
           do {
             // a range longer than the list in pieces (never on a lattice)
             const uint32_t lp = min(le, l + static_cast<uint32_t>(kTileList - 8));
@@ -403,8 +527,12 @@ k_stage_tile(StageArgs A) {
           } while (__any(l < le));
         }
         count += cnt;
-        tile_flush<KERNEL, FLAVOUR, true>(P, tile, a, self8, cnt, acc);
-      } else if (c.over && fluid) {
+        if constexpr (Q == 4) {
+          quad_flush<KERNEL, FLAVOUR, true>(P, tile, a, cnt, acc);
+        } else {
+          tile_flush<KERNEL, FLAVOUR, true>(P, tile, a, self8, cnt, acc);
+        }
+      } else if (c.over && fluid && lead) {
         Target<2> a;
         target_of_record<FLAVOUR>(P, make_double2(A.in.x[0][i], A.in.x[1][i]), A.in.pv[i],
                                   A.in.aux[i], a);
@@ -412,11 +540,11 @@ k_stage_tile(StageArgs A) {
       }
       float vmax;
       unsigned long long dtmin;
-      if (tid == 0 && base + NT >= n_t) drawn = queue.take(A.work);
+      if (tid == 0 && base + NT / Q >= n_t) drawn = queue.take(A.work);
       TargetState<2> ts;
       load_target<2, KIND>(A, c.tank, i, ts);
-      finish_target<2, FLAVOUR, KIND, FINAL>(A, ts, i, in_range, fluid, acc, count, vmax,
-                                             dtmin);
+      finish_target<2, FLAVOUR, KIND, FINAL>(A, ts, i, in_range && lead, fluid && lead, acc,
+                                             count, vmax, dtmin);
       reduce_chunk<KIND, FINAL>(A, c.tank, vmax, dtmin, red);
     }
     if (tid == 0) s_next = queue.next(A.work, drawn);
@@ -426,16 +554,25 @@ k_stage_tile(StageArgs A) {
   red.flush(A);
 }
 
+template <int KERNEL, int FLAVOUR, int KIND, bool FINAL>
+void launch_lanes(hipStream_t s, const StageArgs& a) {
+  if (a.quad) {
+    k_stage_tile<KERNEL, FLAVOUR, KIND, FINAL, 4><<<a.grid_tile, NT, 0, s>>>(a);
+  } else {
+    k_stage_tile<KERNEL, FLAVOUR, KIND, FINAL, 1><<<a.grid_tile, NT, 0, s>>>(a);
+  }
+}
+
 template <int KERNEL, int FLAVOUR>
 void launch_flavour(hipStream_t s, const StageArgs& a, int kind, bool final) {
   if (kind == kRhsOnly) {
-    k_stage_tile<KERNEL, FLAVOUR, kRhsOnly, false><<<a.grid_tile, NT, 0, s>>>(a);
+    launch_lanes<KERNEL, FLAVOUR, kRhsOnly, false>(s, a);
   } else if (kind == kEuler) {
-    k_stage_tile<KERNEL, FLAVOUR, kEuler, false><<<a.grid_tile, NT, 0, s>>>(a);
+    launch_lanes<KERNEL, FLAVOUR, kEuler, false>(s, a);
   } else if (final) {
-    k_stage_tile<KERNEL, FLAVOUR, kCombine, true><<<a.grid_tile, NT, 0, s>>>(a);
+    launch_lanes<KERNEL, FLAVOUR, kCombine, true>(s, a);
   } else {
-    k_stage_tile<KERNEL, FLAVOUR, kCombine, false><<<a.grid_tile, NT, 0, s>>>(a);
+    launch_lanes<KERNEL, FLAVOUR, kCombine, false>(s, a);
   }
 }
 
@@ -457,7 +594,7 @@ void launch_kernel(hipStream_t s, const StageArgs& a, int kind, bool final) {
 int tile_groups_per_cu() {
   int n = 0;
   (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &n, reinterpret_cast<const void*>(k_stage_tile<kKernelC2, kFlavourCfg, kCombine, false>), NT,
+      &n, reinterpret_cast<const void*>(k_stage_tile<kKernelC2, kFlavourCfg, kCombine, false, 1>), NT,
       0);
   return std::max(n, 1);
 }

@@ -1,5 +1,5 @@
 // Learned step (network layout in surrogate.hpp): k-nearest graph, features,
-// training forward/backward on the BF16 MFMA GEMM, Adam, the 4 dt update, the
+// training forward/backward on the BF16 MFMA layers of nn_train.hip, Adam, the 4 dt update, the
 // judge/fallback controller and their C ABI.
 #include <algorithm>
 #include <cmath>
