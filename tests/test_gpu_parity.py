@@ -384,6 +384,82 @@ def test_tile_limits_keep_sets_and_bits(dim, n, box):
         ctx.close()
 
 
+@pytest.mark.parametrize("dim,dr,hf,flavour,masses", [
+    (2, 0.02, 5.0, ta.FLAVOUR_CFG, False), (2, 0.02, 4.0, ta.FLAVOUR_REF, True),
+    (2, 0.0085, 5.0, ta.FLAVOUR_CFG, True), (3, 0.03, 2.0, ta.FLAVOUR_REF, True)])
+def test_windows_too_large_for_a_tile_keep_bits(dim, dr, hf, flavour, masses):
+    """Smoothing lengths at which one row of cells is more than a tile holds:
+    every interior chunk takes its candidates from global memory, and the
+    steps have the bits of the column chunks."""
+    pa = perturbed_dam_break(dim, dr, seed=21,
+                             **({} if dim == 3 else {"tank": [3.22, 2.4], "column": [1.0, 1.9]}))
+    eq = ta.cfg_equations(dim, dr, 1.0, h_factor=hf, kernel=ta.KERNEL_WENDLAND_C4,
+                          flavour=flavour)
+    if masses:
+        pa.m = 1000.0 * dr ** dim * np.random.default_rng(5).uniform(0.9, 1.1, pa.n)
+    outs = []
+    for schedule in (None, (0, 0)):
+        ctx = _ctx(eq, [pa])
+        if schedule:
+            ctx.set_schedule(*schedule)
+        ctx.step(3)
+        outs.append({**ctx.download(), "pairs": ctx.pair_counts()})
+        ctx.close()
+    for f in ("r", "v", "rho", "pairs"):
+        assert np.array_equal(outs[0][f], outs[1][f]), f
+
+
+@pytest.mark.parametrize("per_row", [160, 300])
+def test_long_chunks_that_do_not_fit_keep_sets_and_bits(per_row):
+    """A dense strip one cell wide and 110 rows tall beside sparse particles:
+    the sparse block's rows hold less than a target each, but no window of
+    theirs fits, so its chunks run over as many rows as the builder looks at
+    at once (with four lanes per target and with one)."""
+    h = 0.02
+    rng = np.random.default_rng(per_row)
+    n = 110 * per_row
+    dense = np.stack([rng.uniform(0.068, 0.086, n), rng.uniform(0.0, 2.4, n)], -1)
+    sparse = np.stack([rng.uniform(0.09, 0.17, 60), rng.uniform(0.0, 2.4, 60)], -1)
+    r = np.concatenate([dense, sparse])
+    m = len(r)
+    pa = ta.ParticleArray(2, r, rng.uniform(990.0, 1010.0, m), m, np.zeros((0, 2)),
+                          (0.0, 0.0), (1.0, 2.4))
+    eq = _eq(2, 0.5 * h)
+    eq.h = h
+    ctx = _ctx(eq, [pa])
+    off, _ = ctx.neighbors()
+    assert np.array_equal(ctx.pair_counts().astype(np.int64), np.diff(off.astype(np.int64)) - 1)
+    got = ctx.compute_rhs()
+    ctx.set_schedule(0, 0)
+    ref = ctx.compute_rhs()
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+    ctx.close()
+
+
+def test_chunks_that_do_not_fit_keep_the_lanes_busy():
+    """At h = 5 spacings every chunk is beyond a tile: the default schedule's
+    stage kernel stays within 2.5 times the column chunks' (one row per chunk
+    and one candidate at a time took 4.5 times theirs, now 1.4)."""
+    pa = ta.dam_break(2, 0.02, [3.22, 2.4], [1.0, 2.0])
+    eq = ta.cfg_equations(2, 0.02, 2.0, h_factor=5.0)
+    us = []
+    for schedule in (None, (0, 0)):
+        ctx = _ctx(eq, [pa])
+        if schedule:
+            ctx.set_schedule(*schedule)
+        ctx.step(2)
+        best = 1e30
+        for _ in range(3):
+            ctx.set_profiling(True)
+            ctx.step(2)
+            calls, ms = ctx.kernel_stats()["stage"][:2]
+            ctx.set_profiling(False)
+            best = min(best, ms / calls)
+        us.append(best)
+        ctx.close()
+    assert us[0] < 2.5 * us[1], us
+
+
 @pytest.mark.parametrize("dim,n,width", [(2, 1, 0.1), (2, 1023, 0.5), (2, 1025, 5.0),
                                          (2, 16384, 2.1), (3, 4097, 0.4)])
 def test_small_rebuild_equals_large(dim, n, width):

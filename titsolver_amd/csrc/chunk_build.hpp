@@ -24,6 +24,9 @@ __host__ __device__ __forceinline__ ChunkLimits chunk_limits(uint32_t chunk_targ
   return ChunkLimits{kStage3Threads, lds_cap * kTile3Cap / kStage3LdsCap, kChunkRows3};
 }
 
+// Targets of a chunk that does not fit (several rows of it): one per lane.
+constexpr uint32_t kOverTargets = kTileThreads;
+static_assert(kStage3Threads == kTileThreads, "one limit for both tiles");
 constexpr int kSegRows = 256;
 
 // One wave's scratch: T(z) and W(z) of a segment of rows.
@@ -41,10 +44,13 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Block chunks of block b (all 64 lanes of a wave).  Greedy from the block's
 // first row: a chunk takes as many rows as keep its targets, its window's
 // candidates and its rows within their limits, the lanes testing the possible
-// end rows at once; rows without targets are skipped at both ends.  A single
-// row beyond a limit forms a chunk of its own that does not fit the LDS.  T(z) and W(z): particles of the block's and
-// of the window's columns below row z, each a sum of cell offsets (differences
-// are the counts), for a segment of rows in LDS.  With emit, the chunks are
+// end rows at once; rows without targets are skipped at both ends.  A row
+// beyond a limit by itself does not fit the LDS; consecutive such rows of at
+// most kOverTargets targets together (one at least) form a chunk that takes
+// its candidates from global memory, so that its lanes are busy.  T(z) and
+// W(z): particles of the block's and of the window's columns below row z, each
+// a sum of cell offsets (differences are the counts), for a segment of rows in
+// LDS.  With emit, the chunks are
 // written from `base` on.  Returns their number.
 template <int DIM>
 __device__ __forceinline__ uint32_t block_chunks(const StageArgs& A, uint32_t b, bool emit,
@@ -101,9 +107,15 @@ __device__ __forceinline__ uint32_t block_chunks(const StageArgs& A, uint32_t b,
     const int e = z + 1 + lane;
     const bool ok = lane < lim.rows && e <= nz && Tz(e) - Tz(z) <= lim.targets &&
                     Wz(e + S) - Wz(z - S) <= lim.window;
-    const uint64_t fit = ~__ballot(ok);
-    const int rows = max(1, static_cast<int>(__builtin_ctzll(fit)));
+    uint64_t fit = ~__ballot(ok);
     const uint32_t over = (fit & 1ull) ? 1u : 0u;
+    if (over) {
+      // and the rows after it that do not fit by themselves either
+      const bool with = e <= nz && Tz(e) - Tz(z) <= kOverTargets &&
+                        (Tz(e) - Tz(e - 1) > lim.targets || Wz(e + S) - Wz(e - 1 - S) > lim.window);
+      fit = ~__ballot(with);
+    }
+    const int rows = fit == 0 ? 64 : max(1, static_cast<int>(__builtin_ctzll(fit)));
     m &= rows < 64 ? (1ull << rows) - 1ull : ~0ull;
     const int end = z + 64 - __builtin_clzll(m);
     if (emit && lane == 0) {

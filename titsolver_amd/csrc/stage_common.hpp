@@ -17,16 +17,17 @@ namespace tit_amd {
 
 namespace {
 
-constexpr int kWordsG = 24;    // 32-candidate masks held per lane (global path)
+constexpr int kWordsG = 24;    // 32-candidate masks held per lane (column chunks)
 
-// Positions from global memory (any dimension).
-template <int DIM>
+// Positions from global memory (any dimension), WORDS acceptance masks per
+// lane between two pair loops.
+template <int DIM, int WORDS = kWordsG>
 struct GlobalPos {
   const DevTank& T;
   const DevState& S;
   const uint32_t* coff;
   int cx, cy;    // target column
-  uint32_t* wm;  // this wave's [kWordsG][64] 32-candidate acceptance masks
+  uint32_t* wm;  // this wave's [WORDS][64] 32-candidate acceptance masks
   uint32_t* wj;  // global index of each mask's bit 0
 
   __device__ __forceinline__ bool range(int k, int w0, int w1, uint32_t& b,
@@ -102,8 +103,8 @@ __device__ __forceinline__ bool within(const DevParams& P, const double* xb,
 // Global-memory path, the same scheme with 32-candidate masks (the 3D stencil
 // has 25 short column ranges): all columns' accepted candidates are summed
 // in one loop per lane, in the common candidate order.
-template <int DIM, int KERNEL, int FLAVOUR>
-__device__ __forceinline__ void sum_words_g(const DevParams& P, const GlobalPos<DIM>& ps,
+template <int DIM, int KERNEL, int FLAVOUR, int WORDS>
+__device__ __forceinline__ void sum_words_g(const DevParams& P, const GlobalPos<DIM, WORDS>& ps,
                                             const DevState& S, const Target<DIM>& a,
                                             uint32_t n_acc, Sums<DIM>& acc) {
   const int lane = threadIdx.x & 63;
@@ -114,7 +115,7 @@ __device__ __forceinline__ void sum_words_g(const DevParams& P, const GlobalPos<
     if (m == 0) {
       m = m_next;
       j0 = j_next;
-      w = min(w + 1, kWordsG - 1);
+      w = min(w + 1, WORDS - 1);
       m_next = ps.wm[w * 64 + lane];
       j_next = ps.wj[w * 64 + lane];
     }
@@ -160,9 +161,9 @@ __device__ __forceinline__ void sum_words_g(const DevParams& P, const GlobalPos<
   }
 }
 
-template <int DIM, int KERNEL, int FLAVOUR, int NCOL>
-__device__ __forceinline__ void gather_words_g(const DevParams& P, const GlobalPos<DIM>& ps,
-                                               const DevState& S, const Target<DIM>& a,
+template <int DIM, int KERNEL, int FLAVOUR, int NCOL, int WORDS>
+__device__ __forceinline__ void gather_words_g(const DevParams& P,
+                                               const GlobalPos<DIM, WORDS>& ps, const DevState& S, const Target<DIM>& a,
                                                uint32_t i, int zc, const Windows<DIM, NCOL>& W,
                                                Sums<DIM>& acc, uint32_t& count) {
   const int lane = threadIdx.x & 63;
@@ -172,7 +173,7 @@ __device__ __forceinline__ void gather_words_g(const DevParams& P, const GlobalP
   while (more) {
     int nw = 0;
     uint32_t n_acc = 0;
-    while (nw < kWordsG) {
+    while (nw < WORDS) {
       if (c0 >= e) {  // next non-empty column range
         bool found = false;
         for (; k < NCOL && !found; ++k) {
@@ -419,39 +420,28 @@ __device__ __forceinline__ void finish_target(const StageArgs& A,
   }
 }
 
-// One target (one lane), particle i of cell column (cx, cy) of tank `tank`
-// (col_row: the global index of the column's first cell), by the column-chunk
-// path.
-template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, class Pos>
-__device__ __forceinline__ void target_step(const StageArgs& A, const DevTank& T,
-                                            uint32_t tank, int cx, int cy, uint32_t col_row,
-                                            uint32_t i, bool in_range, const Pos& ps,
-                                            float& vmax, unsigned long long& dtmin) {
+// Pair sums of one fluid target (one lane), particle i of cell column (cx, cy)
+// (col_row: the global index of the column's first cell), every candidate from
+// global memory.
+template <int DIM, int KERNEL, int FLAVOUR, int WORDS>
+__device__ __forceinline__ void sum_from_global(const StageArgs& A, const DevTank& T, int cx,
+                                                int cy, uint32_t col_row, uint32_t i,
+                                                const GlobalPos<DIM, WORDS>& ps, Sums<DIM>& acc,
+                                                uint32_t& count) {
   constexpr int NCOL = DIM == 2 ? kCols2 : kCols2 * kCols2;
   const DevParams& P = A.P;
-  const uint32_t tag = in_range ? A.tag[i] : 1u;
-  const bool fluid = in_range && !(tag & 1u);
-  Sums<DIM> acc;
-  acc.init();
-  uint32_t count = 0;
-  TargetState<DIM> ts;
-  if (fluid) {
-    double xa[DIM], va[DIM];
+  double xa[DIM], va[DIM];
 #pragma unroll
-    for (int k = 0; k < DIM; ++k) {
-      xa[k] = A.in.x[k][i];
-      va[k] = A.in.v[k][i];
-    }
-    Target<DIM> a;
-    make_target<DIM, FLAVOUR>(P, xa, va, A.in.rho[i], A.in.aux[i], a);
-    const int zc = static_cast<int>(A.key[i] - col_row);
-    const Windows<DIM, NCOL> W =
-        stencil_windows<DIM, NCOL>(P, T, xa, cx, cy, zc);
-    gather_words_g<DIM, KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
-    acc.finish();
-    load_target<DIM, KIND>(A, tank, i, ts);
+  for (int k = 0; k < DIM; ++k) {
+    xa[k] = A.in.x[k][i];
+    va[k] = A.in.v[k][i];
   }
-  finish_target<DIM, FLAVOUR, KIND, FINAL>(A, ts, i, in_range, fluid, acc, count, vmax, dtmin);
+  Target<DIM> a;
+  make_target<DIM, FLAVOUR>(P, xa, va, A.in.rho[i], A.in.aux[i], a);
+  const int zc = static_cast<int>(A.key[i] - col_row);
+  const Windows<DIM, NCOL> W = stencil_windows<DIM, NCOL>(P, T, xa, cx, cy, zc);
+  gather_words_g<DIM, KERNEL, FLAVOUR, NCOL>(P, ps, A.in, a, i, zc, W, acc, count);
+  acc.finish();
 }
 
 // The per-wave reductions of one chunk's targets (all of one tank).
@@ -467,14 +457,24 @@ __device__ __forceinline__ void reduce_chunk(const StageArgs& A, uint32_t tank, 
 }
 
 // Targets of one column chunk, one per lane.
-template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, class Pos>
+template <int DIM, int KERNEL, int FLAVOUR, int KIND, bool FINAL, int WORDS>
 __device__ __forceinline__ void chunk_targets(const StageArgs& A, const ChunkInfo& c,
-                                              const Pos& ps, WaveReduce& red) {
+                                              const GlobalPos<DIM, WORDS>& ps, WaveReduce& red) {
   const uint32_t i = c.t0 + threadIdx.x;
+  const bool in_range = i < c.t1;
+  const uint32_t tag = in_range ? A.tag[i] : 1u;
+  const bool fluid = in_range && !(tag & 1u);
+  Sums<DIM> acc;
+  acc.init();
+  uint32_t count = 0;
+  TargetState<DIM> ts;
+  if (fluid) {
+    sum_from_global<DIM, KERNEL, FLAVOUR>(A, c.T, c.cx, c.cy, c.col_row, i, ps, acc, count);
+    load_target<DIM, KIND>(A, c.t, i, ts);
+  }
   float vmax;
   unsigned long long dtmin;
-  target_step<DIM, KERNEL, FLAVOUR, KIND, FINAL>(A, c.T, c.t, c.cx, c.cy, c.col_row, i,
-                                                 i < c.t1, ps, vmax, dtmin);
+  finish_target<DIM, FLAVOUR, KIND, FINAL>(A, ts, i, in_range, fluid, acc, count, vmax, dtmin);
   reduce_chunk<KIND, FINAL>(A, c.t, vmax, dtmin, red);
 }
 

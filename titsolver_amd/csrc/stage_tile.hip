@@ -39,6 +39,17 @@ constexpr int NT = kTileThreads;
 // that a lane can test four candidates at a time past its range's end (past
 // it in the same column lie rows beyond the stencil, which fail it too).
 constexpr uint32_t kPad = kTilePad;
+// Chunks that do not fit (h from 3.8 spacings on, and dense clumps) take their
+// candidates from global memory, one lane per target, with the acceptance
+// masks where the lists are: the column chunks' walk, trimmed stencils and
+// four candidates' loads in flight.  us per launch at h = 4 and 5 spacings,
+// with one candidate at a time of the whole stencil and one row per chunk,
+// and now: 6,218 particles 312, 680 and 121, 207; 131,030 particles 391, 580
+// and 249, 414.
+constexpr int kOverWords = 11;
+constexpr int kListLds = (kTileList + 2) * NT;
+static_assert(kOverWords * 64 * 2 * (NT / 64) * sizeof(uint32_t) <= kListLds * sizeof(uint16_t),
+              "masks fit the lists");
 
 // Pair records as plain vectors (arrays of the HIP vector classes go to
 // scratch memory here).
@@ -299,31 +310,6 @@ __device__ __forceinline__ void quad_column(const DevParams& P, const Tile& t,
   }
 }
 
-// A target whose chunk does not fit: candidates straight from global memory,
-// the whole stencil.
-template <int KERNEL, int FLAVOUR>
-__device__ __forceinline__ void sum_global(const StageArgs& A, const DevTank& T, int cx, int zc,
-                                           uint32_t i, const Target<2>& a, Sums<2>& acc,
-                                           uint32_t& count) {
-  const int z0 = max(zc - kStencil, 0), z1 = min(zc + kStencil, T.nc[1] - 1);
-  for (int ix = max(cx - kStencil, 0); ix <= min(cx + kStencil, T.nc[0] - 1); ++ix) {
-    const uint32_t row = T.cell_off + static_cast<uint32_t>(ix) * T.nc[1];
-    const uint32_t e = A.cell_off[row + z1 + 1];
-    for (uint32_t j = A.cell_off[row + z0]; j < e; ++j) {
-      PairIn<2> p;
-      p.x[0] = A.in.x[0][j];
-      p.x[1] = A.in.x[1][j];
-      if (j == i || !within<2>(A.P, p.x, a.x)) continue;
-      p.pv = A.in.pv[j];
-      p.aux = A.in.aux[j];
-      p.vol = 0.0f;
-      sum_pair<2, KERNEL, FLAVOUR>(A.P, a, p, acc);
-      ++count;
-    }
-  }
-  acc.finish();
-}
-
 // Q: lanes per target, 1 or 4.
 template <int KERNEL, int FLAVOUR, int KIND, bool FINAL, int Q>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kTileWaves, kTileWaves))) void
@@ -331,14 +317,12 @@ k_stage_tile(StageArgs A) {
   __shared__ double2 s_xy[kTileCap + 8];  // a lane loads up to 8 past its range
   __shared__ float4 s_pv[kTileCap];
   __shared__ float2 s_aux[kTileCap];
-  __shared__ __attribute__((aligned(4))) uint16_t s_list[(kTileList + 2) * NT];
+  __shared__ __attribute__((aligned(4))) uint16_t s_list[kListLds];
   __shared__ uint16_t s_row[kWinC][kRows2 + 1];  // LDS index of each row's first candidate
   __shared__ uint32_t s_lb[kWinC + 1], s_d[kWinC];  // LDS index of each column; + d = global
   __shared__ uint32_t s_tb[kBlk2 + 1], s_first[kBlk2];  // targets before column; its first
   const DevParams& P = A.P;
   const int tid = threadIdx.x;
-  const uint32_t slot = tid / Q;           // target of the round
-  const bool lead = Q == 1 || tid % Q == 0;  // the lane that updates it
   __shared__ uint32_t s_next;
   ChunkQueue queue;
   queue.init(A.counts[2]);
@@ -349,6 +333,9 @@ k_stage_tile(StageArgs A) {
     const int nz = T.nc[1];
     const int zlo = max(c.zs - kStencil, 0), zhi = min(c.ze - 1 + kStencil, nz - 1);
     const int nrows = zhi - zlo + 1;
+    const uint32_t per = c.over ? NT : NT / Q;            // targets of a round
+    const uint32_t slot = c.over ? tid : tid / Q;         // this lane's
+    const bool lead = Q == 1 || c.over || tid % Q == 0;   // the lane that updates it
     uint32_t drawn = ~0u;
     // target t of the chunk: its particle, column in the block, tag and row
     auto target_of = [&](uint32_t t, uint32_t& i, int& b, uint32_t& tag, int& zc) {
@@ -456,7 +443,7 @@ k_stage_tile(StageArgs A) {
     }
     // targets, one per lane (a chunk that does not fit may need more rounds)
     const uint32_t n_t = s_tb[kBlk2];
-    for (uint32_t base = 0; base < n_t; base += NT / Q) {
+    for (uint32_t base = 0; base < n_t; base += per) {
       if (c.over) target_of(base + slot, i, b, tag, zc);
       const bool in_range = base + slot < n_t, fluid = !(tag & 1u);
       const int cx = c.bx + b;
@@ -532,15 +519,16 @@ k_stage_tile(StageArgs A) {
         } else {
           tile_flush<KERNEL, FLAVOUR, true>(P, tile, a, self8, cnt, acc);
         }
-      } else if (c.over && fluid && lead) {
-        Target<2> a;
-        target_of_record<FLAVOUR>(P, make_double2(A.in.x[0][i], A.in.x[1][i]), A.in.pv[i],
-                                  A.in.aux[i], a);
-        sum_global<KERNEL, FLAVOUR>(A, T, cx, zc, i, a, acc, count);
+      } else if (c.over && fluid) {
+        uint32_t* words = reinterpret_cast<uint32_t*>(s_list) + (tid >> 6) * kOverWords * 128;
+        const GlobalPos<2, kOverWords> ps{T,  A.in, A.cell_off, cx, 0, words,
+                                          words + kOverWords * 64};
+        sum_from_global<2, KERNEL, FLAVOUR>(
+            A, T, cx, 0, T.cell_off + static_cast<uint32_t>(cx) * nz, i, ps, acc, count);
       }
       float vmax;
       unsigned long long dtmin;
-      if (tid == 0 && base + NT / Q >= n_t) drawn = queue.take(A.work);
+      if (tid == 0 && base + per >= n_t) drawn = queue.take(A.work);
       TargetState<2> ts;
       load_target<2, KIND>(A, c.tank, i, ts);
       finish_target<2, FLAVOUR, KIND, FINAL>(A, ts, i, in_range && lead, fluid && lead, acc,

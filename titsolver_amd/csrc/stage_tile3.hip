@@ -34,6 +34,16 @@ constexpr int NW = kWin3 * kWin3;
 constexpr int NB = kBlk3 * kBlk3;
 static_assert(NW == 64, "one lane of a wave per window column");
 static_assert(kTile3Cap <= 2040, "an LDS index takes 11 bits");
+// Chunks that do not fit take their candidates from global memory (the column
+// chunks' walk), with the acceptance masks where the lists are.  At h = 2
+// spacings every interior window is one (about 3,400 candidates in one row):
+// 1.5M particles take 5,750 us per launch, as many with one candidate at a
+// time of the untrimmed stencil 7,610, column chunks 11,000 (their workgroups
+// read one column's neighbourhood each).
+constexpr int kOverWords = 16;
+constexpr int kListLds = (kTile3List + 2) * NT;
+static_assert(kOverWords * 64 * 2 * (NT / 64) * sizeof(uint32_t) <= kListLds * sizeof(uint16_t),
+              "masks fit the lists");
 constexpr uint32_t kColMax = 255;   // candidates of one window column at most
 constexpr uint32_t kSpanMax = 1u << 27;  // global-index span of a window
 
@@ -104,39 +114,11 @@ __device__ __forceinline__ void tile_flush3(const DevParams& P, const Tile3& t,
   }
 }
 
-// A target whose chunk does not fit: candidates straight from global memory,
-// the whole stencil.
-template <int KERNEL, int FLAVOUR>
-__device__ __forceinline__ void sum_global3(const StageArgs& A, const DevTank& T, int cx, int cy,
-                                            int zc, uint32_t i, const Target<3>& a, Sums<3>& acc,
-                                            uint32_t& count) {
-  const int z0 = max(zc - kStencil, 0), z1 = min(zc + kStencil, T.nc[2] - 1);
-  for (int ix = max(cx - kStencil, 0); ix <= min(cx + kStencil, T.nc[0] - 1); ++ix) {
-    for (int iy = max(cy - kStencil, 0); iy <= min(cy + kStencil, T.nc[1] - 1); ++iy) {
-      const uint32_t row =
-          T.cell_off + (static_cast<uint32_t>(ix) * T.nc[1] + static_cast<uint32_t>(iy)) * T.nc[2];
-      const uint32_t e = A.cell_off[row + z1 + 1];
-      for (uint32_t j = A.cell_off[row + z0]; j < e; ++j) {
-        PairIn<3> p;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) p.x[k] = A.in.x[k][j];
-        if (j == i || !within<3>(A.P, p.x, a.x)) continue;
-        p.pv = A.in.pv[j];
-        p.aux = A.in.aux[j];
-        p.vol = mass_flavour(FLAVOUR) ? A.in.vol[j] : 0.0f;
-        sum_pair<3, KERNEL, FLAVOUR>(A.P, a, p, acc);
-        ++count;
-      }
-    }
-  }
-  acc.finish();
-}
-
 template <int KERNEL, int FLAVOUR, int KIND, bool FINAL>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_stage_tile3(
     StageArgs A) {
   __shared__ double s_x[kTile3Cap + 8], s_y[kTile3Cap + 8], s_z[kTile3Cap + 8];
-  __shared__ uint16_t s_list[(kTile3List + 2) * NT];
+  __shared__ __attribute__((aligned(4))) uint16_t s_list[kListLds];
   __shared__ uint16_t s_row[NW][kRows3 + 1];  // LDS index of each row's first candidate
   __shared__ uint2 s_base[NW];
   __shared__ uint32_t s_lb[NW + 1], s_d[NW];  // LDS index of each column; + d = global
@@ -383,15 +365,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         count += cnt;
         tile_flush3<KERNEL, FLAVOUR, true>(P, tile, a, self_e, cnt, acc);
       } else if (!fits && fluid) {
-        double xa[3], va[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          xa[k] = A.in.x[k][i];
-          va[k] = A.in.v[k][i];
-        }
-        Target<3> a;
-        make_target<3, FLAVOUR>(P, xa, va, A.in.rho[i], A.in.aux[i], a);
-        sum_global3<KERNEL, FLAVOUR>(A, T, bx + b / kBlk3, by + b % kBlk3, zc, i, a, acc, count);
+        const int cx = bx + b / kBlk3, cy = by + b % kBlk3;
+        uint32_t* words = reinterpret_cast<uint32_t*>(s_list) + (tid >> 6) * kOverWords * 128;
+        const GlobalPos<3, kOverWords> ps{T,  A.in, A.cell_off, cx, cy, words,
+                                          words + kOverWords * 64};
+        sum_from_global<3, KERNEL, FLAVOUR>(
+            A, T, cx, cy,
+            T.cell_off + (static_cast<uint32_t>(cx) * T.nc[1] + static_cast<uint32_t>(cy)) * nz, i,
+            ps, acc, count);
       }
       if (tid == 0 && base + NT >= n_t) drawn = queue.take(A.work);
       TargetState<3> ts;
