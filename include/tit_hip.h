@@ -226,7 +226,9 @@ tit_status tit_hip_kernel_stats(tit_hip_ctx* ctx, tit_hip_kernel_stat* out,
  *    a block of cell columns over a few rows (4 columns in 2D, 4 x 4 in 3D)
  *    with the block's window in LDS; lds_capacity bounds the window's
  *    candidates (in 3D in proportion to the kernel's own capacity), and in 2D
- *    chunk_targets the tile's particles (2 chunk_targets of them);
+ *    chunk_targets the tile's particles (2 chunk_targets of them; up to
+ *    24,576 particles in all a 2D tile has four lanes per particle and at most
+ *    64 particles, so values above 32 are as 32);
  *  - column chunks (lds_capacity 0): a workgroup takes at most chunk_targets
  *    consecutive particles of one cell column, one per lane, and reads
  *    positions from global memory.  Results
@@ -247,11 +249,12 @@ tit_status tit_hip_get_schedule(tit_hip_ctx* ctx, tit_hip_schedule* out);
 tit_status tit_hip_set_schedule(tit_hip_ctx* ctx, const tit_hip_schedule* s);
 
 /* Autotuner of the stage schedule: times every candidate (chunk_targets in
- * {32, 48, 64, 96, 128} x LDS capacity {max, max/2, 0}) over
- * steps_per_candidate real steps of the current state (all schedules give the
- * same bits, so the steps are ordinary progress), keeps the fastest and
- * returns it with its time per step.  The result is kept in a per-process
- * cache keyed by (dimension, kernel, term set, walls, one or many tanks, the
+ * {32, 48, 64, 96, 128} x LDS capacity {max, max/2, 0}; one chunk_targets
+ * only where the tiles do not depend on it) over steps_per_candidate real
+ * steps of the current state (all schedules give the same bits, so the steps
+ * are ordinary progress), keeps the fastest and returns it with its time per
+ * step.  The result is kept in a per-process cache keyed by (dimension,
+ * kernel, term set, walls, one or many tanks, the tiles' lanes per target, the
  * particle count's power of two): a later call on a context of the same key
  * applies the cached schedule without timing (best->cached = 1, no steps
  * taken).  No reference counterpart. */

@@ -282,6 +282,36 @@ def test_autotune_cache_reuses_the_schedule(dim):
         x.close()
 
 
+@pytest.mark.parametrize("dim,dr,candidates", [(2, 0.02, 7), (2, 0.009, 15), (3, 0.03, 7)])
+def test_autotune_times_each_schedule_once(dim, dr, candidates):
+    """Tiles that do not depend on the chunk length (3D, and 2D with four lanes
+    per target) are timed once per capacity, every other schedule once."""
+    ta.HipContext.clear_autotune_cache()
+    pa = perturbed_dam_break(dim, dr, seed=4, **({} if dim == 3 else {"tank": [3.2, 2.4],
+                                                                      "column": [1.0, 2.0]}))
+    assert dim == 3 or (pa.n > 24576) == (candidates == 15)
+    ctx = _ctx(_eq(dim, dr), [pa])
+    best = ctx.autotune(2)
+    assert ctx.counts()[2] == candidates * 4  # 2 steps of warm-up, 2 timed
+    if candidates == 7 and best["lds_capacity"] > 0:
+        assert best["chunk_targets"] == (32 if dim == 2 else 128)
+    ctx.close()
+
+
+def test_autotune_cache_splits_at_four_lanes_per_target():
+    """Sets of one power of two on both sides of the four-lane limit (24,576)
+    do not share a cache entry."""
+    ta.HipContext.clear_autotune_cache()
+    sizes = []
+    for dr in (0.0113, 0.0093):
+        pa = ta.dam_break(2, dr, [3.2, 2.4], [1.0, 2.0])
+        sizes.append(pa.n)
+        ctx = _ctx(_eq(2, dr), [pa])
+        assert not ctx.autotune(2)["cached"]
+        ctx.close()
+    assert 16384 <= sizes[0] <= 24576 < sizes[1] < 32768, sizes
+
+
 @pytest.mark.parametrize("dim,dr,schedule", [(2, 0.02, (0, None)), (2, 0.02, (0, 0)),
                                              (2, 0.01, (64, None)), (3, 0.025, (0, None))])
 def test_stage_kernel_sums_exactly_the_neighbour_sets(dim, dr, schedule):

@@ -250,9 +250,8 @@ StageArgs stage_args(tit_hip_ctx* c);
 
 // Whether the 2D tiles give each target four lanes (stage_tile.hip), and the
 // chunk length that the schedule then has: a quarter of the lanes' targets.
-bool quad_tiles(const tit_hip_ctx* c) {
-  return c->dp.dim == 2 && c->lds_cap > 0 && c->n <= kQuadN;
-}
+bool quad_set(const tit_hip_ctx* c) { return c->dp.dim == 2 && c->n <= kQuadN; }
+bool quad_tiles(const tit_hip_ctx* c) { return quad_set(c) && c->lds_cap > 0; }
 uint32_t tile_targets(const tit_hip_ctx* c) {
   return quad_tiles(c) ? std::min<uint32_t>(c->chunk_targets, kChunkMax / 4) : c->chunk_targets;
 }
@@ -663,13 +662,13 @@ NeighborScratch* scratch_ptr(int device) {
 }
 
 // The autotuner's per-process cache: the schedule found for a kind of
-// context (dimension, kernel, term set, walls, one or many tanks) and size
-// (the particle count's power of two).
+// context (dimension, kernel, term set, walls, one or many tanks, four lanes
+// per target in its tiles) and size (the particle count's power of two).
 struct TuneKey {
-  int dim, kernel, flavour, walls, batched, log2n;
+  int dim, kernel, flavour, walls, batched, quad, log2n;
   bool operator<(const TuneKey& o) const {
-    return std::tie(dim, kernel, flavour, walls, batched, log2n) <
-           std::tie(o.dim, o.kernel, o.flavour, o.walls, o.batched, o.log2n);
+    return std::tie(dim, kernel, flavour, walls, batched, quad, log2n) <
+           std::tie(o.dim, o.kernel, o.flavour, o.walls, o.batched, o.quad, o.log2n);
   }
 };
 struct TuneVal {
@@ -683,7 +682,7 @@ TuneKey tune_key(const tit_hip_ctx* c) {
   int log2n = 0;
   while ((static_cast<size_t>(1) << (log2n + 1)) <= c->n) ++log2n;
   return TuneKey{c->prm.dim, c->prm.kernel, c->dp.flavour, c->walls ? 1 : 0,
-                 c->n_tanks > 1 ? 1 : 0, log2n};
+                 c->n_tanks > 1 ? 1 : 0, quad_set(c) ? 1 : 0, log2n};
 }
 
 }  // namespace
@@ -1610,6 +1609,10 @@ tit_status tit_hip_autotune(tit_hip_ctx* c, int steps_per_candidate,
   tit_status st = TIT_OK;
   for (uint32_t ch : chunks) {
     for (uint32_t cap : caps) {
+      // 3D tiles and those of four lanes per target are the same for every
+      // chunk length: timed once, with the length they have
+      if (cap > 0 && c->prm.dim == 3 && ch != kChunkMax) continue;
+      if (cap > 0 && quad_set(c) && ch != kChunkMax / 4) continue;
       c->chunk_targets = ch;
       c->lds_cap = cap;
       st = build_schedule(c);
