@@ -544,10 +544,11 @@ def test_wide_boundary_groups_keep_the_bits(dim, dr):
     b.close()
 
 
-@pytest.mark.parametrize("n", [1, 16384, 16385, 120000, 160001])
+@pytest.mark.parametrize("n", [1, 16384, 16385, 120000, 160001, 262143, 262145])
 def test_download_pieces(n):
     """Frames around the limits of the download's staging (1 MiB in one copy,
-    8 pieces of 1 MiB among the workers): what was uploaded comes back, in
+    8 pieces of 1 MiB among the workers; none in a context's first download
+    below 16 MiB): what was uploaded comes back, in
     the uploaded order."""
     rng = np.random.default_rng(n)
     r = rng.uniform(0.0, 1.0, (n, 3))

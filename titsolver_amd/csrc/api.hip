@@ -1177,18 +1177,26 @@ struct HostCopy {
 };
 
 // Device arrays to pageable host memory through pinned staging.  The runtime's
-// own copy to pageable memory runs on one thread, at 7 to 16 GB/s, much of it
-// page faults of a freshly allocated destination, and costs 25 to 45 us for
-// each array.  Up to one piece (1 MiB) is staged whole and copied out by the
-// caller: 95 -> 52 us for 800 particles, 180 -> 66 us for 4,900.  From 8
-// pieces on, worker threads each own a staging slot: a worker queues its
+// own copy to pageable memory costs some 20 us for each array and runs on one
+// thread, which also faults in the pages of a freshly allocated destination.
+// Up to one piece (1 MiB) is staged whole and copied out by the caller.  From
+// 8 pieces on, worker threads each own a staging slot: a worker queues its
 // piece's transfer, waits for it and copies it out while the other workers'
-// pieces are in flight: 2.3 -> 1.2 ms for 24 MB, 9.4 -> 3.3 ms for 97 MB,
-// 12.8 -> 5.7 ms for 129 MB.  Between the two the runtime's copy is as fast
-// (6 MB: 350 and 360 us).  Smaller pieces wait too often: 97 MB take 7.2 ms in
-// pieces of 256 KiB and 4.8 ms in pieces of 512 KiB.  The staging (8 MiB at
-// most) stays with the context.
+// pieces are in flight.  us into memory touched before and into new pages,
+// runtime and staged: 0.06 MB 91, 105 and 45, 57; 0.8 MB 80, 227 and 79, 228;
+// 6.3 MB 338, 1,508 and 337, 661; 25 MB 1,416, 6,439 and 873, 2,691; 97 MB
+// 5,255, 25,877 and 3,123, 9,645.  Between the two the runtime's copy stays
+// (2.5 MB 147, 570 and 207, 360).  Smaller pieces wait too often: 97 MB take
+// 7.2 ms in pieces of 256 KiB and 4.8 ms in pieces of 512 KiB where pieces of
+// 1 MiB take 3.3.
+// The staging (8 MiB at most) stays with the context.  Making it and touching
+// it first costs 25 to 45 us up to a piece and 0.8 ms for all slots, so a
+// context's first download is staged only from kFirstStagedBytes on, where
+// that is won back in the same call (first downloads, runtime and staged: 0.3
+// MB 70 and 101 us; 11 MB 1.35 and 2.1 ms; 16 MB 2.9 and 2.0; 25 MB 2.9 to 4.4
+// and 2.3 ms).
 // A destination that the runtime knows (pinned memory) is copied to directly.
+constexpr size_t kFirstStagedBytes = size_t(16) << 20;
 constexpr size_t kPiece = size_t(1) << 20;
 constexpr int kSlots = 8;
 
@@ -1211,7 +1219,9 @@ hipError_t copy_out(tit_hip_ctx* c, const HostCopy* copies, int n_copies) {
   }
   if (total == 0) return hipStreamSynchronize(c->stream);
   const bool one = total <= kPiece;
-  staged = staged && (one || n_pieces >= kSlots);
+  staged = staged && (one || n_pieces >= kSlots) &&
+           (c->copied_out || total >= kFirstStagedBytes);
+  c->copied_out = true;
   const size_t need = one ? total : kSlots * kPiece;
   if (staged && c->pinned_bytes < need) {
     if (c->pinned) (void)hipHostFree(c->pinned);

@@ -118,7 +118,9 @@ struct tit_hip_ctx {
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   hipGraph_t graph_def[2] = {nullptr, nullptr};
 
-  // pinned staging of the downloads (tit_hip_download), made on first use
+  // pinned staging of the downloads (tit_hip_download), made on first use;
+  // whether there was a download before
+  bool copied_out = false;
   void* pinned = nullptr;
   size_t pinned_bytes = 0;
 
