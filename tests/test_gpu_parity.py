@@ -490,6 +490,35 @@ def test_chunks_that_do_not_fit_keep_the_lanes_busy():
     assert us[0] < 2.5 * us[1], us
 
 
+@pytest.mark.parametrize("dim,size", [(2, (0.2, 60.0)), (2, (0.3, 110.0)), (2, (100.0, 7.0)),
+                                      (3, (0.1, 0.1, 30.0))])
+def test_chunk_lists_over_many_rows(dim, size):
+    """Tanks of more cell rows than the chunk builder holds at once (by the
+    single-launch rebuild, by wide workgroups, by a wave for each of many
+    blocks, in 3D), with clumps, gaps of hundreds of empty rows and single
+    particles: every target is summed once, over its neighbours."""
+    h = 0.02
+    rng = np.random.default_rng(int(size[0] * 10))
+    lo, hi = np.zeros(dim), np.array(size)
+    spread = rng.uniform(lo, hi, (1500, dim))
+    clumps = np.concatenate([np.clip(rng.normal(c, 0.03, (150, dim)), lo, hi)
+                             for c in rng.uniform(lo, hi, (20, dim))])
+    column = rng.uniform(lo, hi, (1500, dim))
+    column[:, -1] = rng.uniform(0.31 * hi[-1], 0.36 * hi[-1], 1500)
+    ends = np.array([lo, hi])
+    r = np.concatenate([spread, clumps, column, ends])
+    n = len(r)
+    pa = ta.ParticleArray(dim, r, rng.uniform(990.0, 1010.0, n), n, np.zeros((0, dim)),
+                          tuple(lo), tuple(hi))
+    eq = _eq(dim, 0.5 * h)
+    eq.h = h
+    ctx = _ctx(eq, [pa])
+    want = oracle.naive_search(r, 2.0 * h)
+    counts = ctx.pair_counts().astype(np.int64)
+    assert np.array_equal(counts, np.diff(want[0].astype(np.int64)) - 1)
+    ctx.close()
+
+
 @pytest.mark.parametrize("dim,n,width", [(2, 1, 0.1), (2, 1023, 0.5), (2, 1025, 5.0),
                                          (2, 16384, 2.1), (3, 4097, 0.4)])
 def test_small_rebuild_equals_large(dim, n, width):

@@ -446,16 +446,21 @@ tit_status build_schedule(tit_hip_ctx* c) {
     // blocks of kBlk2 columns (2D), kBlk3 x kBlk3 (3D)
     const int bw = dim == 2 ? kBlk2 : kBlk3;
     std::vector<uint4> blocks;
+    size_t rows = 0;
     for (size_t t = 0; t < c->host_tanks.size(); ++t) {
       const DevTank& T = c->host_tanks[t];
       for (int bx = 0; bx < T.nc[0]; bx += bw) {
         for (int by = 0; by < (dim == 2 ? 1 : T.nc[1]); by += bw) {
-          blocks.push_back(make_uint4(static_cast<uint32_t>(t), bx, by, 0u));
+          blocks.push_back(
+              make_uint4(static_cast<uint32_t>(t), bx, by, static_cast<uint32_t>(rows)));
+          rows += T.nc[dim - 1];
         }
       }
     }
     TIT_HIP_TRY(c, dalloc(c, &c->blocks, blocks.size()));
     TIT_HIP_TRY(c, dalloc(c, &c->bcount, blocks.size() + 1));
+    TIT_HIP_TRY(c, dalloc(c, &c->bcuts, rows));
+    c->block_rows = nz_max;
     TIT_HIP_TRY(c, hipMemcpy(c->blocks, blocks.data(), blocks.size() * sizeof(uint4),
                              hipMemcpyHostToDevice));
     c->n_blocks = static_cast<uint32_t>(blocks.size());
@@ -498,6 +503,8 @@ StageArgs stage_args(tit_hip_ctx* c) {
   a.n_blocks = c->n_blocks;
   a.bchunks = c->bchunks;
   a.bcount = c->bcount;
+  a.bcuts = c->bcuts;
+  a.block_rows = c->block_rows;
   a.P = c->dp;
   a.tanks = c->tanks;
   a.key = c->key;
@@ -1140,6 +1147,7 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   c->blocks = nullptr;
   c->bchunks = nullptr;
   c->bcount = nullptr;
+  c->bcuts = nullptr;
   c->n_blocks = 0;
   c->bchunk_cap = 0;
   c->n_cols = 0;

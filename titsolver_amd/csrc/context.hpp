@@ -109,6 +109,8 @@ struct tit_hip_ctx {
   uint32_t n_blocks = 0;
   uint4* bchunks = nullptr;
   uint32_t* bcount = nullptr;
+  uint2* bcuts = nullptr;
+  int block_rows = 0;
   size_t bchunk_cap = 0;
   int n_cu = 0;
   double occupancy = 1.0;  // mean particles per occupied cell at upload

@@ -115,8 +115,9 @@ __global__ __launch_bounds__(NT) void k_rebuild_small(SmallRebuildArgs R) {
   __shared__ __attribute__((aligned(16))) unsigned char raw[sizeof(SortScratchLds)];
   __shared__ uint32_t s_wsum[kWaves], s_fixed, s_active;
   SortScratchLds& S = *reinterpret_cast<SortScratchLds*>(raw);
-  ChunkScratch* chunk_scratch = reinterpret_cast<ChunkScratch*>(raw);
-  static_assert(sizeof(ChunkScratch) * kWaves <= sizeof(SortScratchLds), "scratch overlay");
+  using WaveScratch = ChunkScratch<256>;
+  WaveScratch* chunk_scratch = reinterpret_cast<WaveScratch*>(raw);
+  static_assert(sizeof(WaveScratch) * kWaves <= sizeof(SortScratchLds), "scratch overlay");
   const DevParams& P = R.b.P;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t n = R.n;
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(NT) void k_rebuild_small(SmallRebuildArgs R) {
   const StageArgs& A = R.s;
   if (A.lds_cap > 0) {
     for (uint32_t b = wave; b < A.n_blocks; b += kWaves) {
-      const uint32_t c = block_chunks<DIM>(A, b, false, 0u, chunk_scratch[wave]);
+      const uint32_t c = block_chunks<DIM, 64>(A, b, chunk_scratch[wave]);
       if (lane == 0) A.bcount[b] = c;
     }
     __syncthreads();
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(NT) void k_rebuild_small(SmallRebuildArgs R) {
       __syncthreads();
     }
     for (uint32_t b = wave; b < A.n_blocks; b += kWaves) {
-      (void)block_chunks<DIM>(A, b, true, A.bcount[b], chunk_scratch[wave]);
+      emit_block_chunks<DIM>(A, b, b + 1 < A.n_blocks ? A.bcount[b + 1] : before);
     }
     if (tid == 0) A.counts[2] = before;
   }

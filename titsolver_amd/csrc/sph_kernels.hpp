@@ -83,14 +83,17 @@ struct StageArgs {
   uint32_t grid_tile, grid_global;  // persistent grid sizes
   uint32_t* work;                   // this launch's set of chunk-queue counters
   // with LDS staging (lds_cap > 0): cell-column blocks (tank, first ix,
-  // first iy, 0), rebuilt on the device after every cell rebuild: block
+  // first iy, rows of the blocks before), rebuilt on the device after every cell rebuild: block
   // chunks (2D: tank | does not fit the LDS << 31, first ix, first row, end
-  // row; 3D: block, first row, end row, does not fit) and per-block chunk
-  // counts (scanned in place)
+  // row; 3D: block, first row, end row, does not fit), per-block chunk counts
+  // (scanned in place) and, while the list is made, each block's chunks
+  // (first row, end row | does not fit << 31)
   const uint4* blocks;
   uint32_t n_blocks;
+  int block_rows;              // of the tallest tank
   uint4* bchunks;
   uint32_t* bcount;
+  uint2* bcuts;
   double* dv_last[3];          // final stage: its acceleration (post-integration only)
   // semi-analytic wall (kFlavourWall): per slot, the face terms of drho/dt
   // and dv/dt already divided by gamma, then gamma

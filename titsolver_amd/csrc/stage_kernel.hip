@@ -35,15 +35,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 3))) void
   red.flush(A);
 }
 
-// One wave per block; with emit from the block's scanned offset, otherwise the
-// count goes to bcount.
-template <int DIM>
-__global__ __launch_bounds__(64) void k_block_chunks(StageArgs A, int emit, const uint32_t* ctl) {
+// Chunks of the blocks, one workgroup each, and their counts.
+template <int DIM, int LANES, int ROWS>
+__global__ __launch_bounds__(LANES) void k_block_chunks(StageArgs A, const uint32_t* ctl) {
   if (!ctl[0]) return;
-  __shared__ ChunkScratch sc;
-  const uint32_t b = blockIdx.x;
-  const uint32_t n = block_chunks<DIM>(A, b, emit != 0, emit ? A.bcount[b] : 0u, sc);
-  if (threadIdx.x == 0 && !emit) A.bcount[b] = n;
+  __shared__ ChunkScratch<ROWS> sc;
+  const uint32_t n = block_chunks<DIM, LANES>(A, blockIdx.x, sc);
+  if (threadIdx.x == 0) A.bcount[blockIdx.x] = n;
+}
+
+// The blocks' chunks into one list (counts scanned), one wave per block.
+constexpr int kEmitBlocks = 4;
+template <int DIM>
+__global__ __launch_bounds__(64 * kEmitBlocks) void k_block_emit(StageArgs A,
+                                                                 const uint32_t* ctl) {
+  if (!ctl[0]) return;
+  const uint32_t b = blockIdx.x * kEmitBlocks + (threadIdx.x >> 6);
+  if (b >= A.n_blocks) return;
+  emit_block_chunks<DIM>(A, b, b + 1 < A.n_blocks ? A.bcount[b + 1] : A.counts[2]);
 }
 
 // ---- chunk list (after every cell rebuild) ----------------------------------
@@ -307,20 +316,31 @@ void stage_grids(const DevParams& P, int n_cu, StageGrids* g) {
   g->global = grid(bg);
 }
 
+// 2D blocks of more rows than a wave holds at once get a wide workgroup where
+// they are too few to fill the chip.  The whole list, a wave and a wide
+// workgroup per block: 131,030 particles (92 blocks of 273 rows) 26 and 17 us,
+// 2.0M (366 of 1,090) 69 and 24, 8.0M (732 of 2,180) 128 and 43.  Thousands of
+// blocks fill it with a wave each.
+constexpr uint32_t kWideBlocks = 1024;
+constexpr int kWaveRows = 256;
+
 void launch_build_chunks(hipStream_t s, const StageArgs& a, uint32_t* block_tot,
                          const uint32_t* ctl) {
   if (a.n_cols == 0) return;
   if (a.lds_cap > 0) {
-    if (a.P.dim == 2) {
-      k_block_chunks<2><<<a.n_blocks, 64, 0, s>>>(a, 0, ctl);
+    const uint32_t ne = (a.n_blocks + kEmitBlocks - 1) / kEmitBlocks;
+    if (a.P.dim == 3) {
+      k_block_chunks<3, 256, 1024><<<a.n_blocks, 256, 0, s>>>(a, ctl);
+    } else if (a.block_rows > kWaveRows && a.n_blocks <= kWideBlocks) {
+      k_block_chunks<2, 1024, 2048><<<a.n_blocks, 1024, 0, s>>>(a, ctl);
     } else {
-      k_block_chunks<3><<<a.n_blocks, 64, 0, s>>>(a, 0, ctl);
+      k_block_chunks<2, 64, kWaveRows><<<a.n_blocks, 64, 0, s>>>(a, ctl);
     }
     k_chunk_base<<<1, kScanBlock, 0, s>>>(a.bcount, a.n_blocks, a.counts + 2, ctl);
     if (a.P.dim == 2) {
-      k_block_chunks<2><<<a.n_blocks, 64, 0, s>>>(a, 1, ctl);
+      k_block_emit<2><<<ne, 64 * kEmitBlocks, 0, s>>>(a, ctl);
     } else {
-      k_block_chunks<3><<<a.n_blocks, 64, 0, s>>>(a, 1, ctl);
+      k_block_emit<3><<<ne, 64 * kEmitBlocks, 0, s>>>(a, ctl);
     }
   } else {
     const uint32_t nb = (a.n_cols + kColsPerBlock - 1) / kColsPerBlock;
