@@ -592,6 +592,40 @@ def test_download_pieces(n):
     ctx.close()
 
 
+@pytest.mark.parametrize("dim,speed,form", [(2, 0.0, "rebuild_small"), (2, 25.0, "cell_keys"),
+                                            (3, 25.0, "cell_keys")])
+def test_rebuild_form_follows_the_rate(dim, speed, form):
+    """Some 14,000 particles: near rest the single-launch rebuild stays; where
+    nearly every step rebuilds, the chain of launches takes over after the
+    first steps.  The bits are those of steps taken one by one (whose choice
+    comes at other steps)."""
+    dr = 0.013 if dim == 2 else 0.075
+    pa = ta.dam_break(dim, dr, [3.22, 2.4, 0.475][:dim], [1.0, 2.0, 0.4][:dim])
+    assert 12000 < pa.n <= 16384
+    n = pa.n_fluid
+    pa.v = np.zeros_like(pa.r)
+    pa.v[:n, 0] = speed * pa.r[:n, 1] / 2.0
+    eq = ta.cfg_equations(dim, dr, 2.0, h_factor=2.0 if dim == 2 else 1.3)
+    a, b = _ctx(eq, [pa]), _ctx(eq, [pa])
+    a.step(150)
+    for _ in range(75):
+        b.step(2)
+    rate = a.counts()[1] / 150
+    assert rate < 0.1 if speed == 0.0 else rate > 0.8
+    a.set_profiling(True)
+    a.step(2)
+    stats = a.kernel_stats()
+    a.set_profiling(False)
+    assert form in stats and not {"rebuild_small", "cell_keys"} <= set(stats)
+    b.step(2)
+    x, y = a.download(), b.download()
+    for f in ("r", "v", "rho"):
+        assert np.array_equal(x[f], y[f]), f
+    assert a.counts() == b.counts()
+    a.close()
+    b.close()
+
+
 def test_empty_upload_rejected():
     eq = _eq(2, 0.02)
     ctx = ta.HipContext(eq)

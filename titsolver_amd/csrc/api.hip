@@ -260,6 +260,29 @@ RebuildCtl rebuild_ctl(tit_hip_ctx* c) {
   return RebuildCtl{c->rebuild_ctl, c->tank_need, c->rebuild_count};
 }
 
+// Whether the single-launch rebuild can serve the set; the rebuilds per step
+// at which the chain of launches is as fast (sph_kernels.hpp).
+bool small_set(const tit_hip_ctx* c) { return c->n <= kSmallN && c->n_cells <= kSmallCells; }
+double even_rebuild_rate(const tit_hip_ctx* c) {
+  return kSmallIdle / std::max(small_cost(c->prm.dim, c->n), 1.0);
+}
+
+// After `steps` plain steps and `rebuilds` rebuilds in all: the form of the
+// next steps' rebuild, from the rate of the last kRateSteps steps or more.
+// Both give the same bits.
+constexpr int kRateSteps = 64;
+void choose_rebuild(tit_hip_ctx* c, int steps, uint64_t rebuilds) {
+  c->rate_steps += static_cast<uint64_t>(steps);
+  c->rate_rebuilds += rebuilds - c->rebuilds_seen;
+  c->rebuilds_seen = rebuilds;
+  if (c->rate_steps < kRateSteps) return;
+  const double rate = static_cast<double>(c->rate_rebuilds) / static_cast<double>(c->rate_steps);
+  const double even = even_rebuild_rate(c);
+  if (rate > 1.1 * even) c->chain_rebuild = true;
+  if (rate < 0.9 * even) c->chain_rebuild = false;
+  c->rate_steps = c->rate_rebuilds = 0;
+}
+
 // Cell rebuild: keys -> stable radix sort -> permute into T and copy back ->
 // cell offsets -> chunk list.  Buffers keep their roles; on the device the
 // whole sequence runs only for the tanks marked before it (by step_begin,
@@ -270,7 +293,7 @@ void enqueue_rebuild(tit_hip_ctx* c, RebuildMode mode) {
   const RebuildCtl rc = rebuild_ctl(c);
   if (mode == kRebuildForce) launch_force_rebuild(s, c->n_tanks, rc);
   if (mode == kRebuildPending) launch_pending_rebuild(s, c->n_tanks, rc);
-  if (c->n <= kSmallN && c->n_cells <= kSmallCells) {
+  if (small_set(c) && !c->chain_rebuild) {
     SmallRebuildArgs a{};
     a.n = c->n;
     a.n_cells = c->n_cells;
@@ -618,11 +641,13 @@ tit_status check_launch(tit_hip_ctx* c, const char* what) {
   return TIT_OK;
 }
 
-tit_status read_flags(tit_hip_ctx* c) {
-  uint32_t flags = 0;
-  TIT_HIP_TRY(c, hipMemcpyAsync(&flags, c->counter + 1, sizeof(uint32_t),
+tit_status read_flags(tit_hip_ctx* c, uint64_t* rebuilds) {
+  uint32_t counter[kCounters] = {};
+  TIT_HIP_TRY(c, hipMemcpyAsync(counter, c->counter, sizeof(counter),
                                 hipMemcpyDeviceToHost, c->stream));
   TIT_HIP_TRY(c, hipStreamSynchronize(c->stream));
+  const uint32_t flags = counter[1];
+  if (rebuilds) std::memcpy(rebuilds, counter + kRebuildCount, sizeof(uint64_t));
   if (flags & 2u) {
     return fail(c, TIT_E_NUMERIC, "non-finite particle position");
   }
@@ -697,12 +722,13 @@ TuneKey tune_key(const tit_hip_ctx* c) {
 namespace tit_amd {
 
 // n_steps plain SSPRK steps: pairs of steps replay the two-step graph of the
-// current rebuild parity (captured on first use), an odd remainder runs
+// current rebuild form (captured on first use), an odd remainder runs
 // eagerly.  Synchronises and checks the device flags.
 tit_status run_plain(tit_hip_ctx* c, int n_steps) {
   int done = 0;
   if (!c->prof.enabled && n_steps >= 2) {
-    const int par = 0;  // buffers keep their roles: one graph serves every step
+    // buffers keep their roles: one graph (of each rebuild form) serves every step
+    const int par = c->chain_rebuild ? 1 : 0;
     if (!c->graph[par]) {
       TIT_HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       enqueue_step(c);
@@ -723,7 +749,10 @@ tit_status run_plain(tit_hip_ctx* c, int n_steps) {
   tit_status st = check_launch(c, "step");
   if (st != TIT_OK) return st;
   if (c->prof.enabled) c->prof.collect();
-  return read_flags(c);
+  uint64_t rebuilds = 0;
+  st = read_flags(c, &rebuilds);
+  if (st == TIT_OK && small_set(c)) choose_rebuild(c, n_steps, rebuilds);
+  return st;
 }
 
 }  // namespace tit_amd
@@ -1009,11 +1038,11 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   TIT_HIP_TRY(c, dalloc(c, &c->cell_n_gaps, 1));
   TIT_HIP_TRY(c, dalloc(c, &c->fixed_list, std::max<uint32_t>(c->n_fixed, 1)));
   TIT_HIP_TRY(c, dalloc(c, &c->fixed_active, std::max<uint32_t>(c->n_fixed, 1)));
-  TIT_HIP_TRY(c, dalloc(c, &c->counter, 4));
+  TIT_HIP_TRY(c, dalloc(c, &c->counter, kCounters));
+  c->rebuild_count = reinterpret_cast<unsigned long long*>(c->counter + kRebuildCount);
   TIT_HIP_TRY(c, dalloc(c, &c->rebuild_ctl, 4));
   TIT_HIP_TRY(c, dalloc(c, &c->tank_need, n_tanks));
   TIT_HIP_TRY(c, dalloc(c, &c->work, kWorkSets * kWorkSet));
-  TIT_HIP_TRY(c, dalloc(c, &c->rebuild_count, 1));
   c->sort.max_tiles = radix_sort_tiles(n);
   TIT_HIP_TRY(c, dalloc(c, &c->sort.hist, 2048ull * std::max<uint32_t>(c->sort.max_tiles, 1)));
   TIT_HIP_TRY(c, dalloc(c, &c->sort.tot, 2048));
@@ -1152,6 +1181,8 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   c->bchunk_cap = 0;
   c->n_cols = 0;
   c->chunk_cap = 0;
+  c->chain_rebuild = false;
+  c->rate_steps = c->rate_rebuilds = c->rebuilds_seen = 0;
   c->lds_cap = stage_lds_capacity(dim);
   st = build_schedule(c);
   if (st != TIT_OK) return st;
@@ -1165,8 +1196,15 @@ tit_status tit_hip_step(tit_hip_ctx* c, int n_steps, double* dt_last) {
   if (!c->uploaded) return fail(c, TIT_E_STATE, "step before upload");
   if (n_steps < 0) return fail(c, TIT_E_ARG, "negative step count");
   TIT_HIP_TRY(c, hipSetDevice(c->device));
-  tit_status st = run_plain(c, n_steps);
-  if (st != TIT_OK) return st;
+  // (in blocks where either rebuild form could serve the steps)
+  const bool both = small_set(c) && even_rebuild_rate(c) < 1.0;
+  int done = 0;
+  do {
+    const int k = both ? std::min(n_steps - done, 2 * kRateSteps) : n_steps - done;
+    const tit_status st = run_plain(c, k);
+    if (st != TIT_OK) return st;
+    done += k;
+  } while (done < n_steps);
   if (dt_last) {
     TIT_HIP_TRY(c, hipMemcpy(dt_last, c->dt, sizeof(double), hipMemcpyDeviceToHost));
   }
@@ -1633,6 +1671,7 @@ tit_status tit_hip_autotune(tit_hip_ctx* c, int steps_per_candidate,
       if (cap > 0 && quad_set(c) && ch != kChunkMax / 4) continue;
       c->chunk_targets = ch;
       c->lds_cap = cap;
+      c->rate_steps = c->rate_rebuilds = 0;  // no other rebuild form between the two runs
       st = build_schedule(c);
       if (st == TIT_OK) st = run_plain(c, 2);  // captures this parity's graph
       if (st != TIT_OK) break;

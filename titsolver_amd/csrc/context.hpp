@@ -45,11 +45,17 @@ struct tit_hip_ctx {
   uint32_t* cell_off = nullptr;
   uint32_t* fixed_list = nullptr;
   uint32_t* fixed_active = nullptr;  // fixed particles with fluid in their stencil
-  uint32_t* counter = nullptr;  // [0] fixed count, [1] flags, [2] fixed_active count
+  // [0] fixed count, [1] flags, [2] fixed_active count; rebuild_count is in it
+  // too, from kRebuildCount on
+  uint32_t* counter = nullptr;
   uint32_t* rebuild_ctl = nullptr;       // RebuildCtl::ctl
   uint32_t* work = nullptr;              // chunk-queue counters (kWorkSets sets)
   uint32_t* tank_need = nullptr;         // RebuildCtl::need
   unsigned long long* rebuild_count = nullptr;
+  // a small set's rebuild as the chain of launches, and the steps and rebuilds
+  // that the choice rests on (choose_rebuild)
+  bool chain_rebuild = false;
+  uint64_t rate_steps = 0, rate_rebuilds = 0, rebuilds_seen = 0;
   SortScratch sort;
   DevTank* tanks = nullptr;
   double* normal = nullptr;
@@ -115,8 +121,7 @@ struct tit_hip_ctx {
   int n_cu = 0;
   double occupancy = 1.0;  // mean particles per occupied cell at upload
 
-  // graphs of two steps, one per rebuild parity (every rebuild swaps the
-  // state, key and id/tag pointers)
+  // graphs of two steps, by the rebuild form (chain_rebuild)
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   hipGraph_t graph_def[2] = {nullptr, nullptr};
 
@@ -169,7 +174,7 @@ BoundaryArgs boundary_args(tit_hip_ctx* c, const DevState& st);
 void enqueue_step(tit_hip_ctx* c);
 void enqueue_post_integrate(tit_hip_ctx* c);
 tit_status check_launch(tit_hip_ctx* c, const char* what);
-tit_status read_flags(tit_hip_ctx* c);
+tit_status read_flags(tit_hip_ctx* c, uint64_t* rebuilds = nullptr);
 // n_steps plain SSPRK steps (graph replay where possible); synchronises.
 tit_status run_plain(tit_hip_ctx* c, int n_steps);
 hipError_t alloc_state(tit_hip_ctx* c, DevState& s, uint32_t n, int dim);

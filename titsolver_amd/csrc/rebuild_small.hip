@@ -7,8 +7,9 @@
 // returns at once, 40 us of a 150 us step at 5,000 particles.  One workgroup
 // of 16 waves does the whole sequence for up to kSmallN particles and
 // kSmallCells cells, with the keys sorted in LDS (key and source slot packed
-// in 32 bits).  Beyond that one CU's latency costs more per rebuild than the
-// launches saved over the steps between rebuilds (sph_kernels.hpp has the figures).
+// in 32 bits).  One CU's latency costs more per rebuild than the chain's:
+// beyond that, and where many steps rebuild, the chain runs (sph_kernels.hpp
+// has the figures).
 //
 // Same results as the large form: the same keys, a stable sort by cell, the
 // same offsets, lists (in another order where the order is irrelevant) and

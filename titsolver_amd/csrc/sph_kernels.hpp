@@ -181,13 +181,25 @@ struct RebuildCtl {
 
 // Rebuild of a small set in one launch (rebuild_small.hip): at most kSmallN
 // particles in kSmallCells cells.  Its arrays are those of the large form's
-// kernels; it also resets the displacements.  A full rebuild of 1,865, 6,215,
-// 14,735 and 26,278 particles takes 42, 101, 189 and 298 us in one workgroup,
-// some 100 us in the chain, whose launches cost 40 us of every step without a
-// rebuild: at 16,384 particles one launch wins up to 3 rebuilds in 10 steps
-// (2 to 10 in 100 on dam breaks), at 26,000 up to 2.
+// kernels; it also resets the displacements.  Between the two forms the rate
+// of rebuilds decides: a step without one costs kSmallIdle us less here (the
+// chain's launches), one with it small_cost(n) us more (a single workgroup).
+// us per step, one launch and the chain, at 0, 0.25, 0.57 and 1 rebuilds a
+// step: 2D 6,218 particles 83, 101, 126, 160 and 107, 119, 135, 156; 8,851 84,
+// 109, 141, 186 and 109, 122, 138, 160; 13,727 90, 126, 171, 235 and 114, 128,
+// 144, 167; 3D at 0 and 1: 3,759 particles 269, 369 and 294, 325; 9,488 268,
+// 504 and 295, 336; 14,199 286, 647 and 314, 362.  Near rest 2 to 10 steps in
+// 100 rebuild, a developed dam break's 50 to 60; beyond kSmallN the chain wins
+// from 0.2 (3D: 0.08) on.
 constexpr uint32_t kSmallN = 16384;
 constexpr uint32_t kSmallCells = 65536;
+constexpr double kSmallIdle = 25.0;
+constexpr double small_cost(int dim, double n) {
+  return dim == 2 ? 0.0087 * n - 26.0 : 0.0232 * n - 17.0;
+}
+
+// Entries of the device counters, and where the rebuild count is (8 bytes).
+constexpr int kCounters = 8, kRebuildCount = 4;
 
 // Particles up to which the 2D tiles give each target four lanes.  One and
 // four lanes, us per launch between events: 1,295 and 6,215 particles 24.5 and
