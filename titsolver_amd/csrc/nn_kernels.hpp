@@ -68,12 +68,14 @@ void fill_f32(hipStream_t s, size_t n, float* p, float value);
 
 // ---- dense layers of the training (nn_train.hip) -----------------------------
 // out = act(A . B + bias), A M x K row-major BF16, B = W (K x N row-major) or,
-// with trans, the transpose of the row-major N x K matrix W; K and N are the
-// network's layer sizes.  pre (M x N): the value before the activation;
-// group16: BF16 sums of every eight rows of the output.  With bpre (M x N):
+// with trans, the transpose of the row-major N x K matrix W.  K and N are the
+// network's layer sizes: nn_train.hip instantiates them, another pair does not
+// link.  pre (M x N): the value before the activation;
+// group16: BF16 sums of every kGroupRows rows of the output.  With bpre (M x N):
 // out16 = (A . B) act'(bpre), colsum[n] += its column sums; out16 may be A.
+constexpr int kGroupRows = 8;
 struct DenseArgs {
-  int M = 0, N = 0;
+  int M = 0;
   const bf16* A = nullptr;
   int lda = 0;
   const bf16* W = nullptr;
@@ -91,17 +93,19 @@ struct DenseArgs {
   const float* bpre = nullptr;
   float* colsum = nullptr;
 };
-void dense(hipStream_t s, int K, const DenseArgs& g);
+template <int K, int N>
+void dense(hipStream_t s, const DenseArgs& g);
 // d16[m][n] = dy[m / group][n] act'(pre[m][n]) (M x N), colsum[n] += its
 // column sums.
-void edge_grad(hipStream_t s, int M, int N, const float* dy, int ld_dy, int group,
-               const float* pre, bf16* d16, float* colsum);
+template <int N>
+void edge_grad(hipStream_t s, int M, const float* dy, int ld_dy, int group, const float* pre,
+               bf16* d16, float* colsum);
 // Partial products X^T dY (X: K x M, dY: K x N, BF16 row-major) over
 // wgrad_slices(K) row slices, M x N each; wgrad_sum adds every listed
 // matrix's slices to its place in the gradient.
 int wgrad_slices(size_t K);
-void wgrad_part(hipStream_t s, int M, int N, size_t K, const bf16* X, const bf16* dY,
-                float* part);
+template <int M, int N>
+void wgrad_part(hipStream_t s, size_t K, const bf16* X, const bf16* dY, float* part);
 struct WgradTable {
   static constexpr int kMax = 10;
   int n = 0;

@@ -39,8 +39,9 @@ __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
 // rows at a time; fragment layouts as in nn_kernels.hip: A[m = l % 32]
 // [k = 8 (l / 32) + i], B[k][n = l % 32], C[m = 8 j + 4 (l / 32) + i][n] in
 // accumulator element 4 j + i.
-template <int KS, int NB>
+template <int KS, int N>
 __global__ __launch_bounds__(NT) void k_dense(DenseArgs g) {
+  constexpr int NB = (N + 31) / 32;
   __shared__ __attribute__((aligned(16))) bf16 s_w[NB * KS * kFrag];
   __shared__ float s_sum[kWaves][NB * 32];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -49,7 +50,7 @@ __global__ __launch_bounds__(NT) void k_dense(DenseArgs g) {
     const int f = u >> 6, l = u & 63;
     const int n = 32 * (f / KS) + (l & 31), k = 16 * (f % KS) + 8 * (l >> 5);
     bf16x8 v = {};
-    if (n < g.N) {
+    if (n < N) {
       if (g.trans) {
         v = ld8(g.W + static_cast<size_t>(n) * g.ldw + k);
       } else {
@@ -76,14 +77,14 @@ __global__ __launch_bounds__(NT) void k_dense(DenseArgs g) {
       f32x16 acc = {};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) acc = mfma(a[ks], ld8(s_w + ((nb * KS + ks) * 64 + lane) * 8), acc);
-      const bool in_n = n < g.N;
+      const bool in_n = n < N;
       const float bias = g.bias && in_n ? g.bias[n] : 0.0f;
       if (g.bpre) {  // the gradient through the activation, its column sums
         float pre[16];  // all loads in flight together
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int m = min(m0 + 8 * (e >> 2) + 4 * h + (e & 3), g.M - 1);
-          pre[e] = g.bpre[static_cast<size_t>(m) * g.N + (in_n ? n : 0)];
+          pre[e] = g.bpre[static_cast<size_t>(m) * N + (in_n ? n : 0)];
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -104,13 +105,14 @@ __global__ __launch_bounds__(NT) void k_dense(DenseArgs g) {
           const float x = g.bias ? acc[4 * j + i] + bias : acc[4 * j + i];
           y[i] = g.act == kActHswish ? nn_act(x) : x;
           if (m >= g.M || !in_n) continue;
-          if (g.pre) g.pre[static_cast<size_t>(m) * g.N + n] = x;
+          if (g.pre) g.pre[static_cast<size_t>(m) * N + n] = x;
           if (g.out32) g.out32[static_cast<size_t>(m) * g.ldo32 + n] = y[i];
           if (g.out16) g.out16[static_cast<size_t>(m) * g.ldo16 + n] = static_cast<bf16>(y[i]);
         }
         if (g.group16) {
           // the sum of eight rows (an edge group), in row order: the lower
           // half's four, then the upper half's
+          static_assert(kGroupRows == 8, "four rows of each half");
           float s = 0.0f;
           if (h == 0) s = ((s + y[0]) + y[1]) + y[2] + y[3];
           s = __shfl(s, col);
@@ -130,7 +132,7 @@ __global__ __launch_bounds__(NT) void k_dense(DenseArgs g) {
       if (h == 0) s_sum[wave][32 * nb + col] = s;
     }
     __syncthreads();
-    for (int n = tid; n < g.N; n += NT) {
+    for (int n = tid; n < N; n += NT) {
       float s = 0.0f;
       for (int w = 0; w < kWaves; ++w) s += s_sum[w][n];
       atomicAdd(g.colsum + n, s);
@@ -138,20 +140,13 @@ __global__ __launch_bounds__(NT) void k_dense(DenseArgs g) {
   }
 }
 
-template <int KS, int NB>
-void run_dense(hipStream_t s, const DenseArgs& g) {
-  // four workgroups per CU (LDS and registers) at most, two where each ends
-  // with an atomic per column (11.5 ns each on one address)
-  const int wgs = (g.M + 32 * kWaves - 1) / (32 * kWaves);
-  k_dense<KS, NB><<<std::min(wgs, g.colsum ? 512 : 1024), NT, 0, s>>>(g);
-}
-
 // d = dy act'(pre) for edge rows whose upstream row is shared by `group` of
 // them; BF16, and its column sums.  A thread keeps its column.
 constexpr int kEdgeRows = 256;
-__global__ __launch_bounds__(NT) void k_edge_grad(int M, int N, const float* dy, int ld_dy,
-                                                  int group, const float* pre, bf16* d16,
-                                                  float* colsum) {
+template <int N>
+__global__ __launch_bounds__(NT) void k_edge_grad(int M, const float* dy, int ld_dy, int group,
+                                                  const float* pre, bf16* d16, float* colsum) {
+  static_assert(NT % N == 0, "a thread keeps its column");
   __shared__ float s_sum[NT];
   const int n = threadIdx.x % N, r0 = threadIdx.x / N, step = NT / N;
   float sum = 0.0f;
@@ -206,9 +201,12 @@ __device__ __forceinline__ void put_transposed(bf16* tile, const bf16* src, int 
 // dW[32 MB x 32 NB] of rows [beg, end) of X (M columns) and dY (N columns)
 // into this slice's partial (row-major M x N).  NB == 4: wave w takes output
 // columns 32 w ..; NB == 1: wave w takes output rows 32 w .. .
-template <int MB, int NB>
-__global__ __launch_bounds__(NT) void k_wgrad(int M, int N, int K, const bf16* X, const bf16* dY,
+template <int M, int N>
+__global__ __launch_bounds__(NT) void k_wgrad(int K, const bf16* X, const bf16* dY,
                                               int slice_rows, float* part) {
+  constexpr int MB = (M + 31) / 32, NB = (N + 31) / 32;
+  static_assert(M % 8 == 0 && N % 8 == 0 && (NB == kWaves || (NB == 1 && MB <= kWaves)),
+                "the waves cover the output");
   __shared__ __attribute__((aligned(16))) bf16 sX[32 * MB * kRowPad];
   __shared__ __attribute__((aligned(16))) bf16 sY[32 * NB * kRowPad];
   constexpr int BM = NB == 1 ? 1 : MB;  // output blocks of a wave
@@ -221,7 +219,7 @@ __global__ __launch_bounds__(NT) void k_wgrad(int M, int N, int K, const bf16* X
   f32x16 acc[BM];
 #pragma unroll
   for (int b = 0; b < BM; ++b) acc[b] = f32x16{};
-  const int cx = M / 8, cy = N / 8;
+  constexpr int cx = M / 8, cy = N / 8;
   for (int k0 = beg; k0 < end; k0 += kRows) {
     __syncthreads();
     for (int u = tid; u < (cx + cy) * 8; u += NT) {
@@ -280,53 +278,49 @@ __global__ __launch_bounds__(NT) void k_wgrad_sum(WgradTable t, float* g) {
 
 }  // namespace
 
-void dense(hipStream_t s, int K, const DenseArgs& g) {
+// The waves' row tiles: four workgroups per CU at most (three fit the LDS of
+// the widest layers, whose weights take 40 KB), two where each ends with an
+// atomic per column (11.5 ns each on one address).
+template <int K, int N>
+void dense(hipStream_t s, const DenseArgs& g) {
+  static_assert(K % 16 == 0, "whole MFMA steps");
   if (g.M <= 0) return;
-  const int nb = (g.N + 31) / 32;
-  if (K == 80 && nb == 4) {
-    run_dense<5, 4>(s, g);
-  } else if (K == 128 && nb == 4) {
-    run_dense<8, 4>(s, g);
-  } else if (K == 160 && nb == 4) {
-    run_dense<10, 4>(s, g);
-  } else if (K == 128 && nb == 1) {
-    run_dense<8, 1>(s, g);
-  } else if (K == 16 && nb == 4) {
-    run_dense<1, 4>(s, g);
-  } else if (K == 128 && nb == 5) {
-    run_dense<8, 5>(s, g);
-  } else if (K == 128 && nb == 3) {
-    run_dense<8, 3>(s, g);
-  }
+  const int wgs = (g.M + 32 * kWaves - 1) / (32 * kWaves);
+  k_dense<K / 16, N><<<std::min(wgs, g.colsum ? 512 : 1024), NT, 0, s>>>(g);
 }
+template void dense<80, 128>(hipStream_t, const DenseArgs&);
+template void dense<128, 128>(hipStream_t, const DenseArgs&);
+template void dense<160, 128>(hipStream_t, const DenseArgs&);
+template void dense<128, 16>(hipStream_t, const DenseArgs&);
+template void dense<16, 128>(hipStream_t, const DenseArgs&);
+template void dense<128, 160>(hipStream_t, const DenseArgs&);
+template void dense<128, 80>(hipStream_t, const DenseArgs&);
 
-void edge_grad(hipStream_t s, int M, int N, const float* dy, int ld_dy, int group,
-               const float* pre, bf16* d16, float* colsum) {
+template <int N>
+void edge_grad(hipStream_t s, int M, const float* dy, int ld_dy, int group, const float* pre,
+               bf16* d16, float* colsum) {
   if (M <= 0) return;
-  k_edge_grad<<<(M + kEdgeRows - 1) / kEdgeRows, NT, 0, s>>>(M, N, dy, ld_dy, group, pre, d16,
-                                                            colsum);
+  k_edge_grad<N><<<(M + kEdgeRows - 1) / kEdgeRows, NT, 0, s>>>(M, dy, ld_dy, group, pre, d16,
+                                                               colsum);
 }
+template void edge_grad<128>(hipStream_t, int, const float*, int, int, const float*, bf16*,
+                             float*);
 
 int wgrad_slices(size_t K) {
   return static_cast<int>(std::clamp<size_t>((K + kRows - 1) / kRows, 1, 256));
 }
 
-void wgrad_part(hipStream_t s, int M, int N, size_t K, const bf16* X, const bf16* dY,
-                float* part) {
+template <int M, int N>
+void wgrad_part(hipStream_t s, size_t K, const bf16* X, const bf16* dY, float* part) {
   const int slices = wgrad_slices(K);
   // whole steps per slice; the last slices may be empty (their partial is 0)
   const int per = static_cast<int>((K + slices - 1) / slices + kRows - 1) / kRows * kRows;
-  const int k = static_cast<int>(K);
-  if (M == 80) {
-    k_wgrad<3, 4><<<slices, NT, 0, s>>>(M, N, k, X, dY, per, part);
-  } else if (M == 160) {
-    k_wgrad<5, 4><<<slices, NT, 0, s>>>(M, N, k, X, dY, per, part);
-  } else if (N == 16) {
-    k_wgrad<4, 1><<<slices, NT, 0, s>>>(M, N, k, X, dY, per, part);
-  } else {
-    k_wgrad<4, 4><<<slices, NT, 0, s>>>(M, N, k, X, dY, per, part);
-  }
+  k_wgrad<M, N><<<slices, NT, 0, s>>>(static_cast<int>(K), X, dY, per, part);
 }
+template void wgrad_part<80, 128>(hipStream_t, size_t, const bf16*, const bf16*, float*);
+template void wgrad_part<128, 128>(hipStream_t, size_t, const bf16*, const bf16*, float*);
+template void wgrad_part<160, 128>(hipStream_t, size_t, const bf16*, const bf16*, float*);
+template void wgrad_part<128, 16>(hipStream_t, size_t, const bf16*, const bf16*, float*);
 
 void wgrad_sum(hipStream_t s, WgradTable& t, float* g) {
   uint32_t blocks = 0;

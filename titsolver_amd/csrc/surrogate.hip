@@ -722,7 +722,6 @@ void forward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
   auto layer = [&](int M, int N, const bf16* in, int lda, int w, int bias, int act) {
     DenseArgs g{};
     g.M = M;
-    g.N = N;
     g.A = in;
     g.lda = lda;
     g.W = W.w16 + w;
@@ -736,14 +735,14 @@ void forward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
   g.pre = A.training ? A.pre1[r] : nullptr;
   g.out16 = A.a1[r];
   g.ldo16 = kHidden;
-  dense(s, kEdgeIn, g);
+  dense<kEdgeIn, kHidden>(s, g);
   // messages, summed over each node's edges: y = [H | sum]
   g = layer(me, kHidden, A.a1[r], kHidden, RoundLayout::W2, RoundLayout::b2, kActHswish);
   g.pre = A.training ? A.pre2[r] : nullptr;
   g.group16 = A.Y[r];
   g.ldg = kNodeCat;
   g.colg = kNodeIn;
-  dense(s, kHidden, g);
+  dense<kHidden, kHidden>(s, g);
   k_copy_bf16_cols<<<nblk(static_cast<size_t>(n) * (kNodeIn / 8)), kBlk, 0, s>>>(
       n, kNodeIn, A.H[r], kNodeIn, A.Y[r], kNodeCat, 0);
   // node layers
@@ -751,12 +750,12 @@ void forward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
   g.pre = A.training ? A.pre3[r] : nullptr;
   g.out16 = A.a3[r];
   g.ldo16 = kHidden;
-  dense(s, kNodeCat, g);
+  dense<kNodeCat, kHidden>(s, g);
   g = layer(m, kHidden, A.a3[r], kHidden, RoundLayout::W4, RoundLayout::b4, kActHswish);
   g.pre = A.training ? A.pre4[r] : nullptr;
   g.out16 = A.a4[r];
   g.ldo16 = kHidden;
-  dense(s, kHidden, g);
+  dense<kHidden, kHidden>(s, g);
   g = layer(m, kOut, A.a4[r], kHidden, RoundLayout::W5, RoundLayout::b5, kActNone);
   g.out32 = A.u[r];
   g.ldo32 = kOut;
@@ -766,7 +765,7 @@ void forward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n,
     g.out16 = A.H[r + 1] + kNodeFeat;
     g.ldo16 = kNodeIn;
   }
-  dense(s, kHidden, g);
+  dense<kHidden, kOut>(s, g);
 }
 
 // Backward of round r from A.du (n x kOut FP32).  For r > 0 leaves the
@@ -777,10 +776,12 @@ void backward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n
   const size_t E = static_cast<size_t>(n) * kKnn;
   const RoundW W = round_w(L, r);
   float* g = W.g;
-  auto wgrad = [&](int M, int N, size_t K, const bf16* X, const bf16* dY, int dst) {
+  static_assert(kKnn == kGroupRows, "a node's edges are one row group");
+  static_assert(5 * kRounds <= WgradTable::kMax, "every weight matrix of the network");
+  auto wgrad = [&]<int M, int N>(size_t K, const bf16* X, const bf16* dY, int dst) {
     float* part = A.part + static_cast<size_t>(wgrad_slices(E)) *
                                (static_cast<size_t>(r) * RoundLayout::size + dst);
-    wgrad_part(s, M, N, K, X, dY, part);
+    wgrad_part<M, N>(s, K, X, dY, part);
     wt.part[wt.n] = part;
     wt.slices[wt.n] = wgrad_slices(K);
     wt.size[wt.n] = static_cast<uint32_t>(M * N);
@@ -788,10 +789,9 @@ void backward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n
     ++wt.n;
   };
   // dX = dY W^T; with bpre through the activation that made X, into BF16
-  auto dgrad = [&](int M, int K, int N, const bf16* dY, int w) {
+  auto dgrad = [&](int M, int K, const bf16* dY, int w) {
     DenseArgs d{};
     d.M = M;
-    d.N = N;
     d.A = dY;
     d.lda = K;
     d.W = W.w16 + w;
@@ -804,44 +804,44 @@ void backward_round(hipStream_t s, Learned* L, Activations& A, int r, uint32_t n
   k_to_bf16<<<nblk(static_cast<size_t>(n) * kOut), kBlk, 0, s>>>(
       static_cast<size_t>(n) * kOut, A.du, A.du16);
   column_sum(s, m, kOut, A.du, g + RoundLayout::b5);
-  wgrad(kHidden, kOut, n, A.a4[r], A.du16, RoundLayout::W5);
-  DenseArgs d = dgrad(m, kOut, kHidden, A.du16, RoundLayout::W5);
+  wgrad.template operator()<kHidden, kOut>(n, A.a4[r], A.du16, RoundLayout::W5);
+  DenseArgs d = dgrad(m, kOut, A.du16, RoundLayout::W5);
   d.bpre = A.pre4[r];
   d.out16 = A.dN16;
   d.ldo16 = kHidden;
   d.colsum = g + RoundLayout::b4;
-  dense(s, kOut, d);
+  dense<kOut, kHidden>(s, d);
   // node layer 2
-  wgrad(kHidden, kHidden, n, A.a3[r], A.dN16, RoundLayout::W4);
-  d = dgrad(m, kHidden, kHidden, A.dN16, RoundLayout::W4);
+  wgrad.template operator()<kHidden, kHidden>(n, A.a3[r], A.dN16, RoundLayout::W4);
+  d = dgrad(m, kHidden, A.dN16, RoundLayout::W4);
   d.bpre = A.pre3[r];
   d.out16 = A.dN16;
   d.ldo16 = kHidden;
   d.colsum = g + RoundLayout::b3;
-  dense(s, kHidden, d);
+  dense<kHidden, kHidden>(s, d);
   // node layer 1
-  wgrad(kNodeCat, kHidden, n, A.Y[r], A.dN16, RoundLayout::W3);
-  d = dgrad(m, kHidden, kNodeCat, A.dN16, RoundLayout::W3);
+  wgrad.template operator()<kNodeCat, kHidden>(n, A.Y[r], A.dN16, RoundLayout::W3);
+  d = dgrad(m, kHidden, A.dN16, RoundLayout::W3);
   d.out32 = A.dY;
   d.ldo32 = kNodeCat;
-  dense(s, kHidden, d);
+  dense<kHidden, kNodeCat>(s, d);
   // edge layer 2 (message gradient = dY[:, kNodeIn:] broadcast to the edges)
-  edge_grad(s, me, kHidden, A.dY + kNodeIn, kNodeCat, kKnn, A.pre2[r], A.dE16,
+  edge_grad<kHidden>(s, me, A.dY + kNodeIn, kNodeCat, kKnn, A.pre2[r], A.dE16,
             g + RoundLayout::b2);
-  wgrad(kHidden, kHidden, E, A.a1[r], A.dE16, RoundLayout::W2);
-  d = dgrad(me, kHidden, kHidden, A.dE16, RoundLayout::W2);
+  wgrad.template operator()<kHidden, kHidden>(E, A.a1[r], A.dE16, RoundLayout::W2);
+  d = dgrad(me, kHidden, A.dE16, RoundLayout::W2);
   d.bpre = A.pre1[r];
   d.out16 = A.dE16;
   d.ldo16 = kHidden;
   d.colsum = g + RoundLayout::b1;
-  dense(s, kHidden, d);
+  dense<kHidden, kHidden>(s, d);
   // edge layer 1
-  wgrad(kEdgeIn, kHidden, E, A.X[r], A.dE16, RoundLayout::W1);
+  wgrad.template operator()<kEdgeIn, kHidden>(E, A.X[r], A.dE16, RoundLayout::W1);
   if (r > 0) {
-    d = dgrad(me, kHidden, kEdgeIn, A.dE16, RoundLayout::W1);
+    d = dgrad(me, kHidden, A.dE16, RoundLayout::W1);
     d.out32 = A.dX;
     d.ldo32 = kEdgeIn;
-    dense(s, kHidden, d);
+    dense<kHidden, kEdgeIn>(s, d);
     k_latent_grad_gather<<<nblk(static_cast<size_t>(n) * kLatent), kBlk, 0, s>>>(
         n, A.dY, A.dX, du_prev);
     k_latent_grad_scatter<<<nblk(E * kLatent), kBlk, 0, s>>>(n, A.dX, nbr, du_prev);
