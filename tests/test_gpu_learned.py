@@ -236,6 +236,30 @@ def test_run_with_zero_tolerance_is_the_plain_trajectory():
     ref.close()
 
 
+def test_zero_tolerance_run_restores_either_chunk_list():
+    """A rejected group restores the chunk list of the schedule it ran under,
+    column chunks and then tiles, in a flow of 3 m/s that rebuilds the index on
+    the way: the plain trajectory, bit for bit."""
+    pa = ta.dam_break(2, 0.03, [3.22, 2.4], [1.0, 2.0])
+    pa.v = np.zeros_like(pa.r)
+    pa.v[: pa.n_fluid, 0] = 1.5 * pa.r[: pa.n_fluid, 1]
+    eq = ta.cfg_equations(2, 0.03, 2.0)
+    a, b = ta.HipContext(eq), ta.HipContext(eq)
+    a.upload([pa])
+    b.upload([pa])
+    L = ta.LearnedStep(a, seed=2)
+    for capacity in (0, 1024, 0):
+        a.set_schedule(0, capacity)
+        rep = L.run(3, judge_every=3, tol=0.0)
+        assert rep["rejected"] == rep["judged"] == 1
+        b.step(3 * 4)  # (the judge's own four plain steps are undone too)
+    x, y = a.download(), b.download()
+    for k in ("r", "v", "rho"):
+        assert np.array_equal(x[k], y[k]), k
+    a.close()
+    b.close()
+
+
 def test_run_accepting_advances_four_dt_per_step():
     ctx, eq, pa = _dam(steps=10)
     L = ta.LearnedStep(ctx, seed=2)

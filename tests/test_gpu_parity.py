@@ -355,9 +355,7 @@ def test_escaped_particles_keep_exact_sets(dim, n, radius):
 
 def test_gapped_columns_are_cut_and_sum_exact_sets():
     """A tall tank (300 cell rows) with a fluid block at the bottom and a thin
-    layer 2.6 m above it: each column's 140 particles fall into two equal
-    parts of the chunk schedule, the second spanning the gap, which the
-    builder cuts where it passes 92 cells.  Every particle is still summed
+    layer 2.6 m above it, the rows between them empty.  Every particle is still summed
     over exactly its brute-force neighbour set (a lost or doubled piece would
     leave targets with no pairs or twice their pairs)."""
     dr = 0.005

@@ -440,12 +440,10 @@ tit_status build_schedule(tit_hip_ctx* c) {
     }
   }
   if (cols.size() >= (1ull << 31)) return fail(c, TIT_E_ARG, "too many cell columns");
-  // equal parts: n / chunk_targets + one per column at most; cuts by span:
-  // (nz - 1) / kChunkRows per column at most
   int nz_max = 1;
   for (const DevTank& T : c->host_tanks) nz_max = std::max(nz_max, T.nc[dim - 1]);
-  const size_t need = c->n / c->chunk_targets +
-                      cols.size() * (1 + static_cast<size_t>(nz_max - 1) / kChunkRows) + 1;
+  // column chunks: n / chunk_targets + one per column at most
+  const size_t need = c->lds_cap > 0 ? 0 : c->n / c->chunk_targets + cols.size() + 1;
   if (!c->cols || cols.size() != c->n_cols) {
     forget(c, c->cols);
     forget(c, c->block_tot);
@@ -464,7 +462,7 @@ tit_status build_schedule(tit_hip_ctx* c) {
     TIT_HIP_TRY(c, dalloc(c, &c->chunks, need));
     c->chunk_cap = need;
   }
-  if (!c->chunk_counts) TIT_HIP_TRY(c, dalloc(c, &c->chunk_counts, 4));
+  if (!c->chunk_counts) TIT_HIP_TRY(c, dalloc(c, &c->chunk_counts, 2));
   if (!c->blocks) {
     // blocks of kBlk2 columns (2D), kBlk3 x kBlk3 (3D)
     const int bw = dim == 2 ? kBlk2 : kBlk3;
@@ -488,8 +486,10 @@ tit_status build_schedule(tit_hip_ctx* c) {
                              hipMemcpyHostToDevice));
     c->n_blocks = static_cast<uint32_t>(blocks.size());
   }
-  const size_t bneed = block_chunk_bound(dim, c->n, c->n_blocks, static_cast<size_t>(nz_max),
-                                         tile_targets(c), c->lds_cap);
+  const size_t bneed =
+      c->lds_cap == 0 ? 0
+                      : block_chunk_bound(dim, c->n, c->n_blocks, static_cast<size_t>(nz_max),
+                                          tile_targets(c), c->lds_cap);
   if (bneed > c->bchunk_cap) {
     forget(c, c->bchunks);
     c->bchunks = nullptr;

@@ -251,7 +251,7 @@ __global__ __launch_bounds__(NT) void k_rebuild_small(SmallRebuildArgs R) {
     for (uint32_t b = wave; b < A.n_blocks; b += kWaves) {
       emit_block_chunks<DIM>(A, b, b + 1 < A.n_blocks ? A.bcount[b + 1] : before);
     }
-    if (tid == 0) A.counts[2] = before;
+    if (tid == 0) A.counts[1] = before;
   }
   for (int t = tid; t < R.n_tanks; t += NT) {
     if (R.rc.need[t]) R.disp[t] = 0.0;

@@ -9,9 +9,6 @@ namespace tit_amd {
 // 2D schedule may name.
 constexpr int kChunkMax = 128;
 constexpr int kStageLdsCap = 1024;
-// Cells a column chunk's targets span along a column at most: a column's
-// equal parts are cut further where they span more.
-constexpr int kChunkRows = 92;
 // 2D tiles (stage_tile.hip): the cell columns of a tank in blocks of kBlk2; a
 // chunk holds the particles of one block in a range of at most kChunkRows2
 // rows, at most kTileThreads of them, and its window (the block grown by the
@@ -72,14 +69,14 @@ struct StageArgs {
   // chunk schedule: cell columns (tank, ix, iy, first cell) and, rebuilt on
   // the device after every cell rebuild, chunks (column, first particle,
   // end particle) of at most chunk_targets consecutive particles of a column
-  // spanning at most kChunkRows cells
+  // (lds_cap 0 only)
   const uint4* cols;
   uint32_t n_cols;
   uint32_t chunk_targets;
   uint32_t lds_cap;            // candidate positions staged in LDS at most
   bool quad;                   // 2D tiles: four lanes per target
   uint4* chunks;
-  uint32_t* counts;            // [0] column chunks, [2] block chunks
+  uint32_t* counts;            // [0] column chunks, [1] block chunks
   uint32_t grid_tile, grid_global;  // persistent grid sizes
   uint32_t* work;                   // this launch's set of chunk-queue counters
   // with LDS staging (lds_cap > 0): cell-column blocks (tank, first ix,

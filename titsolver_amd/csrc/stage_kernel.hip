@@ -1,14 +1,16 @@
 // Fused SSPRK stage kernel: continuity + momentum pair sums, EOS, update.
 //
 // Two families of work units, both recut on the device after every cell
-// rebuild and walked by a persistent grid in XCD-major bands (launch index b
+// rebuild and taken by a persistent grid in XCD-major bands (launch index b
 // runs on XCD b % 8 and takes chunks from that XCD's eighth of the list, so
 // each XCD's L2 holds a contiguous band of columns):
 //  - block chunks (schedules with LDS): the particles of a block of cell
 //    columns over a few rows, the block's window staged in LDS: the tile
-//    kernels of stage_tile.hip (2D) and stage_tile3.hip (3D);
+//    kernels of stage_tile.hip (2D) and stage_tile3.hip (3D), which draw
+//    chunks from their band's queue and then from the others';
 //  - column chunks (schedules without LDS): at most chunk_targets consecutive
-//    (cell-sorted) particles of one cell column, positions from global memory.
+//    (cell-sorted) particles of one cell column, positions from global memory,
+//    a fixed share of the band for each workgroup.
 // Every path visits a target's candidates in the same order and rounds
 // identically, so all schedules produce the same bits.
 #include "chunk_build.hpp"
@@ -52,7 +54,7 @@ __global__ __launch_bounds__(64 * kEmitBlocks) void k_block_emit(StageArgs A,
   if (!ctl[0]) return;
   const uint32_t b = blockIdx.x * kEmitBlocks + (threadIdx.x >> 6);
   if (b >= A.n_blocks) return;
-  emit_block_chunks<DIM>(A, b, b + 1 < A.n_blocks ? A.bcount[b + 1] : A.counts[2]);
+  emit_block_chunks<DIM>(A, b, b + 1 < A.n_blocks ? A.bcount[b + 1] : A.counts[1]);
 }
 
 // ---- chunk list (after every cell rebuild) ----------------------------------
@@ -60,11 +62,7 @@ __global__ __launch_bounds__(64 * kEmitBlocks) void k_block_emit(StageArgs A,
 constexpr int kScanBlock = 1024;
 
 // The chunks of a column, in order: the column's particles in
-// ceil(n / chunk_targets) equal parts, each cut further into pieces whose
-// targets span at most kChunkRows cells (a piece starting at particle p ends
-// before the first particle with key >= key[p] + kChunkRows).  A column gains
-// at most (nz - 1) / kChunkRows cuts: each cut starts a piece kChunkRows
-// cells or more above the last, and the parts' spans do not overlap.
+// ceil(n / chunk_targets) equal parts.
 struct ColumnParts {
   uint32_t beg, n, nch;
 };
@@ -78,54 +76,6 @@ __device__ __forceinline__ ColumnParts column_parts(const StageArgs& A, uint32_t
   cp.n = A.cell_off[col.w + nz] - cp.beg;
   cp.nch = (cp.n + A.chunk_targets - 1) / A.chunk_targets;
   return cp;
-}
-
-// The pieces of part k of a column: emit(i, p0, p1) for its i-th piece;
-// returns their count.
-template <class F>
-__device__ __forceinline__ uint32_t part_pieces(const StageArgs& A, const ColumnParts& cp,
-                                                uint32_t k, F&& emit) {
-  const uint32_t p0 = cp.beg + static_cast<uint32_t>((static_cast<uint64_t>(cp.n) * k) / cp.nch);
-  const uint32_t p1 =
-      cp.beg + static_cast<uint32_t>((static_cast<uint64_t>(cp.n) * (k + 1)) / cp.nch);
-  uint32_t p = p0, count = 0;
-  while (p < p1) {
-    const uint32_t lim = A.key[p] + static_cast<uint32_t>(kChunkRows);
-    uint32_t q = p1;
-    if (A.key[p1 - 1] >= lim) {
-      // the first particle in (p, p1) with key >= lim (keys ascend)
-      uint32_t lo = p + 1, hi = p1 - 1;
-      while (lo < hi) {
-        const uint32_t mid = lo + (hi - lo) / 2;
-        if (A.key[mid] >= lim) {
-          hi = mid;
-        } else {
-          lo = mid + 1;
-        }
-      }
-      q = lo;
-    }
-    emit(count, p, q);
-    ++count;
-    p = q;
-  }
-  return count;
-}
-
-// Pieces of the column's parts that lane takes (parts lane, lane + 64, ...).
-__device__ __forceinline__ uint32_t lane_pieces(const StageArgs& A, const ColumnParts& cp,
-                                                int lane) {
-  uint32_t cnt = 0;
-  for (uint32_t k = lane; k < cp.nch; k += 64) {
-    cnt += part_pieces(A, cp, k, [](uint32_t, uint32_t, uint32_t) {});
-  }
-  return cnt;
-}
-
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
 }
 
 // Exclusive scan over a 1024-thread block: wave shuffles, then the 16 wave
@@ -157,9 +107,8 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wsum,
   return r;
 }
 
-// Chunk list in column order, in three passes, one wave per column (its
-// lanes take the column's parts in turn): chunks per column and their
-// per-workgroup totals; an exclusive scan of the totals (one workgroup, also
+// Chunk list in column order, in three passes, one wave per column: chunks
+// per workgroup of columns; an exclusive scan of those (one workgroup, also
 // writes the chunk count); each column's chunks at its scanned offset.
 constexpr uint32_t kColsPerBlock = kScanBlock / 64;
 
@@ -169,10 +118,7 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_count(StageArgs A, uint32_
   __shared__ uint32_t wtot[kColsPerBlock];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t c = blockIdx.x * kColsPerBlock + wave;
-  uint32_t cnt = 0;
-  if (c < A.n_cols) cnt = lane_pieces(A, column_parts(A, c), lane);
-  cnt = wave_sum_u32(cnt);
-  if (lane == 0) wtot[wave] = cnt;
+  if (lane == 0) wtot[wave] = c < A.n_cols ? column_parts(A, c).nch : 0u;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint32_t t = 0;
@@ -181,8 +127,7 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_count(StageArgs A, uint32_
   }
 }
 
-// Exclusive scan of n_blocks counts in place (one workgroup); out[0] = the
-// total (chunks), out[1] = 0 (overflow chunks, appended by the stage kernel).
+// Exclusive scan of n_blocks counts in place (one workgroup); *out = the total.
 __global__ __launch_bounds__(kScanBlock) void k_chunk_base(uint32_t* block_tot, uint32_t n_blocks,
                                                           uint32_t* out, const uint32_t* ctl) {
   if (!ctl[0]) return;
@@ -196,10 +141,7 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_base(uint32_t* block_tot, 
     if (b < n_blocks) block_tot[b] = off;
     base_off += tot;
   }
-  if (threadIdx.x == 0) {
-    out[0] = base_off;
-    out[1] = 0;
-  }
+  if (threadIdx.x == 0) *out = base_off;
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_chunk_emit(StageArgs A,
@@ -210,36 +152,16 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_emit(StageArgs A,
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t c = blockIdx.x * kColsPerBlock + wave;
   // the counts again (the offsets need every earlier column's)
-  ColumnParts cp{0u, 0u, 0u};
-  uint32_t cnt = 0;
-  if (c < A.n_cols) {
-    cp = column_parts(A, c);
-    cnt = lane_pieces(A, cp, lane);
-  }
-  cnt = wave_sum_u32(cnt);
-  if (lane == 0) wtot[wave] = cnt;
+  const ColumnParts cp = c < A.n_cols ? column_parts(A, c) : ColumnParts{0u, 0u, 0u};
+  if (lane == 0) wtot[wave] = cp.nch;
   __syncthreads();
-  if (c >= A.n_cols) return;
   uint32_t off = block_tot[blockIdx.x];
   for (int w = 0; w < wave; ++w) off += wtot[w];
-  // parts in rounds of 64, each part's pieces at its exclusive prefix
-  for (uint32_t k0 = 0; k0 < cp.nch; k0 += 64) {
-    const uint32_t k = k0 + static_cast<uint32_t>(lane);
-    const uint32_t np =
-        k < cp.nch ? part_pieces(A, cp, k, [](uint32_t, uint32_t, uint32_t) {}) : 0u;
-    uint32_t x = np;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t y = __shfl_up(x, d);
-      if (lane >= d) x += y;
-    }
-    const uint32_t base = off + x - np;
-    if (k < cp.nch) {
-      (void)part_pieces(A, cp, k, [&](uint32_t i, uint32_t p0, uint32_t p1) {
-        A.chunks[base + i] = make_uint4(c, p0, p1, 0u);
-      });
-    }
-    off += __shfl(x, 63);
+  for (uint32_t k = lane; k < cp.nch; k += 64) {
+    auto part = [&](uint32_t q) {
+      return cp.beg + static_cast<uint32_t>((static_cast<uint64_t>(cp.n) * q) / cp.nch);
+    };
+    A.chunks[off + k] = make_uint4(c, part(k), part(k + 1), 0u);
   }
 }
 
@@ -336,7 +258,7 @@ void launch_build_chunks(hipStream_t s, const StageArgs& a, uint32_t* block_tot,
     } else {
       k_block_chunks<2, 64, kWaveRows><<<a.n_blocks, 64, 0, s>>>(a, ctl);
     }
-    k_chunk_base<<<1, kScanBlock, 0, s>>>(a.bcount, a.n_blocks, a.counts + 2, ctl);
+    k_chunk_base<<<1, kScanBlock, 0, s>>>(a.bcount, a.n_blocks, a.counts + 1, ctl);
     if (a.P.dim == 2) {
       k_block_emit<2><<<ne, 64 * kEmitBlocks, 0, s>>>(a, ctl);
     } else {

@@ -325,7 +325,7 @@ k_stage_tile(StageArgs A) {
   const int tid = threadIdx.x;
   __shared__ uint32_t s_next;
   ChunkQueue queue;
-  queue.init(A.counts[2]);
+  queue.init(A.counts[1]);
   WaveReduce red;
   for (uint32_t q = queue.q; q != ~0u;) {
     const TileChunk c = tile_chunk(A, q);

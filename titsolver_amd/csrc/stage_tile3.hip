@@ -128,7 +128,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   const DevParams& P = A.P;
   const int tid = threadIdx.x;
   ChunkQueue queue;
-  queue.init(A.counts[2]);
+  queue.init(A.counts[1]);
   WaveReduce red;
   for (uint32_t q = queue.q; q != ~0u;) {
     const uint4 ch = A.bchunks[q];
