@@ -204,10 +204,11 @@ def test_rebuild_interleaved_with_hooks():
 @pytest.mark.parametrize("dim", [2, 3])
 def test_schedules_are_bitwise_identical(dim):
     """Any chunk length, and LDS staging on or off, gives the same bits: each
-    target walks its own stencil in the same order on every path.  With a
-    small LDS capacity most chunks overflow to the global-memory kernel (2D:
-    column chunks; 3D: block chunks); capacity 0 is the column-chunk
-    global-memory path."""
+    target walks its own stencil in the same order on every path.  Here a 2D
+    set of four lanes per target, whose chunk lengths from 32 on are one
+    schedule, and a 3D one whose interior windows do not fit the LDS (h = 2
+    spacings); with a small LDS capacity nearly no window fits.  Capacity 0 is
+    the column-chunk path, positions from global memory."""
     dr = 0.02 if dim == 2 else 0.03
     pa = perturbed_dam_break(dim, dr, seed=9)
     eq = _eq(dim, dr)
@@ -225,6 +226,62 @@ def test_schedules_are_bitwise_identical(dim):
         for f in ("r", "v", "rho"):
             assert np.array_equal(o[f], outs[0][f]), f
     assert base["chunk_targets"] >= 1 and base["occupancy"] > 1.0
+
+
+@pytest.mark.parametrize("dim,dr,h_factor,schedules", [
+    (2, 0.0088, 2.0, [(0, None), (1, None), (37, None), (128, 60), (64, 512), (128, 200)]),
+    (2, 0.02, 2.0, [(0, None), (1, None), (5, None), (16, 512), (32, 60)]),
+    (3, 0.03, 1.3, [(0, None), (0, 300), (0, 1024), (0, 1900)])])
+def test_tile_schedules_are_bitwise_identical(dim, dr, h_factor, schedules):
+    """Chunk lengths and LDS capacities of the tiles themselves (2D with one
+    and with four lanes per target, 3D with windows that fit), against the
+    column chunks."""
+    pa = perturbed_dam_break(dim, dr, seed=9,
+                             **({} if dim == 3 else {"tank": [1.9, 1.6], "column": [1.3, 1.5]}))
+    assert dim == 3 or (pa.n > 24576) == (dr < 0.01)
+    eq = _eq(dim, dr, h_factor=h_factor)
+    outs = []
+    for schedule in [(0, 0)] + schedules:
+        ctx = _ctx(eq, [pa])
+        ctx.set_schedule(*schedule)
+        ctx.step(4)
+        outs.append({**ctx.download(), "pairs": ctx.pair_counts()})
+        ctx.close()
+    for schedule, o in zip(schedules, outs[1:]):
+        for f in ("r", "v", "rho", "pairs"):
+            assert np.array_equal(o[f], outs[0][f]), (schedule, f)
+
+
+@pytest.mark.parametrize("n_tanks", [256, 257, 300])
+def test_step_begin_of_many_tanks(n_tanks):
+    """The step's begin in one workgroup (up to 256 tanks) and in one per tank:
+    tanks of their own speeds, hence of their own step sizes and rebuilds, take
+    the steps that each takes alone."""
+    dr = 0.05
+    rng = np.random.default_rng(n_tanks)
+    arrays = []
+    for _ in range(n_tanks):
+        pa = ta.dam_break(2, dr, [0.5, 0.4], [0.2, 0.25])
+        pa.v = np.zeros_like(pa.r)
+        pa.v[: pa.n_fluid] = rng.uniform(0.0, 2.0) * rng.normal(size=(pa.n_fluid, 2))
+        arrays.append(pa)
+    eq = ta.cfg_equations(2, dr, 1.0)
+    ctx = _ctx(eq, arrays)
+    ctx.step(9)
+    out = ctx.download()
+    t, dt = ctx.tank_clock()
+    n = arrays[0].n
+    for k in (0, 1, n_tanks // 2, 255, n_tanks - 1):
+        one = _ctx(eq, [arrays[k]])
+        one.step(9)
+        alone = one.download()
+        for f in ("r", "v", "rho"):
+            assert np.array_equal(out[f][k * n:(k + 1) * n], alone[f]), (k, f)
+        t1, dt1 = one.tank_clock()
+        assert t[k] == t1[0] and dt[k] == dt1[0]
+        one.close()
+    assert len(set(t.tolist())) > n_tanks // 2
+    ctx.close()
 
 
 def test_autotune_keeps_the_trajectory():
