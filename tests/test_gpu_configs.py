@@ -220,6 +220,23 @@ def test_batched_256_tanks_full_size_properties():
     ctx.close()
 
 
+def test_benchmark_reports_the_index_build_of_small_and_large_sets():
+    """The benchmark's index-build figures, for a set whose index is built in
+    one launch and for one with a launch per pass."""
+    import bench
+
+    for dr, kernel in ((0.02, "rebuild_small"), (0.009, "radix_scatter")):
+        pa = ta.dam_break(2, dr, [3.22, 2.4], [1.0, 2.0])
+        eq = ta.cfg_equations(2, dr, 2.0)
+        ctx = ta.HipContext(eq)
+        ctx.upload([pa])
+        out = bench.search_roofline(ctx, [pa], reps=2)
+        assert kernel in out["kernels"] and kernel in out["per_kernel_us"]
+        assert out["rebuild_us"] > 0.0 and 0.0 < out["frac"] < 1.0
+        assert out["radix_passes"] == 2
+        ctx.close()
+
+
 # ---------------------------------------------------------------------------
 # A run where the front moves
 
