@@ -208,7 +208,9 @@ def main():
                    "fluid_particles": nf, "fixed_particles": n_fixed,
                    "sim_time_s": float(t_step[0]), "dt_next_s": float(dt_next[0]),
                    "schedule": sched, "autotune": tuned},
-        "roofline": {"bound": "hbm", "kernel": "k_stage (fused pair sums + SSPRK update)",
+        # against the HBM roofline; what limits the kernel is VALU issue (its
+        # counters are in profiles/stage_kernel_2d_dam_break_2M_sq_counters.md)
+        "roofline": {"bound": "hbm", "limiter": "valu issue", "kernel": "k_stage (fused pair sums + SSPRK update)",
                      "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic(args.workload, nf),

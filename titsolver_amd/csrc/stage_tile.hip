@@ -18,10 +18,10 @@
 // global-memory path (stage_common.hpp), so every schedule gives the same
 // bits.
 //
-// Bound: VALU issue (93 % of it at 2M particles: 1.52e8 wave instructions per
-// launch, about half in the pair loop, 43 per pair, and a third in the
-// predicate, 10.5 per candidate) and close behind it the LDS, about 80 % busy.
-// The 2M-particle dam break's launch takes 281 us; strips of one column with
+// Bound: VALU issue (96 % of the cycles at 2M particles: 1.55e8 wave
+// instructions per launch; the compiled pair loop takes 43 per pair, the
+// predicate 10.5 per candidate); the LDS is busy for 56 % of them, a third of
+// that in bank conflicts.  The 2M-particle dam break's launch takes 281 us; strips of one column with
 // acceptance masks in registers and the records gathered from L2 took 361 us
 // and 1.71e8 (95 per pair).  Of that, drawing chunks from a queue instead of
 // fixed shares gave 50 us.

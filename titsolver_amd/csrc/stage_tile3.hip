@@ -12,8 +12,9 @@
 // the global-memory path (stage_common.hpp), so every schedule gives the same
 // bits.
 //
-// Bound: latency at two waves per SIMD (VALU issue is 60 % busy, the LDS about
-// half).  2M fluid particles at h = 1.3 spacings: 1,915 us per launch; with
+// Bound: latency at two waves per SIMD (VALU issue takes 61 % of the cycles at
+// 7.0e8 wave instructions per launch, the LDS 41 %, two fifths of that bank
+// conflicts).  2M fluid particles at h = 1.3 spacings: 1,905 us per launch; with
 // acceptance masks queued in registers, three workgroups per CU and fixed
 // shares of the chunk list it took 2,610 us.  Tried: three workgroups with
 // lists of 18 entries (2,430 us: the windows that fit cut chunks to 160
