@@ -252,9 +252,9 @@ def test_tile_schedules_are_bitwise_identical(dim, dr, h_factor, schedules):
             assert np.array_equal(o[f], outs[0][f]), (schedule, f)
 
 
-@pytest.mark.parametrize("n_tanks", [256, 257, 300])
+@pytest.mark.parametrize("n_tanks", [40, 41, 257])
 def test_step_begin_of_many_tanks(n_tanks):
-    """The step's begin in one workgroup (up to 256 tanks) and in one per tank:
+    """The step's begin in one workgroup (up to 40 tanks) and in one per tank:
     tanks of their own speeds, hence of their own step sizes and rebuilds, take
     the steps that each takes alone."""
     dr = 0.05
@@ -271,7 +271,7 @@ def test_step_begin_of_many_tanks(n_tanks):
     out = ctx.download()
     t, dt = ctx.tank_clock()
     n = arrays[0].n
-    for k in (0, 1, n_tanks // 2, 255, n_tanks - 1):
+    for k in (0, 1, n_tanks // 2, n_tanks - 1):
         one = _ctx(eq, [arrays[k]])
         one.step(9)
         alone = one.download()

@@ -695,8 +695,10 @@ __device__ __forceinline__ void clear_work_sets(uint32_t* work) {
 }
 
 // Up to kBeginTanks tanks: one workgroup, which also sets ctl[0] (one launch
-// instead of a clear and an atomic per tank).
-constexpr int kBeginTanks = 256;
+// instead of a clear and an atomic per tank).  Its waves take the tanks in
+// turn: us per step, one workgroup and one per tank, 1 tank 78 and 79; 32
+// tanks 84.5 and 85.5; 48 90.9 and 90.3; 96 99 and 96.5; 256 167 and 154.
+constexpr int kBeginTanks = 40;
 __global__ __launch_bounds__(1024) void k_step_begin(int n_tanks, unsigned long long* dt_min,
                                                      double* dt, uint32_t* vmax,
                                                      const double* disp, double skin_half,
