@@ -231,8 +231,9 @@ tit_status tit_hip_kernel_stats(tit_hip_ctx* ctx, tit_hip_kernel_stat* out,
  *    64 particles, so values above 32 are as 32);
  *  - column chunks (lds_capacity 0): a workgroup takes at most chunk_targets
  *    consecutive particles of one cell column, one per lane, and reads
- *    positions from global memory.  Results
- * are bitwise identical on every schedule.  occupancy is the mean number of
+ *    positions from global memory.
+ * An upload chooses tiles, or column chunks for 2D sets with few particles per
+ * cell.  Results are bitwise identical on every schedule.  occupancy is the mean number of
  * particles per occupied cell at upload.  cached (tit_hip_autotune only): 1
  * when the schedule came from the process's tuning cache.  No reference
  * counterpart (the reference partitions pairs for TBB threads instead,

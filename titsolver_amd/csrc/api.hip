@@ -256,6 +256,26 @@ uint32_t tile_targets(const tit_hip_ctx* c) {
   return quad_tiles(c) ? std::min<uint32_t>(c->chunk_targets, kChunkMax / 4) : c->chunk_targets;
 }
 
+// The default schedule: tiles, but column chunks for 2D sets so sparse that a
+// tile (at most kChunkRows2 rows of kBlk2 cell columns) holds few of the
+// targets its lanes could take.  stretch_fill is the mean of particles per
+// stretch of kChunkRows2 rows of a column, over the stretches that hold any.
+// us per stage launch, tiles and column chunks, of uniform clouds with 0.03,
+// 0.25, 0.5, 1 and 2 particles per cell (fill 1.5, 7, 14, 28, 56): 300,000
+// particles 641, 136, 93, 62, 54 and 48, 57, 55, 64, 76; 60,000 139, 41, 33, 23,
+// 25 and 20, 23, 26, 27, 33; with four lanes per target 20,000 62, 23, 21, 21,
+// 22 and 16, 21, 22, 25, 28; 6,000 31, 17, 16, 17, 17 and 14, 18, 19, 22, 27.  A
+// lattice at h = 2 spacings fills 135.  A thin film fills little too, but its
+// cells are full (as many pairs per target, and columns of few targets): 43,335
+// particles three spacings deep 26 and 55.  So the occupied cells have to be
+// those of a cloud of fewer than 0.7 per cell as well.  (3D tiles lose only
+// below 0.2 per cell.)
+uint32_t default_lds_cap(const tit_hip_ctx* c) {
+  const double least = quad_set(c) ? 5.0 : 20.0;
+  if (c->dp.dim == 2 && c->occupancy < 1.4 && c->stretch_fill < least) return 0;
+  return stage_lds_capacity(c->dp.dim);
+}
+
 RebuildCtl rebuild_ctl(tit_hip_ctx* c) {
   return RebuildCtl{c->rebuild_ctl, c->tank_need, c->rebuild_count};
 }
@@ -1015,6 +1035,16 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
     std::sort(keys.begin(), keys.end());
     const size_t occupied = static_cast<size_t>(std::unique(keys.begin(), keys.end()) - keys.begin());
     c->occupancy = occupied ? static_cast<double>(n_total) / occupied : 1.0;
+    // stretches of kChunkRows2 rows of a cell column that hold particles
+    size_t stretches = 0, t = 0, before = ~size_t(0);
+    for (size_t k = 0; k < occupied; ++k) {
+      while (t + 1 < n_tanks && keys[k] >= ht[t + 1].cell_off) ++t;
+      const size_t local = keys[k] - ht[t].cell_off, nz = static_cast<size_t>(ht[t].nc[dim - 1]);
+      const size_t here = ht[t].cell_off + local / nz * nz + local % nz / kChunkRows2;
+      stretches += here != before ? 1 : 0;
+      before = here;
+    }
+    c->stretch_fill = stretches ? static_cast<double>(n_total) / stretches : 0.0;
   }
   c->host_tanks = ht;
 
@@ -1183,7 +1213,7 @@ tit_status tit_hip_upload_batch(tit_hip_ctx* c, const tit_hip_host_view* views,
   c->chunk_cap = 0;
   c->chain_rebuild = false;
   c->rate_steps = c->rate_rebuilds = c->rebuilds_seen = 0;
-  c->lds_cap = stage_lds_capacity(dim);
+  c->lds_cap = default_lds_cap(c);
   st = build_schedule(c);
   if (st != TIT_OK) return st;
   c->uploaded = true;

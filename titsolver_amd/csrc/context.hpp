@@ -120,6 +120,7 @@ struct tit_hip_ctx {
   size_t bchunk_cap = 0;
   int n_cu = 0;
   double occupancy = 1.0;  // mean particles per occupied cell at upload
+  double stretch_fill = 0.0;  // and per occupied stretch of a column (default_lds_cap)
 
   // graphs of two steps, by the rebuild form (chain_rebuild)
   hipGraphExec_t graph[2] = {nullptr, nullptr};
