@@ -256,9 +256,9 @@ tit_status tit_hip_set_schedule(tit_hip_ctx* ctx, const tit_hip_schedule* s);
  * are ordinary progress), keeps the fastest and returns it with its time per
  * step.  The result is kept in a per-process cache keyed by (dimension,
  * kernel, term set, walls, one or many tanks, the tiles' lanes per target, the
- * particle count's power of two): a later call on a context of the same key
- * applies the cached schedule without timing (best->cached = 1, no steps
- * taken).  No reference counterpart. */
+ * occupancy's and the particle count's powers of two): a later call on a
+ * context of the same key applies the cached schedule without timing
+ * (best->cached = 1, no steps taken).  No reference counterpart. */
 tit_status tit_hip_autotune(tit_hip_ctx* ctx, int steps_per_candidate,
                             tit_hip_schedule* best, double* best_ms_per_step);
 /* Empties the autotuner's cache. */

@@ -369,6 +369,24 @@ def test_autotune_cache_splits_at_four_lanes_per_target():
     assert 16384 <= sizes[0] <= 24576 < sizes[1] < 32768, sizes
 
 
+def test_autotune_cache_splits_by_occupancy():
+    """A lattice and a sparse cloud of as many particles, and a lattice at a
+    larger smoothing length, do not share a cache entry (tiles suit the first,
+    column chunks the others)."""
+    ta.HipContext.clear_autotune_cache()
+    pa = ta.dam_break(2, 0.02, [3.22, 2.4], [1.0, 2.0])
+    rng = np.random.default_rng(2)
+    cloud = ta.ParticleArray(2, rng.uniform(0.0, 20.0, (pa.n, 2)), np.full(pa.n, 1000.0), pa.n,
+                             np.zeros((0, 2)), (0.0, 0.0), (20.0, 20.0))
+    for arrays, h_factor in (([pa], 2.0), ([cloud], 2.0), ([pa], 4.0)):
+        ctx = _ctx(_eq(2, 0.02, h_factor=h_factor), arrays)
+        assert not ctx.autotune(2)["cached"]
+        ctx.close()
+    ctx = _ctx(_eq(2, 0.02), [pa])
+    assert ctx.autotune(2)["cached"]
+    ctx.close()
+
+
 @pytest.mark.parametrize("dim,dr,schedule", [(2, 0.02, (0, None)), (2, 0.02, (0, 0)),
                                              (2, 0.01, (64, None)), (3, 0.025, (0, None))])
 def test_stage_kernel_sums_exactly_the_neighbour_sets(dim, dr, schedule):

@@ -715,12 +715,14 @@ NeighborScratch* scratch_ptr(int device) {
 
 // The autotuner's per-process cache: the schedule found for a kind of
 // context (dimension, kernel, term set, walls, one or many tanks, four lanes
-// per target in its tiles) and size (the particle count's power of two).
+// per target in its tiles), its density (the cells' occupancy, which the best
+// schedule depends on most: sparse sets and large smoothing lengths take column
+// chunks) and size, the last two by their powers of two.
 struct TuneKey {
-  int dim, kernel, flavour, walls, batched, quad, log2n;
+  int dim, kernel, flavour, walls, batched, quad, log2occ, log2n;
   bool operator<(const TuneKey& o) const {
-    return std::tie(dim, kernel, flavour, walls, batched, quad, log2n) <
-           std::tie(o.dim, o.kernel, o.flavour, o.walls, o.batched, o.quad, o.log2n);
+    return std::tie(dim, kernel, flavour, walls, batched, quad, log2occ, log2n) <
+           std::tie(o.dim, o.kernel, o.flavour, o.walls, o.batched, o.quad, o.log2occ, o.log2n);
   }
 };
 struct TuneVal {
@@ -734,7 +736,7 @@ TuneKey tune_key(const tit_hip_ctx* c) {
   int log2n = 0;
   while ((static_cast<size_t>(1) << (log2n + 1)) <= c->n) ++log2n;
   return TuneKey{c->prm.dim, c->prm.kernel, c->dp.flavour, c->walls ? 1 : 0,
-                 c->n_tanks > 1 ? 1 : 0, quad_set(c) ? 1 : 0, log2n};
+                 c->n_tanks > 1 ? 1 : 0, quad_set(c) ? 1 : 0, std::ilogb(c->occupancy), log2n};
 }
 
 }  // namespace
